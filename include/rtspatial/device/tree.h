@@ -42,14 +42,16 @@ struct Box64 {
 };
 static_assert(sizeof(Box64) == sizeof(rts_envelope_d), "Box64 is rts_envelope_d");
 
-// The tree's top: a cut of the tree into 2 * kTopPairs disjoint subtrees
-// (or leaves), in leaf order, two to a record in the node record's format
-// (two adjacent leaf ranges: meta {ref 0, ref 1, first leaf of 0, last leaf
-// of 1}, live {live 0, live 1, last leaf of 0, 0}), so that a wavefront's
-// first expansion step tests all of them at once instead of descending the
-// top levels one dependent step at a time. Unused entries hold the empty box
-// (no test passes).
-constexpr int kTopPairs = 64;
+// The packed tree, which the library's own kernels walk: an implicit 8-ary
+// tree over the leaves in Hilbert order. With depth D (8^D >= n, D >= 1) its
+// levels 0..D-1 hold one box per run of 8^(D-d) consecutive leaves, in heap
+// order: node i's children are 8i + 1 .. 8i + 8, the root is 0, and heap
+// index leaf0 + k (leaf0 = (8^D - 1) / 7) is leaf k. Nothing but boxes and
+// live counts is stored: a node's leaves follow from its index. A node with
+// no live leaf, and every entry of a child octet past the level's end, holds
+// NaN bounds, so that no test enters it.
+constexpr int kFan = 8;
+constexpr int kMaxDepth = 10;  // 8^10 leaves
 
 struct TreeView {
   const float4* leaf_boxes;
@@ -61,8 +63,26 @@ struct TreeView {
   uint32_t leaf_size;         // ranges with <= leaf_size leaves are scanned directly
   uint32_t* error;            // device word: bit 1 refit walk, bit 2 traversal bound
   const Box64* boxes64;       // double index: the boxes by id (else null)
-  const NodeRec* top = nullptr;  // kTopPairs records of the tree's top, or null
+  // Packed tree.
+  const float4* wide = nullptr;         // bounds of node i at wide[i]
+  const uint32_t* wide_live = nullptr;  // live leaves below node i
+  uint32_t leaf0 = 0;                   // heap index of leaf 0
+  uint32_t depth = 0;                   // D
+  uint32_t start = 0, start_n = 0;      // the deepest level of at most 64 nodes
 };
+
+// First heap index of level d, and the heap index of leaf 0 at depth D.
+__host__ __device__ constexpr uint32_t wide_level0(uint32_t d) {
+  return 0x09249249u & ((1u << (3 * d)) - 1u);  // (8^d - 1) / 7, d <= kMaxDepth - 1
+}
+__host__ __device__ constexpr uint32_t wide_depth(uint64_t n) {
+  uint32_t d = 1;
+  while ((1ull << (3 * d)) < n) d++;
+  return d;
+}
+__host__ __device__ constexpr uint32_t wide_leaf0(uint32_t depth) {
+  return (uint32_t)(((1ull << (3 * depth)) - 1) / 7);
+}
 
 // Internal predicate id of line-segment queries (closed segment meets closed
 // box); not an rts_predicate value.

@@ -10,7 +10,6 @@ namespace rts {
 constexpr uint32_t kReqPoints = 1u;       // queries are points (float2)
 constexpr uint32_t kReqPredShift = 1;     // bits 1-2: rts_predicate
 constexpr uint32_t kReqWaveTiles = 8u;    // one query per wavefront (else 64 per tile)
-constexpr uint32_t kReqLeafShift = 4;     // bits 4-6: log2(leaf_size) + 1, 0 = the tree's
 constexpr uint32_t kReqExt = 128u;        // walked by per-request launches (BatchExt), no tiles
 
 struct BatchRequest {
@@ -32,7 +31,7 @@ constexpr int kClassWaveIntersects = 0;
 constexpr int kClassWaveWithin = 1;
 constexpr int kClassWaveContains = 2;
 constexpr int kClassWavePoints = 3;
-constexpr int kClassLane = 4;  // 64 queries per tile, one per lane, any predicate
+constexpr int kClassLane = 4;  // 64 queries per tile, one per octet, any predicate
 constexpr int kClasses = 5;
 
 // Requests the batch kernels do not walk (segments, double queries) come
@@ -74,23 +73,20 @@ struct BatchHeader {
   uint32_t pad;
 };
 
-// Counts of a batch. The count pass gives each query a bound on its results:
-// exact for lane tiles and extension requests, an upper bound for wave tiles
-// (their count walks do not test the leaves of partly covered ranges). The
-// scan of the bounds places each query's pairs in the arena, and the write
-// pass, which tests those leaves, records each query's exact count. Query q's
-// pairs are then arena[offsets[q], offsets[q] + exact[q]).
+// Counts of a batch. The count pass gives each query its number of results
+// (its wave walks log them); their scan places each query's pairs in the
+// arena. Query q's pairs are arena[offsets[q], offsets[q] + exact[q]).
 struct BatchArgs {
   const BatchHeader* header;     // device
   const BatchRequest* requests;  // device, sorted by tbase
   uint32_t* tile_counters;       // kTileCounterWords: per-pass, per-class, per-XCD counters
-  uint32_t* counts;              // per global query: result bound
+  uint32_t* counts;              // per global query: results
   uint32_t* exact;               // per global query: results
   uint64_t* offsets;             // per global query: exclusive scan of counts
   uint64_t* exact_offsets;       // per global query: exclusive scan of exact (with collect)
   uint64_t* seg_sums;            // scan scratch (batch_seg_sums_words())
-  uint64_t* total;               // [0] sum of the bounds, [2] of the exact counts
-  uint64_t* ranges;              // per request: {first arena slot, slots (bounds), results}
+  uint64_t* total;               // [0] sum of the counts, [2] of the exact counts
+  uint64_t* ranges;              // per request: {first arena slot, slots, results}
   rts_pair* arena;               // results
   uint64_t arena_cap;            // pairs the arena holds
   const uint32_t* order;         // wave tiles in Morton order (tile -> tile), or null
@@ -122,7 +118,7 @@ struct BatchSort {
 // the batch are counted and written by one wave launch each (query.hip, the
 // plain path's kernels) into the batch's counts, offsets and arena.
 struct BatchExt {
-  QueryLaunch ql;  // tree, queries, n, qid_base, pred, point_queries, f64, leaf size
+  QueryLaunch ql;  // tree, queries, n, qid_base, pred, point_queries, f64
   uint64_t qbase;
   bool none;       // a predicate that matches nothing (segments under RTS_CONTAINS)
 };

@@ -4,22 +4,20 @@
 // A batch is a list of requests (queries pointer, count, point/envelope,
 // predicate, tile mode) laid out in one query space: request r owns global
 // queries [qbase_r, qbase_r + n_r) and tiles [tbase_r, tbase_r + tiles_r).
-// A tile is either 64 queries of one request answered one per lane (lane
-// tiles: points and data-contains-query, few results each) or one query
+// A tile is either 64 queries of one request answered one per octet of lanes
+// (lane tiles: points and data-contains-query, few results each) or one query
 // answered by a whole wavefront (wave tiles: intersects / within). Requests
 // are listed class by class (batch.h), and one persistent kernel per pass
 // takes the tiles of every class: per class, each XCD first drains its own
 // contiguous eighth of the class's tiles, which keeps neighbouring queries on
 // one L2, and then steals from the other XCDs.
 //
-// Two passes: the count pass writes a bound on each query's results (exact
-// for lane tiles; a wave tile's count walk counts the leaf ranges it would
-// have to test as a whole and logs them), a scan turns the bounds into
-// exclusive offsets into the slot's result arena, and the write pass tests
-// the logged ranges, writes each query's pairs at the start of its slots
-// and records its exact count. Per request, the batch reports its first
-// slot, its slots and its results. Every launch reads the batch's sizes from
-// device memory.
+// Two passes: the count pass writes each query's number of results and logs a
+// wave tile's (range_log.h), a scan turns the numbers into exclusive offsets
+// into the slot's result arena, and the write pass emits the logged results
+// (a lane tile's walk is cheap and taken again) at the query's offset. Per
+// request, the batch reports its first slot, its slots and its results. Every
+// launch reads the batch's sizes from device memory.
 #include <algorithm>
 
 #include "batch.h"
@@ -28,6 +26,7 @@
 #include "range_log.h"
 #include "rtspatial/device/traverse.h"
 #include "rtspatial/device/wave.h"
+#include "wide.h"
 
 namespace rts {
 namespace {
@@ -84,13 +83,49 @@ __device__ __forceinline__ uint32_t grab_tile(uint32_t* counters, const uint32_t
   return readlane_u32(got, 0);
 }
 
+union TileLds {
+  WideLds wide;
+  uint32_t oct[kWave / kFan][kOctStack];
+};
+
 // One tile of the batch: a wave tile's one query (by the whole wave) or a
 // lane tile's 64 queries. With skip_giants a wave tile whose query is on a
 // giant list is left to that list.
+// Queries and results of a lane tile's octet walk.
+struct TileSource {
+  const void* queries;
+  bool points;
+  int pred;
+  __device__ void operator()(uint32_t i, QueryRT& q) const {
+    q.b = load_query(queries, points, i);
+    q.pred = pred;
+  }
+};
+struct TileCount {
+  uint32_t* counts;
+  uint32_t* exact;
+  __device__ void hits(bool, uint64_t, uint32_t, uint32_t, uint32_t) const {}
+  __device__ void finish(uint32_t i, uint32_t found) const {
+    if ((lane_id() & 7u) == 0) counts[i] = exact[i] = found;
+  }
+};
+struct TileWrite {
+  const uint64_t* offsets;
+  rts_pair* arena;
+  uint64_t cap;
+  uint32_t qid_base;
+  __device__ void hits(bool hit, uint64_t, uint32_t i, uint32_t k, uint32_t gid) const {
+    if (!hit) return;
+    const uint64_t slot = offsets[i] + k;
+    if (slot < cap) store_pair(arena + slot, gid, i + qid_base);
+  }
+  __device__ void finish(uint32_t, uint32_t) const {}
+};
+
 template <bool WRITE>
-__device__ __forceinline__ void run_tile(const TreeView& t0, TreeView& t, const BatchArgs& a,
+__device__ __forceinline__ void run_tile(const TreeView& t, const BatchArgs& a,
                                          const BatchHeader& h, uint32_t tile, bool skip_giants,
-                                         LogCursor& lc, WaveLds& lds) {
+                                         LogCursor& lc, TileLds& lds) {
   const uint32_t ri = find_request(a.requests, h.n_requests, tile);
   const BatchRequest r = a.requests[ri];
   const uint32_t local = tile - r.tbase;
@@ -119,27 +154,27 @@ __device__ __forceinline__ void run_tile(const TreeView& t0, TreeView& t, const 
     }
     return;
   }
-  const uint32_t lb = (r.flags >> kReqLeafShift) & 7u;
-  t.leaf_size = lb ? 1u << (lb - 1) : t0.leaf_size;
   const bool points = r.flags & kReqPoints;
   const int pred = points ? (int)RTS_CONTAINS : (int)((r.flags >> kReqPredShift) & 3u);
   if (wave) {
     if (local >= r.n) return;
-    const QueryRT qb{load_query(r.queries, points, local), pred};
     const uint64_t g = r.qbase + local;
     if (WRITE) {
-      RangeLog lg = log_for_write(a.log, g);
-      const uint64_t e = wave_query<0, false, true, true>(
-          t, qb, local + r.qid_base, QueueEmit{a.arena, a.arena_cap, a.offsets[g]}, lds, &lg);
-      if (lane_id() == 0) a.exact[g] = (uint32_t)e;
+      const RangeLog lg = log_for_write(a.log, g);
+      const QueueEmit emit{a.arena, a.arena_cap, a.offsets[g]};
+      if (lg.n_in != kLogOverflow) {
+        wide_replay(t, lg, local + r.qid_base, emit);
+      } else {
+        const QueryRT qb{load_query(r.queries, points, local), pred};
+        wide_walk<0, false, true, false>(t, qb, local + r.qid_base, emit, lds.wide);
+      }
     } else {
-      // The bound: the write pass tests the logged ranges' leaves.
+      const QueryRT qb{load_query(r.queries, points, local), pred};
       RangeLog lg = log_for_count(lc);
-      const uint64_t c =
-          wave_query<0, false, false, true, true>(t, qb, local, NoEmit{}, lds, &lg);
+      const uint64_t c = wide_walk<0, false, false, true>(t, qb, local, NoEmit{}, lds.wide, &lg);
       log_commit(lc, a.log, g, lg);
       if (lane_id() == 0) {
-        a.counts[g] = (uint32_t)c;
+        a.counts[g] = a.exact[g] = (uint32_t)c;
         // Giants are listed as they are counted (rare: one atomic each).
         if (a.giants && c >= giant_min(kGiantBuckets - 1)) {
           int b = kGiantBuckets - 1;
@@ -151,15 +186,17 @@ __device__ __forceinline__ void run_tile(const TreeView& t0, TreeView& t, const 
       }
     }
   } else {
-    const uint32_t q = local * kWave + lane_id();
-    if (q >= r.n) return;
-    const QueryRT qb{load_query(r.queries, points, q), pred};
-    const uint64_t g = r.qbase + q;
+    const uint32_t first = local * kWave;
+    if (first >= r.n) return;
+    const uint32_t last = first + kWave < r.n ? first + kWave : r.n;
+    const TileSource src{r.queries, points, pred};
+    uint32_t* stack = lds.oct[lane_id() / kFan];
     if (WRITE) {
-      lane_query<0, false, true>(t, qb, q + r.qid_base,
-                                 QueueEmit{a.arena, a.arena_cap, a.offsets[g]});
+      TileWrite sink{a.offsets + r.qbase, a.arena, a.arena_cap, r.qid_base};
+      oct_walk<0, false, false, QueryRT>(t, stack, first, last, src, sink);
     } else {
-      a.counts[g] = a.exact[g] = (uint32_t)lane_query<0, false, false>(t, qb, q, NoEmit{});
+      TileCount sink{a.counts + r.qbase, a.exact + r.qbase};
+      oct_walk<0, false, true, QueryRT>(t, stack, first, last, src, sink);
     }
   }
 }
@@ -171,15 +208,10 @@ __device__ __forceinline__ void run_tile(const TreeView& t0, TreeView& t, const 
 // workgroup: a workgroup's slot is freed as soon as its one wave runs out of
 // tiles (four-wave workgroups held theirs until the slowest wave ended). The
 // write pass first takes the giant tiles, largest bucket first.
-// The write pass is pinned at 6 waves per SIMD (80 VGPRs), which the range
-// logs would otherwise push just past (81); the count pass, which tests no
-// leaves of wave tiles, needs 58 VGPRs and runs 8 (at least 7).
 template <bool WRITE>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WRITE ? 6 : 7)))
-k_batch(const TreeView* tv, const BatchArgs a) {
-  __shared__ WaveLds s_lds;
-  const TreeView t0 = *tv;
-  TreeView t = t0;  // leaf_size may differ per request
+__global__ void __launch_bounds__(kWave) k_batch(const TreeView* tv, const BatchArgs a) {
+  __shared__ TileLds s_lds;
+  const TreeView t = *tv;
   const BatchHeader h = *a.header;
   if (h.n_tiles == 0 || h.n_requests == 0) return;
   // An empty index (no boxes inserted, or cleared) has no tree: the count
@@ -224,7 +256,7 @@ k_batch(const TreeView* tv, const BatchArgs a) {
       // lead with the class).
       if (a.order && tile < wave_end) tile = a.order[tile];
     }
-    run_tile<WRITE>(t0, t, a, h, tile, giants && !listed, lc, s_lds);
+    run_tile<WRITE>(t, a, h, tile, giants && !listed, lc, s_lds);
   }
 }
 

@@ -1,18 +1,22 @@
 // LBVH construction and maintenance kernels.
 //
-//   scene bounds  -> 30-bit Morton codes of FP32 box centres (15 bits/axis)
+//   scene bounds  -> 30-bit Hilbert codes of FP32 box centres (15 bits/axis)
 //   radix sort    -> (sort.hip)
-//   Karras 2012   -> binary hierarchy over the sorted codes ("Maximizing
-//                    Parallelism in the Construction of BVHs, Octrees, and k-d
-//                    Trees"), ties broken by position; small nodes answered
-//                    from an LDS window of the keys
-//   refit         -> bottom-up union of child bounds in three levels (LDS
-//                    node state per chunk, then the nodes that span chunks);
-//                    a build's refit also gathers the boxes into Morton order
-//                    and the id -> sorted-position map
+//   packed tree   -> bounds of 8, 64, 512, ... consecutive leaves, in one pass
+//                    over the leaves; a build's pass also gathers the boxes
+//                    into code order and the id -> sorted-position map
 //
 // Mutations (replacing the reference's OptiX refits, spatial_index.cuh:208-336)
-// write boxes by id and in sorted position, then refit the tree.
+// write boxes by id and in sorted position, then take that pass again.
+//
+// Kernels a caller compiles around its own handler walk a binary tree over the
+// same leaves, made when its view is asked for:
+//
+//   Karras 2012   -> binary hierarchy over the sorted codes ("Maximizing
+//                    Parallelism in the Construction of BVHs, Octrees, and k-d
+//                    Trees"), ties broken by position
+//   refit         -> bottom-up union of child bounds in three levels (LDS
+//                    node state per chunk, then the nodes that span chunks)
 //
 // Every kernel is memory-bound integer/compare work; none uses MFMA.
 #include <cfloat>
@@ -80,7 +84,25 @@ __global__ void __launch_bounds__(kThreads) k_reduce_bounds(const float4* __rest
   if (threadIdx.x == 0) out[0] = sh[0];
 }
 
-// ------------------------------------------------------------ morton ----
+// ------------------------------------------------------------- codes ----
+__global__ void __launch_bounds__(kThreads) k_hilbert_boxes(const float4* __restrict__ boxes,
+                                                            uint32_t n,
+                                                            const float4* __restrict__ scene,
+                                                            uint32_t* __restrict__ keys) {
+  __shared__ uint8_t table[256];
+  static_assert(kThreads == 256, "one table byte per thread");
+  table[threadIdx.x] = kHilbertTable.v[threadIdx.x];
+  __syncthreads();
+  const float4 s = scene[0];
+  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
+    const float4 b = boxes[i];
+    const float cx = 0.5f * (b.x + b.z), cy = 0.5f * (b.y + b.w);
+    // Deleted boxes (NaN) sort last.
+    keys[i] = (cx == cx && cy == cy) ? hilbert_of_morton(morton_of(cx, cy, s), table)
+                                     : (1u << kMortonBits) - 1;
+  }
+}
+
 __global__ void __launch_bounds__(kThreads) k_morton_boxes(const float4* __restrict__ boxes, uint32_t n,
                                                            const float4* __restrict__ scene,
                                                            uint32_t* __restrict__ keys) {
@@ -99,6 +121,138 @@ __global__ void __launch_bounds__(kThreads) k_morton_points(const float2* __rest
     float2 p = pts[i];
     keys[i] = morton_of(p.x, p.y, s);
   }
+}
+
+// ------------------------------------------------------- packed tree ----
+// Bounds of the runs of 8, 64 and 512 consecutive entries of one level: a
+// workgroup takes 512 entries, one per thread; an octet's bounds are united
+// with lane moves, a wave's eight octets' with shuffles, the workgroup's eight
+// waves' through LDS. Three levels per launch (10M leaves: three launches),
+// every input read once and every node written once: bound by HBM, and in a
+// build by the gather of the boxes by id. The Karras tree with its refit that
+// this replaces in the library's own walks wrote 64 bytes per box.
+constexpr int kLevelThreads = 512;
+
+struct NodeAcc {
+  float4 b;
+  uint32_t live;
+};
+
+// Lane moves within an octet: lane ^ 1, lane ^ 2, and 7 - lane (once a quad
+// agrees, the other quad's value).
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141;
+template <int CTRL>
+__device__ __forceinline__ float moved(float v) {
+  return __int_as_float((int)dpp_move<CTRL>((uint32_t)__float_as_int(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ NodeAcc united(const NodeAcc a) {
+  return NodeAcc{make_float4(fminf(a.b.x, moved<CTRL>(a.b.x)), fminf(a.b.y, moved<CTRL>(a.b.y)),
+                             fmaxf(a.b.z, moved<CTRL>(a.b.z)), fmaxf(a.b.w, moved<CTRL>(a.b.w))),
+                 a.live + dpp_move<CTRL>(a.live)};
+}
+// The union over this lane's octet. NaN bounds (nothing live) give way to any
+// other: fminf and fmaxf return the other operand.
+__device__ __forceinline__ NodeAcc octet_union(NodeAcc a) {
+  return united<kDppHalfMirror>(united<kDppXor2>(united<kDppXor1>(a)));
+}
+// The union over the wave's octets, each holding its own in every lane.
+__device__ __forceinline__ NodeAcc wave_union(NodeAcc a) {
+#pragma unroll
+  for (int d = 8; d < 64; d <<= 1) {
+    a.b.x = fminf(a.b.x, __shfl_xor(a.b.x, d, 64));
+    a.b.y = fminf(a.b.y, __shfl_xor(a.b.y, d, 64));
+    a.b.z = fmaxf(a.b.z, __shfl_xor(a.b.z, d, 64));
+    a.b.w = fmaxf(a.b.w, __shfl_xor(a.b.w, d, 64));
+    a.live += (uint32_t)__shfl_xor((int)a.live, d, 64);
+  }
+  return a;
+}
+
+// Writes the three levels above `level` (whose entry of this thread is `a`,
+// position p) into the heap; levels above the root do not exist.
+__device__ __forceinline__ void write_levels(NodeAcc a, uint32_t p, uint32_t level,
+                                             float4* __restrict__ wide,
+                                             uint32_t* __restrict__ wide_live) {
+  __shared__ NodeAcc s_wave[kLevelThreads / kWave];
+  const uint32_t lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  a = octet_union(a);
+  // Positions of a level of 8^k entries past its end belong to no node.
+  if ((lane & 7u) == 0 && (p >> 3) < (1u << (3 * (level - 1)))) {
+    const uint32_t at = wide_level0(level - 1) + (p >> 3);
+    wide[at] = a.b;
+    wide_live[at] = a.live;
+  }
+  if (level < 2) return;
+  a = wave_union(a);
+  if (lane == 0) {
+    if ((p >> 6) < (1u << (3 * (level - 2)))) {
+      const uint32_t at = wide_level0(level - 2) + (p >> 6);
+      wide[at] = a.b;
+      wide_live[at] = a.live;
+    }
+    s_wave[w] = a;
+  }
+  if (level < 3) return;
+  __syncthreads();
+  if (threadIdx.x < kLevelThreads / kWave) {
+    a = octet_union(s_wave[threadIdx.x]);
+    if (threadIdx.x == 0 && (p >> 9) < (1u << (3 * (level - 3)))) {
+      const uint32_t at = wide_level0(level - 3) + (p >> 9);
+      wide[at] = a.b;
+      wide_live[at] = a.live;
+    }
+  }
+}
+
+// The leaves: GATHER takes leaf k's box by id (ids counted from `off`,
+// rewritten to the ids themselves when off > 0) into tree order and notes its
+// position.
+template <bool GATHER>
+__global__ void __launch_bounds__(kLevelThreads) k_wide_leaves(
+    float4* __restrict__ leaf_boxes, uint32_t n, uint32_t depth, float4* __restrict__ wide,
+    uint32_t* __restrict__ wide_live, uint32_t* error, const float4* __restrict__ boxes,
+    uint32_t* __restrict__ ids, uint32_t off, uint32_t* __restrict__ leaf_of_id) {
+  const uint32_t k = blockIdx.x * kLevelThreads + threadIdx.x;
+  const float x = __builtin_nanf("");
+  NodeAcc a{make_float4(x, x, x, x), 0u};
+  if (k < n) {
+    float4 b = a.b;
+    if (GATHER) {
+      const uint32_t local = ids[k];
+      if (local >= n) {  // unreachable for a correct sort; keeps reads in bounds
+        atomicOr(error, 2u);
+      } else {
+        const uint32_t id = local + off;
+        if (off) ids[k] = id;
+        b = boxes[id];
+        leaf_boxes[k] = b;
+        leaf_of_id[id] = off + k;
+      }
+    } else {
+      b = leaf_boxes[k];
+    }
+    // Bounds cover the box's extent even if its corners are swapped, so a
+    // node inside a query implies every live box below it matches.
+    if (!box_dead(b))
+      a = NodeAcc{make_float4(fminf(b.x, b.z), fminf(b.y, b.w), fmaxf(b.x, b.z), fmaxf(b.y, b.w)),
+                  1u};
+  }
+  write_levels(a, k, depth, wide, wide_live);
+}
+
+// The levels above `level` (>= 1), of which `m` nodes exist.
+__global__ void __launch_bounds__(kLevelThreads) k_wide_levels(float4* __restrict__ wide,
+                                                               uint32_t* __restrict__ wide_live,
+                                                               uint32_t level, uint32_t m) {
+  const uint32_t p = blockIdx.x * kLevelThreads + threadIdx.x;
+  const float x = __builtin_nanf("");
+  NodeAcc a{make_float4(x, x, x, x), 0u};
+  if (p < m) {
+    a.b = wide[wide_level0(level) + p];
+    a.live = wide_live[wide_level0(level) + p];
+  }
+  write_levels(a, p, level, wide, wide_live);
 }
 
 // ------------------------------------------------------------ karras ----
@@ -222,13 +376,11 @@ __device__ __forceinline__ void push_boundary(uint32_t* slots, uint32_t code, ui
 // of LDS per workgroup and four 16-byte stores per record, 806 vs 672 us on
 // 10M boxes.)
 constexpr uint32_t kEndShift = 20;
-template <bool GATHER>
 __global__ void __launch_bounds__(kRefitThreads) k_refit_chunk(
-    float4* __restrict__ leaf_boxes, uint32_t n, uint32_t chunk_log2,
+    const float4* __restrict__ leaf_boxes, uint32_t n, uint32_t chunk_log2,
     const uint32_t* __restrict__ parent, NodeRec* nodes, float4* __restrict__ root_box,
     uint32_t* __restrict__ root_live, uint32_t* error, uint32_t* boundary,
-    const uint32_t* __restrict__ node_end, const float4* __restrict__ boxes,
-    uint32_t* __restrict__ ids, uint32_t off, uint32_t* __restrict__ leaf_of_id) {
+    const uint32_t* __restrict__ node_end) {
   extern __shared__ float4 s_box[];
   const uint32_t C = 1u << chunk_log2;
   uint32_t* s_cnt = reinterpret_cast<uint32_t*>(s_box + C);
@@ -246,21 +398,7 @@ __global__ void __launch_bounds__(kRefitThreads) k_refit_chunk(
   }
   __syncthreads();
   for (uint32_t k = c0 + threadIdx.x; k <= c1; k += kRefitThreads) {
-    float4 b;
-    if (GATHER) {
-      const uint32_t local = ids[k];
-      if (local >= n) {  // unreachable for a correct sort; keeps reads in bounds
-        atomicOr(error, 2u);
-        continue;
-      }
-      const uint32_t id = local + off;
-      if (off) ids[k] = id;
-      b = boxes[id];
-      leaf_boxes[k] = b;
-      leaf_of_id[id] = off + k;
-    } else {
-      b = leaf_boxes[k];
-    }
+    float4 b = leaf_boxes[k];
     uint32_t live = 1;
     if (box_dead(b)) {
       b = empty_box();
@@ -390,118 +528,28 @@ __global__ void __launch_bounds__(TOP ? kRefitTopThreads : kRefitSpanThreads) k_
   }
 }
 
-// ------------------------------------------------------------- top ----
-// The tree's top (TreeView::top): starting from the root's two children,
-// every round splits internal entries into their two children, in place (so
-// leaf order is kept), the largest first when the 2 * kTopPairs entries
-// would overflow, until no entry can be split. One wavefront; each round is
-// one dependent load of node records.
-constexpr uint32_t kTopEntries = 2 * kTopPairs;
-__global__ void __launch_bounds__(kWave) k_tree_top(const NodeRec* __restrict__ nodes,
-                                                     NodeRec* __restrict__ top) {
-  __shared__ float4 s_box[2][kTopEntries];
-  __shared__ uint32_t s_ref[2][kTopEntries], s_first[2][kTopEntries], s_cnt[2][kTopEntries],
-      s_live[2][kTopEntries];
-  const uint32_t lane = threadIdx.x;
-  // The two children of internal node `node` as entries at..at+1 of buffer b.
-  auto children = [&](uint32_t node, int b, uint32_t at) {
-    const NodeRec nd = nodes[node];
-    const uint32_t gamma = nd.meta.x & ~kLeafFlag;
-    s_box[b][at] = nd.box[0];
-    s_box[b][at + 1] = nd.box[1];
-    s_ref[b][at] = nd.meta.x;
-    s_ref[b][at + 1] = nd.meta.y;
-    s_first[b][at] = nd.meta.z;
-    s_first[b][at + 1] = gamma + 1;
-    s_cnt[b][at] = gamma - nd.meta.z + 1;
-    s_cnt[b][at + 1] = nd.meta.w - gamma;
-    s_live[b][at] = nd.live.x;
-    s_live[b][at + 1] = nd.live.y;
-  };
-  if (lane == 0) children(0, 0, 0);
-  __syncthreads();
-  uint32_t m = 2, cur = 0;  // wave-uniform
-  // Each round splits at least one entry or stops, and m <= kTopEntries.
-  for (uint32_t round = 0; round < kTopEntries; round++) {
-    bool split[2];
-    for (int k = 0; k < 2; k++) {
-      const uint32_t i = lane + k * kWave;
-      split[k] = i < m && !(s_ref[cur][i] & kLeafFlag);
-    }
-    const uint32_t splittable =
-        (uint32_t)__popcll(ballot(split[0])) + (uint32_t)__popcll(ballot(split[1]));
-    const uint32_t room = kTopEntries - m;
-    if (splittable == 0 || room == 0) break;
-    if (splittable > room) {
-      // The `room` largest (ties: the earlier entry).
-      for (int k = 0; k < 2; k++) {
-        if (!split[k]) continue;
-        const uint32_t i = lane + k * kWave, c = s_cnt[cur][i];
-        uint32_t rank = 0;
-        for (uint32_t j = 0; j < m; j++) {
-          if (s_ref[cur][j] & kLeafFlag) continue;
-          const uint32_t cj = s_cnt[cur][j];
-          rank += (cj > c || (cj == c && j < i)) ? 1u : 0u;
-        }
-        split[k] = rank < room;
-      }
-    }
-    // Entry i moves to i + (splits before i).
-    const uint32_t a0 = split[0] ? 1u : 0u, a1 = split[1] ? 1u : 0u;
-    const uint32_t inc0 = wave_inclusive_sum(a0);
-    const uint32_t tot0 = readlane_u32(inc0, kWave - 1);
-    const uint32_t inc1 = wave_inclusive_sum(a1);
-    const uint32_t before[2] = {inc0 - a0, tot0 + inc1 - a1};
-    const int nxt = cur ^ 1;
-    for (int k = 0; k < 2; k++) {
-      const uint32_t i = lane + k * kWave;
-      if (i >= m) continue;
-      const uint32_t at = i + before[k];
-      if (split[k]) {
-        children(s_ref[cur][i], nxt, at);
-      } else {
-        s_box[nxt][at] = s_box[cur][i];
-        s_ref[nxt][at] = s_ref[cur][i];
-        s_first[nxt][at] = s_first[cur][i];
-        s_cnt[nxt][at] = s_cnt[cur][i];
-        s_live[nxt][at] = s_live[cur][i];
-      }
-    }
-    m += tot0 + readlane_u32(inc1, kWave - 1);
-    cur = nxt;
-    __syncthreads();
-  }
-  // Record `lane`: entries 2 lane (left) and 2 lane + 1 (right); entries
-  // past m are empty (the right one then covers no leaves).
-  const uint32_t i0 = 2 * lane, i1 = i0 + 1;
-  const bool ok0 = i0 < m, ok1 = i1 < m;
-  const uint32_t last0 = ok0 ? s_first[cur][i0] + s_cnt[cur][i0] - 1 : 0u;
-  NodeRec r;
-  r.box[0] = ok0 ? s_box[cur][i0] : empty_box();
-  r.box[1] = ok1 ? s_box[cur][i1] : empty_box();
-  r.meta = make_uint4(ok0 ? s_ref[cur][i0] : kLeafFlag, ok1 ? s_ref[cur][i1] : kLeafFlag,
-                      ok0 ? s_first[cur][i0] : 0u,
-                      ok1 ? s_first[cur][i1] + s_cnt[cur][i1] - 1 : last0);
-  r.live = make_uint4(ok0 ? s_live[cur][i0] : 0u, ok1 ? s_live[cur][i1] : 0u, last0, 0u);
-  top[lane] = r;
-}
-
 __global__ void __launch_bounds__(kThreads) k_clear_flags(uint32_t* flags, uint32_t m) {
   for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < m; i += gridDim.x * kThreads) flags[i] = 0;
 }
 
 // ------------------------------------------------------------ cost ------
-// Sum of half-perimeters of all nodes below the root, divided by the root's:
-// the expected number of node visits of small random range queries, up to a
-// constant. Non-finite (empty) boxes contribute nothing.
-__global__ void __launch_bounds__(kThreads) k_tree_cost(const NodeRec* __restrict__ nodes, uint32_t m,
-                                                        double* __restrict__ out) {
+// Sum of half-perimeters of the packed tree's nodes below the root, divided by
+// the root's: the expected number of node visits of small random range
+// queries, up to a constant. Nodes with nothing live (NaN bounds) and
+// unbounded ones contribute nothing.
+__global__ void __launch_bounds__(kThreads) k_tree_cost(const float4* __restrict__ wide, uint32_t n,
+                                                        uint32_t depth, double* __restrict__ out) {
   __shared__ double sh[kThreads / kWave];
   double acc = 0.0;
-  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < m; i += gridDim.x * kThreads) {
-    float4 b = nodes[i >> 1].box[i & 1];
-    double hp = (double)(b.z - b.x) + (double)(b.w - b.y);
-    if (hp >= 0.0 && hp < 1e300) acc += hp;
+  for (uint32_t d = 1; d < depth; d++) {
+    const uint32_t shift = 3 * (depth - d);
+    const uint32_t m = (uint32_t)(((uint64_t)n + (1ull << shift) - 1) >> shift);
+    const float4* lv = wide + wide_level0(d);
+    for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < m; i += gridDim.x * kThreads) {
+      const float4 b = lv[i];
+      const double hp = (double)(b.z - b.x) + (double)(b.w - b.y);
+      if (hp >= 0.0 && hp < 1e300) acc += hp;
+    }
   }
   acc = wave_sum_f64(acc);
   if (lane_id() == 0) sh[threadIdx.x / kWave] = acc;
@@ -513,9 +561,9 @@ __global__ void __launch_bounds__(kThreads) k_tree_cost(const NodeRec* __restric
   }
 }
 
-__global__ void k_cost_finish(const float4* __restrict__ root_box, double* out) {
-  float4 r = root_box[0];
-  double hp = (double)(r.z - r.x) + (double)(r.w - r.y);
+__global__ void k_cost_finish(const float4* __restrict__ wide, double* out) {
+  const float4 r = wide[0];
+  const double hp = (double)(r.z - r.x) + (double)(r.w - r.y);
   out[1] = (hp > 0.0 && hp < 1e300) ? (out[0] + hp) / hp : 1.0;
 }
 
@@ -569,6 +617,40 @@ hipError_t launch_scene_bounds(const float4* boxes, uint32_t n, float4* partials
                      partials);
   hipLaunchKernelGGL(k_reduce_bounds, dim3(1), dim3(kThreads), 0, stream, partials, n_partials,
                      scene);
+  return hipGetLastError();
+}
+
+hipError_t launch_hilbert_boxes(const float4* boxes, uint32_t n, const float4* scene,
+                                uint32_t* keys, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_hilbert_boxes, dim3(grid_for(n)), dim3(kThreads), 0, stream, boxes, n, scene,
+                     keys);
+  return hipGetLastError();
+}
+
+hipError_t launch_wide_tree(const WideArgs& a, hipStream_t stream) {
+  if (a.n == 0) return hipSuccess;
+  const uint32_t depth = wide_depth(a.n);
+  // Whole octets of workgroups: the third level up is then filled to a whole
+  // octet too (past the last leaf with empty nodes).
+  auto blocks = [](uint64_t m) {
+    const uint64_t b = (m + kLevelThreads - 1) / kLevelThreads;
+    return dim3((uint32_t)((b + kFan - 1) / kFan * kFan));
+  };
+  if (a.boxes)
+    hipLaunchKernelGGL(k_wide_leaves<true>, blocks(a.n), dim3(kLevelThreads), 0, stream,
+                       a.leaf_boxes, a.n, depth, a.wide, a.wide_live, a.error, a.boxes, a.ids,
+                       a.off, a.leaf_of_id);
+  else
+    hipLaunchKernelGGL(k_wide_leaves<false>, blocks(a.n), dim3(kLevelThreads), 0, stream,
+                       a.leaf_boxes, a.n, depth, a.wide, a.wide_live, a.error, nullptr, nullptr, 0u,
+                       nullptr);
+  for (int level = (int)depth - 3; level > 0; level -= 3) {
+    const uint32_t shift = 3 * (depth - (uint32_t)level);
+    const uint64_t m = ((uint64_t)a.n + (1ull << shift) - 1) >> shift;
+    hipLaunchKernelGGL(k_wide_levels, blocks(m), dim3(kLevelThreads), 0, stream, a.wide,
+                       a.wide_live, (uint32_t)level, (uint32_t)m);
+  }
   return hipGetLastError();
 }
 
@@ -638,14 +720,9 @@ hipError_t launch_refit(const RefitArgs& a, hipStream_t stream) {
                        n - 1);
   }
   const size_t lds = refit_chunk_lds_bytes(lg);
-  if (a.gather)
-    hipLaunchKernelGGL(k_refit_chunk<true>, dim3(chunks), dim3(kRefitThreads), lds, stream,
-                       a.leaf_boxes, n, lg, a.parent, a.nodes, a.root_box, a.root_live, a.error,
-                       a.boundary, a.node_end, a.boxes, a.ids, a.off, a.leaf_of_id);
-  else
-    hipLaunchKernelGGL(k_refit_chunk<false>, dim3(chunks), dim3(kRefitThreads), lds, stream,
-                       a.leaf_boxes, n, lg, a.parent, a.nodes, a.root_box, a.root_live, a.error,
-                       a.boundary, a.node_end, nullptr, nullptr, 0u, nullptr);
+  hipLaunchKernelGGL(k_refit_chunk, dim3(chunks), dim3(kRefitThreads), lds, stream, a.leaf_boxes, n,
+                     lg, a.parent, a.nodes, a.root_box, a.root_live, a.error, a.boundary,
+                     a.node_end);
   if (chunks > 1) {
     const uint32_t groups = (chunks + kRefitGroup - 1) / kRefitGroup;
     hipLaunchKernelGGL(k_refit_span<false>, dim3(groups), dim3(kRefitSpanThreads), 0, stream,
@@ -655,19 +732,16 @@ hipError_t launch_refit(const RefitArgs& a, hipStream_t stream) {
                        a.nodes, n, lg, chunks, a.root_box, a.root_live, a.flags, a.error,
                        a.boundary);
   }
-  if (a.top && n >= kTopMinLeaves)
-    hipLaunchKernelGGL(k_tree_top, dim3(1), dim3(kWave), 0, stream, a.nodes, a.top);
   return hipGetLastError();
 }
 
-hipError_t launch_tree_cost(const NodeRec* nodes, const float4* root_box, uint32_t n,
-                            double* out, hipStream_t stream) {
+hipError_t launch_tree_cost(const float4* wide, uint32_t n, double* out, hipStream_t stream) {
   hipError_t e = launch_fill_u32(reinterpret_cast<uint32_t*>(out), 0u, 4, stream);
   if (e != hipSuccess) return e;
-  if (n > 1)
-    hipLaunchKernelGGL(k_tree_cost, dim3(grid_for(2 * (uint64_t)(n - 1), 2048)), dim3(kThreads), 0,
-                       stream, nodes, 2 * (n - 1), out);
-  hipLaunchKernelGGL(k_cost_finish, dim3(1), dim3(1), 0, stream, root_box, out);
+  if (n > 8)
+    hipLaunchKernelGGL(k_tree_cost, dim3(grid_for(n / 8, 512)), dim3(kThreads), 0, stream, wide, n,
+                       wide_depth(n), out);
+  hipLaunchKernelGGL(k_cost_finish, dim3(1), dim3(1), 0, stream, wide, out);
   return hipGetLastError();
 }
 

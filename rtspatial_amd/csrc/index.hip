@@ -96,6 +96,13 @@ int ensure_id_capacity(rts_index* ix, uint64_t need, hipStream_t stream) {
   return RTS_OK;
 }
 
+// Entries of a packed tree's node array over up to n leaves.
+uint64_t wide_words(uint64_t n) { return wide_leaf0(wide_depth(n)) + (uint64_t)(kFan - 1); }
+// Leaves a delta tree may have next to a main tree in arrays of `cap` leaves.
+uint64_t delta_cap(const rts_index* ix, uint64_t cap) {
+  return std::min<uint64_t>(cap, cap * ix->cfg.insert_delta_pct / 100);
+}
+
 int ensure_tree_capacity(rts_index* ix, uint64_t n) {
   if (n <= ix->tcap) return RTS_OK;
   RTS_HIP(hipDeviceSynchronize());
@@ -107,11 +114,10 @@ int ensure_tree_capacity(rts_index* ix, uint64_t n) {
   dev_free(ix->keys);
   dev_free(ix->keys_alt);
   dev_free(ix->vals_alt);
-  dev_free(ix->nodes);
-  dev_free(ix->parent);
-  dev_free(ix->node_end);
-  dev_free(ix->top);
-  dev_free(ix->flags);
+  dev_free(ix->wide_mem);
+  dev_free(ix->wide_live);
+  dev_free(ix->delta_wide_mem);
+  dev_free(ix->delta_wide_live);
   dev_free(ix->sort_scratch);
   dev_free(ix->partials);
   RTS_HIP(dev_alloc(&ix->leaf_boxes, cap));
@@ -119,11 +125,11 @@ int ensure_tree_capacity(rts_index* ix, uint64_t n) {
   RTS_HIP(dev_alloc(&ix->keys, cap));
   RTS_HIP(dev_alloc(&ix->keys_alt, cap));
   RTS_HIP(dev_alloc(&ix->vals_alt, cap));
-  RTS_HIP(dev_alloc(&ix->nodes, cap));
-  RTS_HIP(dev_alloc(&ix->parent, 2 * cap));
-  RTS_HIP(dev_alloc(&ix->node_end, cap));
-  RTS_HIP(dev_alloc(&ix->top, kTopPairs));
-  RTS_HIP(dev_alloc(&ix->flags, cap + refit_boundary_words(cap)));
+  RTS_HIP(dev_alloc(&ix->wide_mem, wide_words(cap)));
+  RTS_HIP(dev_alloc(&ix->wide_live, wide_words(cap)));
+  const uint64_t dcap = delta_cap(ix, cap);
+  RTS_HIP(dev_alloc(&ix->delta_wide_mem, dcap ? wide_words(dcap) : 0));
+  RTS_HIP(dev_alloc(&ix->delta_wide_live, dcap ? wide_words(dcap) : 0));
   RTS_HIP(dev_alloc(&ix->sort_scratch, sort_scratch_bytes(cap)));
   sort_scratch_carve(ix->sort_scratch, cap, &ix->ss);
   ix->n_partials_cap = scene_bounds_partials((uint32_t)cap);
@@ -156,7 +162,7 @@ int measure_cost(rts_index* ix, bool after_build, hipStream_t stream) {
   } else if (ix->cost_refit_pending || ix->cost_build_pending) {
     return RTS_OK;  // a measurement is still in flight; skip this one
   }
-  RTS_HIP(launch_tree_cost(ix->nodes, ix->root_box, (uint32_t)ix->n_main, ix->cost, stream));
+  RTS_HIP(launch_tree_cost(ix->wide(), (uint32_t)ix->n_main, ix->cost, stream));
   double* dst = after_build ? ix->h_cost : ix->h_cost + 2;
   RTS_HIP(hipMemcpyAsync(dst, ix->cost, 2 * sizeof(double), hipMemcpyDeviceToHost, stream));
   if (after_build) {
@@ -170,24 +176,63 @@ int measure_cost(rts_index* ix, bool after_build, hipStream_t stream) {
   return RTS_OK;
 }
 
-// Refit of the main tree, or (delta) of the delta tree, whose leaves, nodes
-// and parents start at n_main, n_main and 2 n_main. Both share the flag and
-// boundary words; refits run one after the other on a stream.
-RefitArgs refit_args(rts_index* ix, bool delta) {
+// The packed tree of the main leaves, or (delta) of the delta tree's, which
+// start at position n_main; with `gather`, from the boxes by id (a build).
+WideArgs wide_args(rts_index* ix, bool delta, bool gather) {
   const uint64_t off = delta ? ix->n_main : 0;
-  RefitArgs a;
+  WideArgs a;
   a.leaf_boxes = ix->leaf_boxes + off;
   a.n = (uint32_t)(delta ? ix->n_delta : ix->n_main);
-  a.parent = ix->parent + 2 * off;
-  a.node_end = ix->node_end + off;
-  a.top = delta ? nullptr : ix->top;
-  a.nodes = ix->nodes + off;
-  a.root_box = delta ? ix->delta_root_box : ix->root_box;
-  a.root_live = delta ? ix->delta_root_live : ix->root_live;
+  a.wide = delta ? ix->delta_wide() : ix->wide();
+  a.wide_live = delta ? ix->delta_wide_live : ix->wide_live;
+  a.error = ix->error;
+  if (gather) {
+    a.boxes = ix->boxes;
+    a.ids = ix->leaf_ids + off;
+    a.off = (uint32_t)off;
+    a.leaf_of_id = ix->leaf_of_id;
+  }
+  return a;
+}
+
+// Brings the binary tree over the main tree's leaves up to date; there is no
+// delta tree (ensure_built with `single`).
+int ensure_binary(rts_index* ix, hipStream_t stream) {
+  if (ix->bcap < ix->n_main) {
+    RTS_HIP(hipDeviceSynchronize());
+    dev_free(ix->nodes);
+    dev_free(ix->parent);
+    dev_free(ix->node_end);
+    dev_free(ix->flags);
+    ix->bcap = 0;
+    ix->bin_valid = false;
+    RTS_HIP(dev_alloc(&ix->nodes, ix->tcap));
+    RTS_HIP(dev_alloc(&ix->parent, 2 * ix->tcap));
+    RTS_HIP(dev_alloc(&ix->node_end, ix->tcap));
+    RTS_HIP(dev_alloc(&ix->flags, ix->tcap + refit_boundary_words(ix->tcap)));
+    ix->bcap = ix->tcap;
+  }
+  const uint32_t n = (uint32_t)ix->n_main;
+  if (ix->bin_valid && !ix->bin_refit_needed) return RTS_OK;
+  PhaseToken ph = phase_begin(ix->bin_valid ? RTS_PHASE_REFIT : RTS_PHASE_BUILD_TREE, stream);
+  if (!ix->bin_valid)
+    RTS_HIP(launch_karras(ix->keys, n, ix->nodes, ix->parent, ix->node_end, stream));
+  RefitArgs a;
+  a.leaf_boxes = ix->leaf_boxes;
+  a.n = n;
+  a.parent = ix->parent;
+  a.node_end = ix->node_end;
+  a.nodes = ix->nodes;
+  a.root_box = ix->root_box;
+  a.root_live = ix->root_live;
   a.flags = ix->flags;
   a.error = ix->error;
-  a.boundary = ix->flags + ix->tcap;  // after the n - 1 node flags
-  return a;
+  a.boundary = ix->flags + ix->bcap;  // after the n - 1 node flags
+  RTS_HIP(launch_refit(a, stream));
+  phase_end(ph, stream);
+  ix->bin_valid = true;
+  ix->bin_refit_needed = false;
+  return RTS_OK;
 }
 
 int build_tree(rts_index* ix, hipStream_t stream) {
@@ -203,7 +248,7 @@ int build_tree(rts_index* ix, hipStream_t stream) {
   const uint32_t parts = scene_bounds_partials(n);
   PhaseToken ph = phase_begin(RTS_PHASE_BUILD_MORTON, stream);
   RTS_HIP(launch_scene_bounds(ix->boxes, n, ix->partials, parts, ix->scene, stream));
-  RTS_HIP(launch_morton_boxes(ix->boxes, n, ix->scene, ix->keys, stream));
+  RTS_HIP(launch_hilbert_boxes(ix->boxes, n, ix->scene, ix->keys, stream));
   phase_end(ph, stream);
   bool in_b = false;
   ph = phase_begin(RTS_PHASE_BUILD_SORT, stream);
@@ -215,16 +260,10 @@ int build_tree(rts_index* ix, hipStream_t stream) {
     std::swap(ix->leaf_ids, ix->vals_alt);
   }
   ph = phase_begin(RTS_PHASE_BUILD_TREE, stream);
-  RTS_HIP(launch_karras(ix->keys, n, ix->nodes, ix->parent, ix->node_end, stream));
   ix->n_main = N;
   ix->n_delta = 0;
-  RefitArgs ra = refit_args(ix, false);  // the refit also gathers the leaves
-  ra.gather = true;
-  ra.boxes = ix->boxes;
-  ra.ids = ix->leaf_ids;
-  ra.off = 0;
-  ra.leaf_of_id = ix->leaf_of_id;
-  RTS_HIP(launch_refit(ra, stream));
+  ix->bin_valid = false;
+  RTS_HIP(launch_wide_tree(wide_args(ix, false, true), stream));
   phase_end(ph, stream);
   ix->n_tree = N;
   ix->stale = false;
@@ -245,7 +284,7 @@ int build_delta(rts_index* ix, hipStream_t stream) {
   const uint32_t parts = scene_bounds_partials(nd);
   PhaseToken ph = phase_begin(RTS_PHASE_BUILD_MORTON, stream);
   RTS_HIP(launch_scene_bounds(ix->boxes + off, nd, ix->partials, parts, ix->delta_scene, stream));
-  RTS_HIP(launch_morton_boxes(ix->boxes + off, nd, ix->delta_scene, ix->keys + off, stream));
+  RTS_HIP(launch_hilbert_boxes(ix->boxes + off, nd, ix->delta_scene, ix->keys + off, stream));
   phase_end(ph, stream);
   bool in_b = false;
   ph = phase_begin(RTS_PHASE_BUILD_SORT, stream);
@@ -259,16 +298,8 @@ int build_delta(rts_index* ix, hipStream_t stream) {
                            hipMemcpyDeviceToDevice, stream));
   }
   ph = phase_begin(RTS_PHASE_BUILD_TREE, stream);
-  RTS_HIP(launch_karras(ix->keys + off, nd, ix->nodes + off, ix->parent + 2 * off,
-                        ix->node_end + off, stream));
   ix->n_delta = nd;
-  RefitArgs ra = refit_args(ix, true);  // the refit also gathers the leaves
-  ra.gather = true;
-  ra.boxes = ix->boxes;
-  ra.ids = ix->leaf_ids + off;
-  ra.off = (uint32_t)off;
-  ra.leaf_of_id = ix->leaf_of_id;
-  RTS_HIP(launch_refit(ra, stream));
+  RTS_HIP(launch_wide_tree(wide_args(ix, true, true), stream));
   phase_end(ph, stream);
   ix->n_tree = ix->n;
   ix->delta_builds++;
@@ -301,6 +332,7 @@ constexpr uint64_t kRebuildUpdateShare = 200;
 // `updated`: boxes given new envelopes (0 for deletes, which only shrink
 // node bounds).
 int after_mutation(rts_index* ix, uint64_t updated) {
+  ix->bin_refit_needed = true;
   if (ix->stale) return RTS_OK;  // the next query rebuilds anyway
   if (ix->cfg.rebuild_policy == RTS_REBUILD_ALWAYS) {
     ix->stale = true;
@@ -320,8 +352,8 @@ int after_mutation(rts_index* ix, uint64_t updated) {
 int refit_tree(rts_index* ix, hipStream_t stream) {
   ix->refit_needed = false;
   PhaseToken ph = phase_begin(RTS_PHASE_REFIT, stream);
-  RTS_HIP(launch_refit(refit_args(ix, false), stream));
-  if (ix->n_delta) RTS_HIP(launch_refit(refit_args(ix, true), stream));
+  RTS_HIP(launch_wide_tree(wide_args(ix, false, false), stream));
+  if (ix->n_delta) RTS_HIP(launch_wide_tree(wide_args(ix, true, false), stream));
   phase_end(ph, stream);
   ix->refits++;
   if (ix->cfg.rebuild_policy == RTS_REBUILD_SAH) return measure_cost(ix, false, stream);
@@ -349,6 +381,21 @@ int check_device_error(rts_index* ix) {
 
 namespace rts {
 
+// The number of leaves and what the walks derive from it.
+static void set_leaves(TreeView& t, uint64_t n) {
+  t.n = (uint32_t)n;
+  t.depth = wide_depth(n);
+  t.leaf0 = wide_leaf0(t.depth);
+  // The deepest level of at most kWave nodes: wave walks start there.
+  for (uint32_t d = 0; d < t.depth; d++) {
+    const uint32_t shift = 3 * (t.depth - d);
+    const uint64_t m = (n + (1ull << shift) - 1) >> shift;
+    if (m > (uint64_t)kWave) break;
+    t.start = wide_level0(d);
+    t.start_n = (uint32_t)m;
+  }
+}
+
 TreeView tree_view(const rts_index* ix) {
   TreeView t;
   t.leaf_boxes = ix->leaf_boxes;
@@ -356,12 +403,12 @@ TreeView tree_view(const rts_index* ix) {
   t.nodes = ix->nodes;
   t.root_box = ix->root_box;
   t.root_live = ix->root_live;
-  t.n = (uint32_t)ix->n_main;
   t.leaf_size = ix->cfg.leaf_size;
   t.error = ix->error;
   t.boxes64 = ix->cfg.coord == RTS_COORD_F64 ? ix->boxes64 : nullptr;
-  // The top is rebuilt by every refit of the main tree (builds included).
-  t.top = ix->n_main >= kTopMinLeaves ? ix->top : nullptr;
+  t.wide = ix->wide();
+  t.wide_live = ix->wide_live;
+  set_leaves(t, ix->n_main);
   return t;
 }
 
@@ -370,11 +417,10 @@ TreeView delta_view(const rts_index* ix) {
   const uint64_t off = ix->n_main;
   t.leaf_boxes = ix->leaf_boxes + off;
   t.leaf_ids = ix->leaf_ids + off;
-  t.nodes = ix->nodes + off;
-  t.root_box = ix->delta_root_box;
-  t.root_live = ix->delta_root_live;
-  t.n = (uint32_t)ix->n_delta;
-  t.top = nullptr;  // the delta tree is walked from its root
+  t.nodes = nullptr;  // there is no binary tree over it
+  t.wide = ix->delta_wide();
+  t.wide_live = ix->delta_wide_live;
+  set_leaves(t, ix->n_delta);
   return t;
 }
 
@@ -448,8 +494,6 @@ int rts_index_create(const rts_config* cfg, rts_index** out) {
   ix->error = reinterpret_cast<uint32_t*>(ix->small + 64);
   ix->root_live = reinterpret_cast<uint32_t*>(ix->small + 80);
   ix->delta_scene = reinterpret_cast<float4*>(ix->small + 96);
-  ix->delta_root_box = reinterpret_cast<float4*>(ix->small + 112);
-  ix->delta_root_live = reinterpret_cast<uint32_t*>(ix->small + 128);
   RTS_HIP(hipMemset(ix->small, 0, 256));
   // Complete before any stream (including non-blocking ones) uses the index.
   RTS_HIP(hipDeviceSynchronize());
@@ -482,8 +526,11 @@ int rts_index_destroy(rts_index* ix) {
   dev_free(ix->nodes);
   dev_free(ix->parent);
   dev_free(ix->node_end);
-  dev_free(ix->top);
   dev_free(ix->flags);
+  dev_free(ix->wide_mem);
+  dev_free(ix->wide_live);
+  dev_free(ix->delta_wide_mem);
+  dev_free(ix->delta_wide_live);
   dev_free(ix->sort_scratch);
   dev_free(ix->partials);
   dev_free(ix->small);
@@ -753,12 +800,15 @@ struct Plan {
 // The plan of a query call. Explicit config settings win; a plan stored by
 // rts_index_autotune fills the settings left on auto; otherwise: one query
 // per wavefront where queries have many results (envelope intersects /
-// within), one per lane otherwise (points, envelope contains), and Morton
-// ordering of batches of 64K queries or more (neighbouring lanes share their
-// descent; neighbouring waves, which take consecutive queries on one XCD,
-// share that XCD's L2).
-// Calls of at least this many queries are Morton-ordered unless a tuning
-// moved the threshold (TunedPlan::sort_min_n).
+// within), one per octet of lanes otherwise (points, envelope contains), and
+// Morton ordering of wavefront batches of 64K queries or more (neighbouring
+// waves, which take consecutive queries on one XCD, share that XCD's L2: the
+// 10M x 1M join counts in 4.6 ms with the order and 7.7 ms without). Octet
+// walks keep the input order: ordering 1M points costs 0.11 ms and made their
+// walk no faster at 1M (2.01 against 1.36 ms for 10M points), 10M (2.61
+// against 1.88) and 60M boxes (4.06 against 3.79); at 100M boxes it gains 3%.
+// Wavefront calls of at least this many queries are Morton-ordered unless a
+// tuning moved the threshold (TunedPlan::sort_min_n).
 constexpr uint64_t kSortMinQueries = 65536;
 // The autotuner times query ordering on the whole query set up to this size.
 constexpr uint64_t kOrderTuneQueries = 1ull << 22;
@@ -780,7 +830,7 @@ Plan plan_query(const rts_index* ix, int pred, bool points, uint64_t nq) {
   else if (t.valid && t.sort_tuned)
     p.sort = nq >= t.sort_min_n;
   else
-    p.sort = nq >= kSortMinQueries;
+    p.sort = p.traversal == RTS_TRAVERSAL_WAVE && nq >= kSortMinQueries;
   p.leaf_size = t.valid ? t.leaf_size : ix->cfg.leaf_size;
   return p;
 }
@@ -1128,6 +1178,7 @@ int rts_index_tree_view(rts_index* ix, rts_stream_t stream, rts_tree_view* out) 
   out->leaf_size = ix->cfg.leaf_size;
   if (ix->n == 0) return RTS_OK;
   int rc = ensure_built(ix, stream, true);  // one tree: a delta tree is merged first
+  if (!rc) rc = ensure_binary(ix, stream);
   if (rc) return rc;
   const TreeView t = tree_view(ix);
   out->leaf_boxes = t.leaf_boxes;
@@ -1185,12 +1236,14 @@ int rts_index_memory(rts_index* ix, rts_memory_usage* out) {
   const uint64_t cap = ix->cap, t = ix->tcap;
   out->geometries = cap * (sizeof(float4) + sizeof(uint32_t)) + (ix->boxes64 ? cap * sizeof(Box64) : 0);
   out->aabbs = t * sizeof(float4);
-  out->bvh = t ? (t * sizeof(uint32_t) * 4                      // leaf ids, keys, keys/vals alt
-                  + t * sizeof(NodeRec) + 3 * t * sizeof(uint32_t) // nodes, parents, far ends
-                  + kTopPairs * sizeof(NodeRec)                     // the tree's top
-                  + (t + refit_boundary_words(t)) * sizeof(uint32_t) // flags + boundary list
+  const uint64_t d = t ? delta_cap(ix, t) : 0, b = ix->bcap;
+  out->bvh = t ? (t * sizeof(uint32_t) * 4  // leaf ids, keys, keys/vals alt
+                  + (wide_words(t) + (d ? wide_words(d) : 0)) * (sizeof(float4) + sizeof(uint32_t))
                   + sort_scratch_bytes(t) + ix->n_partials_cap * sizeof(float4))
                : 0;
+  if (b)  // the binary tree: nodes, parents, far ends, flags and boundary list
+    out->bvh += b * sizeof(NodeRec) + 3 * b * sizeof(uint32_t) +
+                (b + refit_boundary_words(b)) * sizeof(uint32_t);
   out->total = out->geometries + out->aabbs + out->bvh + 256;
   return RTS_OK;
 }

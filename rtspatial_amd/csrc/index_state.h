@@ -24,9 +24,8 @@ struct rts_index {
   // Trees (valid for n_tree leaves unless stale). The main tree holds ids
   // [0, n_main) at sorted positions [0, n_main); a small delta tree of boxes
   // inserted since the last full build holds ids [n_main, n_tree) at
-  // positions [n_main, n_tree) of the same leaf arrays, its nodes at
-  // nodes[n_main ...] and its parents at parent[2 n_main ...]. Ids in
-  // [n_tree, n) are inserted but in no tree yet.
+  // positions [n_main, n_tree) of the same leaf arrays, with nodes of its own.
+  // Ids in [n_tree, n) are inserted but in no tree yet.
   uint64_t tcap = 0;
   uint64_t n_tree = 0;
   uint64_t n_main = 0;
@@ -38,10 +37,23 @@ struct rts_index {
   uint32_t* keys = nullptr;
   uint32_t* keys_alt = nullptr;
   uint32_t* vals_alt = nullptr;
+  // Packed nodes (tree.h) of the main and the delta tree: boxes, allocated
+  // kFan - 1 entries ahead so that child octets start on a 128-byte line, and
+  // live counts.
+  float4* wide_mem = nullptr;
+  uint32_t* wide_live = nullptr;
+  float4* delta_wide_mem = nullptr;
+  uint32_t* delta_wide_live = nullptr;
+  float4* wide() const { return wide_mem + (rts::kFan - 1); }
+  float4* delta_wide() const { return delta_wide_mem + (rts::kFan - 1); }
+  // Binary tree over the main tree's leaves, for caller-compiled handlers:
+  // allocated and built by the first rts_index_tree_view after a build.
+  uint64_t bcap = 0;
+  bool bin_valid = false;         // it has the current leaves' hierarchy
+  bool bin_refit_needed = false;  // boxes changed in place since it was fitted
   rts::NodeRec* nodes = nullptr;
   uint32_t* parent = nullptr;
   uint32_t* node_end = nullptr;  // far end of each internal node's leaf range (refit meta)
-  rts::NodeRec* top = nullptr;   // the main tree's top (kTopPairs records)
   uint32_t* flags = nullptr;
   char* sort_scratch = nullptr;
   rts::SortScratch ss{};
@@ -54,8 +66,6 @@ struct rts_index {
   float4* root_box = nullptr;
   uint32_t* root_live = nullptr;
   float4* delta_scene = nullptr;
-  float4* delta_root_box = nullptr;
-  uint32_t* delta_root_live = nullptr;
   double* cost = nullptr;
   uint32_t* error = nullptr;  // device error bits (kErr*)
 

@@ -1,10 +1,14 @@
-// Range logs of two-pass wave walks (traverse.h RangeLog), laid out per
-// wavefront: each persistent wave of a count pass appends the entries of the
-// queries it walks to its own region of the log (per_wave entries, one wave
-// per workgroup), and each query records where its entries
-// start and how many there are. The write pass replays a query's entries
-// instead of walking the tree. A query whose entries do not fit -- more than
-// kLogQueryMax, or past the end of its wave's region -- is walked again.
+// Range logs of two-pass wave walks: what a query's counting walk found, so
+// that its write pass emits the results without walking or testing again.
+// Each persistent wave of a count pass appends the entries of the queries it
+// walks to its own region of the log (per_wave entries, one wave per
+// workgroup), and each query records where its entries start and how many
+// there are. A query whose entries do not fit -- more than kLogQueryMax, or
+// past the end of its wave's region -- is walked again by the write pass.
+//
+// An entry is 8 bytes: {first leaf, mask} for a block of 8 leaves whose bits
+// in `mask` are results, or {first leaf | kLogRange, leaves} for a run of
+// leaves that all are.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,6 +21,27 @@
 namespace rts {
 
 constexpr uint32_t kLogQueryMax = 4096;
+constexpr uint32_t kLogOverflow = 0xFFFFFFFFu;
+constexpr uint32_t kLogRange = 0x80000000u;
+
+// Log entries bypass the caches both ways (written once, read once), so
+// that they do not evict the nodes and leaf data the walks re-read.
+__device__ __forceinline__ void log_store(uint2* p, uint32_t x, uint32_t y) {
+  __builtin_nontemporal_store(((uint64_t)y << 32) | x, reinterpret_cast<uint64_t*>(p));
+}
+__device__ __forceinline__ uint2 log_load(const uint2* p) {
+  const uint64_t v = __builtin_nontemporal_load(reinterpret_cast<const uint64_t*>(p));
+  return make_uint2((uint32_t)v, (uint32_t)(v >> 32));
+}
+
+// The log of one walk: a counting walk appends up to `cap` entries and sets
+// `logged` to the number it found (more than cap: they did not all fit).
+struct RangeLog {
+  uint2* entries = nullptr;
+  uint32_t cap = 0;
+  uint32_t logged = 0;           // counting walk (wave-uniform)
+  uint32_t n_in = kLogOverflow;  // writing walk: entries to emit (kLogOverflow: walk the tree)
+};
 
 // A count-pass wave's place in its region.
 struct LogCursor {

@@ -50,6 +50,26 @@ hipError_t launch_scene_bounds(const float4* boxes, uint32_t n, float4* partials
 uint32_t scene_bounds_partials(uint32_t n);
 hipError_t launch_morton_boxes(const float4* boxes, uint32_t n, const float4* scene,
                                uint32_t* keys, hipStream_t stream);
+hipError_t launch_hilbert_boxes(const float4* boxes, uint32_t n, const float4* scene,
+                                uint32_t* keys, hipStream_t stream);
+// The packed tree over n leaves (tree.h), from leaf_boxes; with `boxes`, leaf
+// k's box is first gathered: boxes[id] with id = ids[k] + off (ids counted
+// from off, rewritten to the ids themselves when off > 0), stored to
+// leaf_boxes[k], and leaf_of_id[id] = off + k. off > 0 places a delta tree
+// over ids [off, off + n) at positions [off, off + n): leaf_boxes and ids are
+// then passed advanced by off.
+struct WideArgs {
+  float4* leaf_boxes;
+  uint32_t n;
+  float4* wide;  // wide_leaf0(wide_depth(n)) entries and the last octet's end
+  uint32_t* wide_live;
+  uint32_t* error;
+  const float4* boxes = nullptr;
+  uint32_t* ids = nullptr;
+  uint32_t off = 0;
+  uint32_t* leaf_of_id = nullptr;
+};
+hipError_t launch_wide_tree(const WideArgs& a, hipStream_t stream);
 hipError_t launch_morton_points(const float2* pts, uint32_t n, const float4* scene,
                                 uint32_t* keys, hipStream_t stream);
 // Every stride-th element of src (elem_bytes 8, 16 or 32) into dst[0, m).
@@ -62,7 +82,7 @@ hipError_t launch_gather_strided(const void* src, uint32_t elem_bytes, uint64_t 
 hipError_t launch_karras(const uint32_t* sorted_keys, uint32_t n, NodeRec* nodes, uint32_t* parent,
                          uint32_t* node_end, hipStream_t stream);
 struct RefitArgs {
-  float4* leaf_boxes;
+  const float4* leaf_boxes;
   uint32_t n;
   const uint32_t* parent;
   NodeRec* nodes;
@@ -72,17 +92,6 @@ struct RefitArgs {
   uint32_t* error;
   uint32_t* boundary;  // refit_boundary_words(n): per-chunk boundary slots, then the top list
   const uint32_t* node_end;  // the hierarchy kernel's far ends (records' meta)
-  NodeRec* top = nullptr;    // main tree of kTopMinLeaves or more: its top, rebuilt after the refit
-  // Build refits also gather the leaves: leaf k's box is boxes[id] with
-  // id = ids[k] + off (ids counted from off, rewritten to the ids themselves
-  // when off > 0), stored to leaf_boxes[k], and leaf_of_id[id] = off + k. off
-  // > 0 places a delta tree over ids [off, off + n) at positions [off, off +
-  // n): leaf_boxes and ids are then passed advanced by off.
-  bool gather = false;
-  const float4* boxes = nullptr;
-  uint32_t* ids = nullptr;
-  uint32_t off = 0;
-  uint32_t* leaf_of_id = nullptr;
 };
 // Refit chunks: C = 2^refit_chunk_log2(n) leaves per level-1 workgroup, whose
 // LDS holds 24 bytes per node of the chunk (48 KB at 2048 leaves).
@@ -107,10 +116,8 @@ __host__ __device__ inline uint64_t refit_boundary_words(uint64_t n) {
   return (n / 2048 + 1) * kRefitChunkStride + refit_top_words(n);
 }
 hipError_t launch_refit(const RefitArgs& a, hipStream_t stream);
-// Trees of at least this many leaves get a top (TreeView::top) for the wave walks.
-constexpr uint32_t kTopMinLeaves = 4096;
-hipError_t launch_tree_cost(const NodeRec* nodes, const float4* root_box, uint32_t n,
-                            double* out, hipStream_t stream);
+// out[0] = the packed tree's summed half-perimeters, out[1] = its cost.
+hipError_t launch_tree_cost(const float4* wide, uint32_t n, double* out, hipStream_t stream);
 hipError_t launch_delete(const uint64_t* ids, uint64_t n_ids, float4* boxes, uint64_t n_boxes,
                          float4* leaf_boxes, const uint32_t* leaf_of_id, uint64_t n_tree,
                          Box64* boxes64, hipStream_t stream);
@@ -169,7 +176,13 @@ struct WaveArgs {
   uint32_t* tickets;  // kWaveTicketWords words, cleared by the launch
   RangeLogArgs log;   // two-pass calls: the count walks' range logs
 };
-constexpr uint32_t kWaveTicketWords = 8 * 16;
+// Tickets (one 64-byte line per XCD), then the counting launches' kSumSlots
+// partial sums.
+constexpr uint32_t kSumSlots = 64;
+constexpr uint32_t kWaveTicketWords = 8 * 16 + 2 * kSumSlots;
+__host__ __device__ inline unsigned long long* wave_sums(uint32_t* tickets) {
+  return reinterpret_cast<unsigned long long*>(tickets + 8 * 16);
+}
 // Wave-per-query traversal. phase 0: per-query counts -> a.counts;
 // 1: counts added to the counting handler's counter; 2: pairs written at
 // queue slot a.base[0] + a.offsets[query]; 3: pairs collected in one pass

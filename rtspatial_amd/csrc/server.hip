@@ -367,7 +367,7 @@ int copy_out(Engine& E, const Chunk& c, const rts_pair* src, const BatchArgs* ba
   return RTS_OK;
 }
 
-// Tile mode and leaf-range size of a request: the serve config's traversal
+// Tile mode of a request: the serve config's traversal
 // if it names one, else the plan stored by rts_index_autotune for this
 // (predicate, query kind), else one query per wavefront for envelope
 // intersects / within and 64 per tile otherwise.
@@ -385,11 +385,6 @@ uint32_t tile_flags(const Engine& E, const rts_request& r) {
   else
     wave = !pts && r.predicate != RTS_CONTAINS;
   if (wave) f |= kReqWaveTiles;
-  if (tp.valid && tp.leaf_size >= 1 && tp.leaf_size <= 64) {
-    uint32_t lg = 0;
-    while ((2u << lg) <= tp.leaf_size) lg++;
-    f |= (lg + 1) << kReqLeafShift;
-  }
   return f;
 }
 
@@ -664,9 +659,6 @@ int launch_slot(Engine& E, Slot& s, std::vector<Chunk> chunks) {
       x.ql.f64 = E.ix->f64() ? 1 : 0;
       x.ql.sink = SinkArgs{RTS_HANDLER_COUNT, nullptr};
       x.ql.traversal = RTS_TRAVERSAL_WAVE;
-      const rts_index::TunedPlan& tp = E.ix->tuned[r.predicate & 3][r.points == kPoints ? 1 : 0];
-      x.ql.tree.leaf_size =
-          (!seg && tp.valid && tp.leaf_size >= 1) ? tp.leaf_size : E.ix->cfg.leaf_size;
       x.qbase = qb;
       x.none = seg && r.predicate != RTS_INTERSECTS;  // no box lies inside a segment
       s.ext.push_back(x);

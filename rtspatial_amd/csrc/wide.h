@@ -1,0 +1,376 @@
+// Walks of the packed tree (TreeView::wide, tree.h).
+//
+// A step of either walk gives each of the wave's eight octets (8 lanes) one
+// node: the octet reads the node's eight child boxes as one 128-byte line,
+// one box per lane, and tests them together. Child and leaf addresses follow
+// from the heap index, so a step depends on memory once.
+//
+//   oct_walk    one query per octet, depth first: few results per query.
+//   wide_walk   one query per wavefront, kWideRounds x 8 nodes per step, each
+//               lane with kWideRounds independent loads in flight.
+//   wide_replay emits what a counting wide_walk logged (range_log.h).
+//
+// Node tests are necessary conditions of the leaf predicate on exact bounds
+// (traverse.h), and a run of leaves is taken whole only when its node lies
+// inside the query and every leaf of it is live. No index read from memory
+// steers a walk, and every pop is strictly deeper than the last on its path,
+// so a walk ends within the tree's nodes.
+#pragma once
+
+#include "range_log.h"
+#include "rtspatial/device/traverse.h"
+#include "rtspatial/device/wave.h"
+
+namespace rts {
+
+// A float query whose predicate is chosen at run time: RTS_INTERSECTS,
+// RTS_WITHIN or RTS_CONTAINS (data box contains the query). A point is the
+// degenerate envelope (x, y, x, y) under RTS_CONTAINS: contains_box(b, (x, y,
+// x, y)) is contains_point(b, x, y) comparison for comparison, and no subtree
+// lies inside a point. The persistent batch kernel answers every request kind
+// with one instantiation of each walk this way; `pred` is the same for every
+// lane of a wave (a request's), so the tests branch on scalar registers.
+struct QueryRT {
+  float4 b;
+  int pred;
+};
+template <int PRED, bool POINTS>
+__device__ __forceinline__ bool node_test(const float4 n, const QueryRT& q) {
+  return q.pred == RTS_CONTAINS ? contains_box(n, q.b) : intersects(n, q.b);
+}
+template <int PRED, bool POINTS>
+__device__ __forceinline__ bool inside_test(const float4 n, const QueryRT& q) {
+  return q.pred != RTS_CONTAINS && contains_box(q.b, n);
+}
+template <int PRED, bool POINTS>
+__device__ __forceinline__ bool leaf_test(const TreeView&, uint32_t, const float4 b,
+                                          const QueryRT& q) {
+  if (q.pred == RTS_INTERSECTS) return intersects(b, q.b);
+  if (q.pred == RTS_WITHIN) return contains_box(q.b, b);
+  return contains_box(b, q.b);
+}
+
+// -------------------------------------------------------------- tickets ----
+// Wave kernels take queries from per-XCD ticket counters as grab_query
+// (traverse.h) does, but the first three quarters of a slice kTicketQueries at
+// a time: a counter answers one atomic per ~14 ns, which at one query each
+// bounds a pass over 1M queries at 1.7 ms. The last quarter goes singly, so
+// that a heavy group is not left to one wave at the end.
+constexpr uint32_t kTicketQueries = 4;
+
+// The next queries [*begin, *end) for this wave; empty when every slice is
+// drained. `slice` is the slice to try first; it becomes the one taken from.
+__device__ __forceinline__ void grab_queries(uint32_t* tickets, uint32_t n, uint32_t& slice,
+                                             uint32_t* begin, uint32_t* end) {
+  const uint32_t per = (n + kXcds - 1) / kXcds;
+  uint32_t b = 0, e = 0, from = slice;
+  if (lane_id() == 0) {
+    for (uint32_t k = 0; k < kXcds; k++) {
+      const uint32_t x = (slice + k) % kXcds;
+      const uint32_t lo = x * per;
+      const uint32_t hi = lo + per < n ? lo + per : n;
+      if (lo >= hi) continue;
+      const uint32_t m = hi - lo;
+      const uint32_t groups = m / 4 * 3 / kTicketQueries;
+      const uint32_t v = atomicAdd(tickets + x * kTicketStride, 1u);
+      if (v < groups) {
+        b = lo + v * kTicketQueries;
+        e = b + kTicketQueries;
+        from = x;
+        break;
+      }
+      const uint32_t single = groups * kTicketQueries + (v - groups);
+      if (single < m) {
+        b = lo + single;
+        e = b + 1;
+        from = x;
+        break;
+      }
+    }
+  }
+  slice = readlane_u32(from, 0);
+  *begin = readlane_u32(b, 0);
+  *end = readlane_u32(e, 0);
+}
+
+// Level of heap index i, and the leaves below node i: 8^(D - level) of them
+// from `first`, cut at n.
+__device__ __forceinline__ uint32_t wide_level(uint32_t i) {
+  return (31u - (uint32_t)__builtin_clz(7u * i + 1u)) / 3u;
+}
+__device__ __forceinline__ void wide_leaves(const TreeView& t, uint32_t i, uint32_t* first,
+                                            uint32_t* count) {
+  const uint32_t lv = wide_level(i), shift = 3u * (t.depth - lv);
+  const uint32_t f = (i - wide_level0(lv)) << shift;
+  const uint32_t left = t.n - f;
+  *first = f;
+  *count = (1u << shift) < left ? (1u << shift) : left;
+}
+
+__device__ __forceinline__ float4 nan_box() {
+  const float x = __builtin_nanf("");
+  return make_float4(x, x, x, x);
+}
+
+// ---------------------------------------------------------------- octet ----
+// Depth-first stack of one octet: a pop pushes at most 8 and each level
+// leaves at most 7 behind, so 1 + 7 (kMaxDepth - 1) entries suffice.
+constexpr int kOctStack = 64;
+static_assert(1 + 7 * (kMaxDepth - 1) <= kOctStack, "octet stack");
+
+// The wave answers queries [first, last): octet o takes first + o, first + o
+// + 8, ... `src(i, q)` loads query i; `sink.hits(...)` is called by the whole
+// wave at every step that found results, and `sink.finish(i, found)` by an
+// octet that completed query i. COUNT walks count subtrees inside the query
+// from their live counts. `stack` is this octet's, in LDS.
+template <int PRED, bool POINTS, bool COUNT, typename Q, typename Src, typename Sink>
+__device__ void oct_walk(const TreeView& t, uint32_t* stack, uint32_t first, uint32_t last,
+                         const Src& src, Sink& sink) {
+  const uint32_t lane = lane_id(), j = lane & 7u, oct = lane >> 3;
+  uint32_t i = first + oct;
+  bool have = i < last;
+  Q q{}, qn{};
+  if (have) src(i, q);
+  // The next query's load is in flight while this one is walked.
+  if (i + kFan < last) src(i + kFan, qn);
+  uint32_t sp = have ? 1u : 0u;  // octet-uniform
+  uint32_t found = 0;            // octet-uniform
+  if (have && j == 0) stack[0] = 0;
+  lds_fence();
+  while (ballot(have)) {
+    const uint32_t e = have ? stack[sp - 1] : 0u;
+    const uint32_t child = kFan * e + 1u + j;
+    const bool at_leaf = child >= t.leaf0;  // octet-uniform
+    const uint32_t leaf = child - t.leaf0;
+    const bool ok = have && (!at_leaf || leaf < t.n);
+    float4 b = nan_box();
+    uint32_t gid = 0;
+    if (ok) {
+      b = *(at_leaf ? t.leaf_boxes + leaf : t.wide + child);
+      if (!COUNT && at_leaf) gid = t.leaf_ids[leaf];
+    }
+    bool hit = false;
+    if (ok) hit = at_leaf ? leaf_test<PRED, POINTS>(t, leaf, b, q) : node_test<PRED, POINTS>(b, q);
+    if (COUNT && !POINTS) {
+      const bool inside = hit && !at_leaf && inside_test<PRED, POINTS>(b, q);
+      if (ballot(inside)) {
+        uint32_t live = inside ? t.wide_live[child] : 0u;
+        live += __shfl_xor(live, 1, 64);
+        live += __shfl_xor(live, 2, 64);
+        live += __shfl_xor(live, 4, 64);
+        found += live;
+        if (inside) hit = false;
+      }
+    }
+    const uint64_t push = ballot(hit && !at_leaf);
+    const uint32_t m8 = (uint32_t)(push >> (8u * oct)) & 0xFFu;
+    if (have) sp--;
+    if (hit && !at_leaf) stack[sp + (uint32_t)__popc(m8 & ((1u << j) - 1u))] = child;
+    sp += (uint32_t)__popc(m8);
+    const uint64_t leaves = ballot(hit && at_leaf);
+    if (leaves) {
+      const uint32_t h8 = (uint32_t)(leaves >> (8u * oct)) & 0xFFu;
+      sink.hits(hit && at_leaf, leaves, i, found + (uint32_t)__popc(h8 & ((1u << j) - 1u)), gid);
+      found += (uint32_t)__popc(h8);
+    }
+    if (have && sp == 0) {
+      sink.finish(i, found);
+      i += kFan;
+      have = i < last;
+      q = qn;
+      found = 0;
+      if (have) {
+        sp = 1;
+        if (j == 0) stack[0] = 0;
+        if (i + kFan < last) src(i + kFan, qn);
+      }
+    }
+    lds_fence();
+  }
+}
+
+// ----------------------------------------------------------------- wave ----
+constexpr int kWideRounds = 4;
+constexpr uint32_t kWidePop = kWideRounds * kFan;  // nodes per step
+// Steps pop fewer nodes when the stack could pass kWideSoft, down to one;
+// from there the walk is depth first and adds at most 7 per level.
+constexpr uint32_t kWideSoft = 320;
+constexpr uint32_t kWideStack = kWideSoft + 7 * kMaxDepth + 8;
+static_assert(7 * kWidePop + 64 <= kWideSoft, "a full step fits");
+
+struct WideLds {
+  uint32_t stack[kWideStack];
+};
+
+// Returns the query's number of results (wave-uniform). WRITE emits every
+// pair, numbered from 0 in emission order; LOG (counting walks) records the
+// results in `log`; a counting walk without LOG counts subtrees inside the
+// query from their live counts.
+template <int PRED, bool POINTS, bool WRITE, bool LOG, typename Q, typename Emit>
+__device__ uint64_t wide_walk(const TreeView& t, const Q& q, const uint32_t qid, Emit&& emit,
+                              WideLds& L, RangeLog* log = nullptr) {
+  const uint32_t lane = lane_id(), j = lane & 7u, oct = lane >> 3;
+  uint32_t* stack = L.stack;
+  uint32_t sp = t.start_n;  // wave-uniform
+  uint64_t emitted = 0;     // wave-uniform: results emitted, or counted leaf by leaf
+  uint64_t inside_live = 0; // per lane: counting walks, leaves of nodes inside the query
+  uint32_t nlog = 0;        // wave-uniform
+  if (lane < sp) stack[lane] = t.start + lane;
+  lds_fence();
+  while (sp > 0) {
+    uint32_t c = sp + 7 < kWideSoft ? (kWideSoft - sp) / 7u : 1u;
+    c = c < kWidePop ? c : kWidePop;
+    c = c < sp ? c : sp;
+    uint32_t child[kWideRounds];
+    uint32_t live[kWideRounds];
+    float4 b[kWideRounds];
+    uint32_t okm = 0;
+#pragma unroll
+    for (int r = 0; r < kWideRounds; r++) {
+      const uint32_t k = r * kFan + oct;
+      const bool ok = k < c;
+      const uint32_t e = ok ? stack[sp - 1 - k] : 0u;
+      child[r] = kFan * e + 1u + j;
+      const bool at_leaf = child[r] >= t.leaf0;
+      const uint32_t leaf = child[r] - t.leaf0;
+      const bool in = !at_leaf || leaf < t.n;
+      // Lanes without a child load a box that exists and drop it.
+      const float4* p = at_leaf ? t.leaf_boxes + (in ? leaf : 0u) : t.wide + child[r];
+      b[r] = *p;
+      okm |= (ok && in ? 1u : 0u) << r;
+    }
+    sp -= c;
+    lds_fence();
+#pragma unroll
+    for (int r = 0; r < kWideRounds; r++) {
+      if ((uint32_t)(r * kFan) >= c) break;
+      const bool ok = (okm >> r) & 1u;
+      const bool at_leaf = child[r] >= t.leaf0;
+      const uint32_t leaf = child[r] - t.leaf0;
+      bool hit = false;
+      if (ok)
+        hit = at_leaf ? leaf_test<PRED, POINTS>(t, leaf, b[r], q)
+                      : node_test<PRED, POINTS>(b[r], q);
+      bool range = false;  // a run of leaves that all are results
+      uint32_t rf = 0, rn = 0;
+      const bool inside = hit && !at_leaf && inside_test<PRED, POINTS>(b[r], q);
+      if (inside) {
+        live[r] = t.wide_live[child[r]];
+        if (!WRITE && !LOG) {
+          inside_live += live[r];
+          hit = false;
+        } else {
+          wide_leaves(t, child[r], &rf, &rn);
+          if (live[r] == rn) {  // otherwise a deleted box lies below: descend
+            range = true;
+            hit = false;
+            if (!WRITE) inside_live += rn;
+          }
+        }
+      }
+      const bool push = hit && !at_leaf;
+      const uint64_t pm = ballot(push);
+      if (push) stack[sp + mask_rank(pm)] = child[r];
+      sp += (uint32_t)__popcll(pm);
+      const uint64_t lm = ballot(hit && at_leaf);
+      const uint32_t nl = (uint32_t)__popcll(lm);
+      if (LOG) {
+        const uint32_t h8 = (uint32_t)(lm >> (8u * oct)) & 0xFFu;
+        const bool entry = range || (j == 0 && h8);
+        const uint64_t em = ballot(entry);
+        if (entry) {
+          // A whole block of 8 is an ordinary block entry.
+          const bool run = range && rn > kFan;
+          const uint32_t x = range ? rf | (run ? kLogRange : 0u) : leaf;
+          const uint32_t y = range ? (run ? rn : (1u << rn) - 1u) : h8;
+          const uint32_t at = nlog + mask_rank(em);
+          if (at < log->cap) log_store(log->entries + at, x, y);
+        }
+        nlog += (uint32_t)__popcll(em);
+      }
+      if (WRITE) {
+        if constexpr (HasBeginStep<Emit>::value) {
+          if (nl) emit.begin_step(emitted, nl);
+        }
+        if (hit && at_leaf) emit(emitted + mask_rank(lm), t.leaf_ids[leaf], qid);
+      }
+      emitted += nl;
+      if (WRITE) {
+        uint64_t rm = ballot(range);
+        while (rm) {
+          const int l = __builtin_ctzll(rm);
+          rm &= rm - 1;
+          const uint32_t f = readlane_u32(rf, l), n = readlane_u32(rn, l);
+          for (uint32_t k = 0; k < n; k += kWave) {
+            const uint32_t m = n - k < (uint32_t)kWave ? n - k : (uint32_t)kWave;
+            if constexpr (HasBeginStep<Emit>::value) emit.begin_step(emitted, m);
+            if (lane < m) emit(emitted + lane, t.leaf_ids[f + k + lane], qid);
+            emitted += m;
+          }
+        }
+      }
+    }
+    lds_fence();
+  }
+  if (LOG) log->logged = nlog;
+  return WRITE ? emitted : emitted + wave_sum_u64(inside_live);
+}
+
+// Emits the logged results of one query and returns their number. Blocks are
+// taken 8 at a time, one per octet: each lane stores the result its mask bit
+// names, and the wave's stores of a round are consecutive pairs. Runs of
+// leaves are copied 64 (4 x 64 while they last) at a time.
+template <typename Emit>
+__device__ uint64_t wide_replay(const TreeView& t, const RangeLog& lg, const uint32_t qid,
+                                const Emit& emit) {
+  const uint32_t lane = lane_id(), j = lane & 7u, oct = lane >> 3;
+  uint64_t emitted = 0;  // wave-uniform
+  for (uint32_t b0 = 0; b0 < lg.n_in; b0 += kWave) {
+    const uint32_t m = lg.n_in - b0 < (uint32_t)kWave ? lg.n_in - b0 : (uint32_t)kWave;
+    const uint2 en = lane < m ? log_load(lg.entries + b0 + lane) : make_uint2(0u, 0u);
+    const bool run = en.x & kLogRange;
+    const uint32_t cnt = run ? en.y : (uint32_t)__popc(en.y);
+    const uint32_t inc = wave_inclusive_sum(cnt);
+    const uint32_t off = inc - cnt;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      if ((uint32_t)(h * 32) >= m) break;
+      uint32_t gid[4], at[4];
+      uint32_t hm = 0;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int s = h * 32 + r * 8 + (int)oct;
+        const uint32_t x = (uint32_t)__shfl((int)en.x, s, 64);
+        const uint32_t y = (uint32_t)__shfl((int)en.y, s, 64);
+        at[r] = (uint32_t)__shfl((int)off, s, 64) + (uint32_t)__popc(y & ((1u << j) - 1u));
+        const bool hit = !(x & kLogRange) && ((y >> j) & 1u);
+        hm |= (hit ? 1u : 0u) << r;
+        gid[r] = hit ? t.leaf_ids[x + j] : 0u;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if ((hm >> r) & 1u) emit(emitted + at[r], gid[r], qid);
+    }
+    uint64_t rm = ballot(run);
+    while (rm) {
+      const int l = __builtin_ctzll(rm);
+      rm &= rm - 1;
+      const uint32_t f = readlane_u32(en.x, l) & ~kLogRange, n = readlane_u32(en.y, l);
+      const uint64_t at = emitted + readlane_u32(off, l);
+      uint32_t k = 0;
+      for (; k + 4 * kWave <= n; k += 4 * kWave) {
+        uint32_t gid[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) gid[u] = t.leaf_ids[f + k + u * kWave + lane];
+#pragma unroll
+        for (int u = 0; u < 4; u++) emit(at + k + u * kWave + lane, gid[u], qid);
+      }
+      for (; k < n; k += kWave)
+        if (k + lane < n) emit(at + k + lane, t.leaf_ids[f + k + lane], qid);
+    }
+    emitted += readlane_u32(inc, kWave - 1);
+  }
+  return emitted;
+}
+
+}  // namespace rts

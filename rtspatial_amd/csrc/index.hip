@@ -508,6 +508,8 @@ int rts_index_create(const rts_config* cfg, rts_index** out) {
       return rc;
     }
   }
+  workspace_index_begin(ix->device);
+  ix->counted = true;
   *out = ix;
   return RTS_OK;
 }
@@ -537,6 +539,7 @@ int rts_index_destroy(rts_index* ix) {
   if (ix->h_cost) (void)hipHostFree(ix->h_cost);
   if (ix->ev_cost_build) (void)hipEventDestroy(ix->ev_cost_build);
   if (ix->ev_cost_refit) (void)hipEventDestroy(ix->ev_cost_refit);
+  if (ix->counted) workspace_index_end(ix->device);
   delete ix;
   return RTS_OK;
 }
@@ -643,44 +646,9 @@ int rts_index_update_d(rts_index* ix, const rts_update_d* ups, uint64_t n, rts_s
 
 namespace {
 
-// Per-call device scratch, carved from one stream-ordered allocation.
-// Stream-ordered scratch of query calls (range logs take gigabytes) comes
-// from one memory pool per device that keeps its memory: the default pool
-// hands freed memory back at every synchronisation, so each call paid for
-// the driver's allocation again (the per-request path's p99 rose from 272
-// ms to 1.69 s with range logs). The pools live until the process ends.
-hipError_t scratch_alloc(void** p, size_t bytes, hipStream_t stream) {
-  static std::mutex mu;
-  static hipMemPool_t pools[64] = {};
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
-  hipMemPool_t pool;
-  {
-    std::lock_guard<std::mutex> lk(mu);
-    if (!pools[dev]) {
-      hipMemPoolProps props = {};
-      props.allocType = hipMemAllocationTypePinned;
-      props.handleTypes = hipMemHandleTypeNone;
-      props.location.type = hipMemLocationTypeDevice;
-      props.location.id = dev;
-      e = hipMemPoolCreate(&pools[dev], &props);
-      if (e != hipSuccess) {
-        pools[dev] = nullptr;
-        return e;
-      }
-      uint64_t keep = UINT64_MAX;
-      e = hipMemPoolSetAttribute(pools[dev], hipMemPoolAttrReleaseThreshold, &keep);
-      if (e != hipSuccess) return e;
-    }
-    pool = pools[dev];
-  }
-  return hipMallocFromPoolAsync(p, bytes, pool, stream);
-}
-
+// Per-call device scratch, carved from one leased block (workspace.hip).
 struct QueryScratch {
-  char* block = nullptr;
+  Scratch block;
   const uint32_t* order = nullptr;  // Morton permutation (optional)
   uint32_t* counts = nullptr;       // wave two-pass: per-query counts
   uint64_t* offsets = nullptr;      //                exclusive scan of counts
@@ -694,8 +662,7 @@ size_t align_up(size_t x) { return (x + 255) & ~size_t(255); }
 
 // Carves the scratch of a query call over nq queries. With `ext` (the
 // allocation-free entry point) the block is ext's first ext_bytes bytes, and
-// a call needing more is an error; otherwise it is allocated on `stream`
-// (and qs->block is freed by the caller).
+// a call needing more is an error; otherwise it is leased for `stream`.
 int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t stream,
                   QueryScratch* qs, size_t* order_off, size_t* sort_off, char* ext = nullptr,
                   size_t ext_bytes = 0, char** base_out = nullptr) {
@@ -739,8 +706,8 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
     b = ext;
   } else {
     if (off == 0) return RTS_OK;
-    RTS_HIP(scratch_alloc(reinterpret_cast<void**>(&qs->block), off, stream));
-    b = qs->block;
+    RTS_HIP(qs->block.lease(off, stream));
+    b = qs->block.get();
   }
   if (base_out) *base_out = b;
   if (wave) qs->tickets = reinterpret_cast<uint32_t*>(b + o_tk);
@@ -911,7 +878,6 @@ int run_plan(rts_index* ix, const Plan& plan, int pred, const void* queries, uin
         phase_end(ph, stream);
       }
     }
-    if (qs.block) RTS_HIP(hipFreeAsync(qs.block, stream));
   }
   return RTS_OK;
 }
@@ -929,27 +895,17 @@ int check_query_args(int pred, const void* queries, uint64_t nq, bool points, rt
   return RTS_OK;
 }
 
-// Queries of a double index with coord RTS_COORD_F64_AS_F32, rounded to
-// nearest floats in a stream-ordered buffer that the destructor releases.
-struct RoundedQueries {
-  void* p = nullptr;
-  hipStream_t stream = nullptr;
-  ~RoundedQueries() {
-    if (p) (void)hipFreeAsync(p, stream);
-  }
-};
-
 // The queries as the kernels take them: unchanged, or, on an index that
-// rounds doubles to floats, rounded into `rq`. *f64 tells which.
+// rounds doubles to floats, rounded into `rq`, a leased buffer. *f64 tells
+// which.
 int kernel_queries(rts_index* ix, const void* queries, uint64_t nq, bool points,
-                   hipStream_t stream, RoundedQueries* rq, const void** out, bool* f64) {
+                   hipStream_t stream, Scratch* rq, const void** out, bool* f64) {
   *out = queries;
   *f64 = ix->cfg.coord == RTS_COORD_F64;
   if (ix->cfg.coord != RTS_COORD_F64_AS_F32) return RTS_OK;
-  rq->stream = stream;
-  RTS_HIP(scratch_alloc(&rq->p, nq * query_bytes(points, false), stream));
-  RTS_HIP(launch_round_queries64(queries, points, nq, rq->p, stream));
-  *out = rq->p;
+  RTS_HIP(rq->lease(nq * query_bytes(points, false), stream));
+  RTS_HIP(launch_round_queries64(queries, points, nq, rq->get(), stream));
+  *out = rq->get();
   return RTS_OK;
 }
 
@@ -966,7 +922,7 @@ int run_query(rts_index* ix, int pred, const void* queries, uint64_t nq, bool po
   if (ix->n == 0) return RTS_OK;  // spatial_index.cuh:354-356
   rc = ensure_built(ix, stream);
   if (rc) return rc;
-  RoundedQueries rq;
+  Scratch rq;
   const void* kq = nullptr;
   bool f64 = false;
   rc = kernel_queries(ix, queries, nq, points, stream, &rq, &kq, &f64);
@@ -1154,17 +1110,15 @@ int rts_index_order_queries(rts_index* ix, const void* queries, uint64_t n, int 
   RTS_CHECK_ARG(queries && order, "rts_index_order_queries: null array");
   std::lock_guard<std::mutex> lk(ix->mu);
   RTS_HIP(hipSetDevice(ix->device));
-  char* block = nullptr;
+  Scratch block;
   const size_t keys_bytes = align_up(4 * n * sizeof(uint32_t));
-  RTS_HIP(scratch_alloc(reinterpret_cast<void**>(&block), keys_bytes + sort_scratch_bytes(n),
-                        stream));
+  RTS_HIP(block.lease(keys_bytes + sort_scratch_bytes(n), stream));
   const uint32_t* perm = nullptr;
   // Envelopes and segments share a layout; a segment is ordered by the
   // centre of its bounding box.
-  int rc = order_queries(ix, queries, n, points == RTS_QUERY_POINTS, ix->f64(), block,
-                         block + keys_bytes, stream, &perm);
+  int rc = order_queries(ix, queries, n, points == RTS_QUERY_POINTS, ix->f64(), block.get(),
+                         block.get() + keys_bytes, stream, &perm);
   if (!rc) RTS_HIP(hipMemcpyAsync(order, perm, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream));
-  RTS_HIP(hipFreeAsync(block, stream));
   return rc;
 }
 
@@ -1255,10 +1209,9 @@ int rts_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* k
   RTS_CHECK_ARG(n < (1ull << 30), "rts_sort_pairs: n must be below 2^30");
   if (n == 0) return RTS_OK;
   const size_t scratch = sort_scratch_bytes(n);
-  char* base = nullptr;
-  RTS_HIP(scratch_alloc(reinterpret_cast<void**>(&base), 2 * n * sizeof(uint32_t) + scratch + 256,
-                        stream));
-  uint32_t* kb = reinterpret_cast<uint32_t*>(base);
+  Scratch block;
+  RTS_HIP(block.lease(2 * n * sizeof(uint32_t) + scratch + 256, stream));
+  uint32_t* kb = reinterpret_cast<uint32_t*>(block.get());
   uint32_t* vb = kb + n;
   char* sbase = reinterpret_cast<char*>(
       (reinterpret_cast<uintptr_t>(vb + n) + 255) & ~uintptr_t(255));
@@ -1276,7 +1229,6 @@ int rts_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* k
   }
   uint32_t err = 0;
   RTS_HIP(hipMemcpyAsync(&err, ss.error, sizeof(err), hipMemcpyDeviceToHost, stream));
-  RTS_HIP(hipFreeAsync(base, stream));
   RTS_HIP(hipStreamSynchronize(stream));
   if (err) {
     set_error("rts_sort_pairs: look-back exceeded its wait bound");

@@ -11,6 +11,7 @@
 struct rts_index {
   rts_config cfg{};
   int device = 0;
+  bool counted = false;  // among the device's live indexes (workspace.hip)
   std::mutex mu;  // serializes host-side state changes of one index
 
   // Boxes by id (the reference's envelopes_, spatial_index.cuh:919) and the

@@ -200,6 +200,31 @@ hipError_t launch_exclusive_scan(const uint32_t* counts, uint64_t n, uint64_t* o
 hipError_t launch_reserve(const void* dev_queue, const uint64_t* total, uint64_t* base,
                           hipStream_t stream);
 
+// workspace.hip: device scratch kept between calls. A lease is for work on
+// `stream`; the destructor returns it once that work is queued.
+struct Lease {
+  void* p = nullptr;
+  size_t bytes = 0;
+  hipEvent_t done = nullptr;
+  hipStream_t stream = nullptr;
+  int device = 0;
+  bool stream_ordered = false;
+};
+hipError_t workspace_lease(size_t bytes, hipStream_t stream, Lease* out);
+void workspace_return(Lease* lease);
+struct Scratch {
+  Lease l;
+  Scratch() = default;
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  ~Scratch() { workspace_return(&l); }
+  hipError_t lease(size_t bytes, hipStream_t stream) { return workspace_lease(bytes, stream, &l); }
+  char* get() const { return static_cast<char*>(l.p); }
+};
+// An index lives on the device from _begin to _end.
+void workspace_index_begin(int dev);
+void workspace_index_end(int dev);
+
 // index.hip
 void set_error(const std::string& msg);
 

@@ -34,6 +34,7 @@
 #include <deque>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "batch.h"
@@ -148,6 +149,7 @@ struct Slot {
   char* h_desc = nullptr;                // pinned: [TreeView | BatchHeader | BatchRequest x max]
   uint64_t* h_ranges = nullptr;          // pinned: 3 x max
   unsigned long long* h_hash = nullptr;  // pinned: max
+  Scratch block;                         // the device buffers below
   char* d_desc = nullptr;
   uint32_t* d_counters = nullptr;
   uint32_t* d_giants = nullptr;  // kGiantBuckets x max_batch_queries tile ids
@@ -454,39 +456,55 @@ int record_slot_work(Engine& E, Slot& s, size_t up_bytes, size_t n_req) {
   return RTS_OK;
 }
 
+// A slot's device buffers are carved from one leased block and its pinned ones
+// from one allocation: a run pays for neither's mapping again.
 int slot_init(Engine& E, Slot& s) {
   const uint32_t maxr = E.cfg.max_batch_requests;
   const uint64_t maxq = E.cfg.max_batch_queries;
   SRV_HIP(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking));
   SRV_HIP(hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
-  SRV_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.h_desc), E.desc_bytes));
-  SRV_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.h_ranges), 3 * maxr * sizeof(uint64_t)));
-  SRV_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.h_hash), maxr * sizeof(unsigned long long)));
-  SRV_HIP(hipMalloc(&s.d_desc, E.desc_bytes));
-  SRV_HIP(hipMalloc(&s.d_counters, kTileCounterWords * sizeof(uint32_t)));
-  SRV_HIP(hipMalloc(&s.d_giants, kGiantBuckets * maxq * sizeof(uint32_t)));
-  SRV_HIP(hipMalloc(&s.d_log, serve_log_entries(maxq) * sizeof(uint2)));
-  SRV_HIP(hipMalloc(&s.d_log_off, maxq * sizeof(uint32_t)));
-  SRV_HIP(hipMalloc(&s.d_log_n, maxq * sizeof(uint32_t)));
-  SRV_HIP(hipMalloc(&s.d_counts, maxq * sizeof(uint32_t)));
-  SRV_HIP(hipMalloc(&s.d_exact, maxq * sizeof(uint32_t)));
-  SRV_HIP(hipMalloc(&s.d_offsets, maxq * sizeof(uint64_t)));
-  SRV_HIP(hipMalloc(&s.d_exact_off, maxq * sizeof(uint64_t)));
-  SRV_HIP(hipMalloc(&s.d_seg, batch_seg_sums_words() * sizeof(uint64_t)));
-  // [0] bound total, [1] the extension launches' queue counter, [2] exact total
-  SRV_HIP(hipMalloc(&s.d_total, 4 * sizeof(uint64_t)));
-  SRV_HIP(hipMalloc(&s.d_ranges, 3 * maxr * sizeof(uint64_t)));
-  SRV_HIP(hipMalloc(&s.d_hash, maxr * sizeof(unsigned long long)));
-  SRV_HIP(hipMalloc(&s.d_arena, E.cfg.arena_pairs * sizeof(rts_pair)));
-  SRV_HIP(hipMalloc(&s.d_sort, 4 * maxq * sizeof(uint32_t) + sort_scratch_bytes(maxq)));
-  SRV_HIP(hipMalloc(&s.d_ext, 64 + kWaveTicketWords * sizeof(uint32_t)));
+  const size_t desc = (E.desc_bytes + 255) & ~size_t(255);
+  SRV_HIP(hipHostMalloc(reinterpret_cast<void**>(&s.h_desc), desc + 4 * maxr * sizeof(uint64_t)));
+  s.h_ranges = reinterpret_cast<uint64_t*>(s.h_desc + desc);
+  s.h_hash = reinterpret_cast<unsigned long long*>(s.h_ranges + 3 * (uint64_t)maxr);
+  size_t need = 0;
+  auto carve = [&](auto** p, uint64_t bytes) {
+    if (s.block.get()) *p = reinterpret_cast<std::remove_reference_t<decltype(*p)>>(s.block.get() + need);
+    need += (bytes + 255) & ~uint64_t(255);
+  };
+  // Once for the size, once for the addresses.
+  for (int pass = 0; pass < 2; pass++) {
+    need = 0;
+    carve(&s.d_desc, E.desc_bytes);
+    carve(&s.d_counters, kTileCounterWords * sizeof(uint32_t));
+    carve(&s.d_giants, kGiantBuckets * maxq * sizeof(uint32_t));
+    carve(&s.d_log, serve_log_entries(maxq) * sizeof(uint2));
+    carve(&s.d_log_off, maxq * sizeof(uint32_t));
+    carve(&s.d_log_n, maxq * sizeof(uint32_t));
+    carve(&s.d_counts, maxq * sizeof(uint32_t));
+    carve(&s.d_exact, maxq * sizeof(uint32_t));
+    carve(&s.d_offsets, maxq * sizeof(uint64_t));
+    carve(&s.d_exact_off, maxq * sizeof(uint64_t));
+    carve(&s.d_seg, batch_seg_sums_words() * sizeof(uint64_t));
+    // [0] bound total, [1] the extension launches' queue counter, [2] exact total
+    carve(&s.d_total, 4 * sizeof(uint64_t));
+    carve(&s.d_ranges, 3 * maxr * sizeof(uint64_t));
+    carve(&s.d_hash, maxr * sizeof(unsigned long long));
+    carve(&s.d_arena, E.cfg.arena_pairs * sizeof(rts_pair));
+    carve(&s.d_sort, 4 * maxq * sizeof(uint32_t) + sort_scratch_bytes(maxq));
+    carve(&s.d_ext, 64 + kWaveTicketWords * sizeof(uint32_t));
+    if (pass == 0) SRV_HIP(s.block.lease(need, s.stream));
+  }
   {
     // The arena as a result queue for the extension launches' write pass
-    // (which stores at exact offsets and never touches the counter).
+    // (which stores at exact offsets and never touches the counter); set up on
+    // the slot's stream, which does not wait for the null stream.
     const rts_dev_queue q{s.d_arena, E.cfg.arena_pairs,
                           reinterpret_cast<unsigned long long*>(s.d_total + 1)};
-    SRV_HIP(hipMemset(s.d_ext, 0, 64));
-    SRV_HIP(hipMemcpy(s.d_ext, &q, sizeof(q), hipMemcpyHostToDevice));
+    std::memset(s.h_desc, 0, 64);
+    std::memcpy(s.h_desc, &q, sizeof(q));
+    SRV_HIP(hipMemcpyAsync(s.d_ext, s.h_desc, 64, hipMemcpyHostToDevice, s.stream));
+    SRV_HIP(hipStreamSynchronize(s.stream));
   }
   std::memset(s.h_desc, 0, E.desc_bytes);
   SRV_TRACE("slot buffers ready (arena %llu pairs)", (unsigned long long)E.cfg.arena_pairs);
@@ -496,17 +514,12 @@ int slot_init(Engine& E, Slot& s) {
 void slot_free(Slot& s) {
   if (s.stream) (void)hipStreamSynchronize(s.stream);
   if (s.h_desc) (void)hipHostFree(s.h_desc);
-  if (s.h_ranges) (void)hipHostFree(s.h_ranges);
-  if (s.h_hash) (void)hipHostFree(s.h_hash);
-  for (void* p : {(void*)s.d_desc, (void*)s.d_counters, (void*)s.d_giants, (void*)s.d_log,
-                  (void*)s.d_log_off, (void*)s.d_log_n, (void*)s.d_counts,
-                  (void*)s.d_exact, (void*)s.d_offsets, (void*)s.d_exact_off,
-                  (void*)s.d_seg, (void*)s.d_total, (void*)s.d_ranges, (void*)s.d_hash,
-                  (void*)s.d_arena, (void*)s.d_sort, (void*)s.d_ext})
-    if (p) (void)hipFree(p);
+  workspace_return(&s.block.l);
   if (s.done) (void)hipEventDestroy(s.done);
   if (s.stream) (void)hipStreamDestroy(s.stream);
-  s = Slot();
+  s.stream = nullptr;
+  s.done = nullptr;
+  s.h_desc = nullptr;
 }
 
 // Seeds the per-kind estimates with a counting query over a sample of the
@@ -731,6 +744,7 @@ struct PlainChunk {
 int run_plain(Engine& E) {
   constexpr uint32_t kRing = 1024;
   hipStream_t stream = nullptr;
+  Scratch arena_block;
   rts_pair* arena = nullptr;
   unsigned long long* d_counter = nullptr;
   rts_dev_queue* d_queue = nullptr;
@@ -740,7 +754,8 @@ int run_plain(Engine& E) {
   unsigned long long* h_hash = nullptr;
   std::vector<hipEvent_t> evs(kRing, nullptr);
   SRV_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  SRV_HIP(hipMalloc(&arena, E.cfg.arena_pairs * sizeof(rts_pair)));
+  SRV_HIP(arena_block.lease(E.cfg.arena_pairs * sizeof(rts_pair), stream));
+  arena = reinterpret_cast<rts_pair*>(arena_block.get());
   SRV_HIP(hipMalloc(&d_counter, sizeof(unsigned long long)));
   SRV_HIP(hipMalloc(&d_queue, sizeof(rts_dev_queue)));
   SRV_HIP(hipMalloc(&d_spans, 2 * kRing * sizeof(uint64_t)));
@@ -837,7 +852,7 @@ int run_plain(Engine& E) {
   (void)hipStreamSynchronize(stream);
   for (auto& e : evs)
     if (e) (void)hipEventDestroy(e);
-  (void)hipFree(arena);
+  workspace_return(&arena_block.l);
   (void)hipFree(d_counter);
   (void)hipFree(d_queue);
   (void)hipFree(d_spans);

@@ -416,7 +416,7 @@ int rts_index_autotune(rts_index* index, rts_predicate pred, const void* queries
                        int points, rts_handler handler, const rts_tune_config* cfg,
                        rts_tune_result* out, rts_stream_t stream);
 
-/* Standalone LDS-staged onesweep radix sort of (uint32 key, uint32 value)
+/* Standalone LDS-staged radix sort of (uint32 key, uint32 value)
  * pairs on bits [0, key_bits) of the key, stable. `vals_in` NULL means values
  * 0..n-1. Outputs must not alias inputs. Scratch is allocated on `stream`. */
 int rts_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
@@ -546,7 +546,7 @@ int rts_serve_run(rts_index* index, const rts_serve_config* cfg, const rts_reque
  * stopwatches and stream syncs). */
 enum {
   RTS_PHASE_BUILD_MORTON = 0,  /* scene bounds + Morton codes */
-  RTS_PHASE_BUILD_SORT = 1,    /* onesweep radix sort of the codes */
+  RTS_PHASE_BUILD_SORT = 1,    /* radix sort of the codes */
   RTS_PHASE_BUILD_TREE = 2,    /* leaf gather + Karras hierarchy + refit */
   RTS_PHASE_REFIT = 3,         /* refit after Update/Delete */
   RTS_PHASE_MUTATE = 4,        /* Update/Delete scatter */

@@ -89,7 +89,6 @@ __host__ __device__ constexpr uint32_t wide_leaf0(uint32_t depth) {
 constexpr int kPredLine = 3;
 
 // Device error bits (the index's error word).
-constexpr uint32_t kErrSortWait = 1u;
 constexpr uint32_t kErrRefitWalk = 2u;
 constexpr uint32_t kErrTraversal = 4u;
 

@@ -361,14 +361,10 @@ int refit_tree(rts_index* ix, hipStream_t stream) {
 }
 
 int check_device_error(rts_index* ix) {
-  uint32_t err = 0, sort_err = 0;
+  uint32_t err = 0;
   RTS_HIP(hipMemcpy(&err, ix->error, sizeof(err), hipMemcpyDeviceToHost));
-  if (ix->ss.error)
-    RTS_HIP(hipMemcpy(&sort_err, ix->ss.error, sizeof(sort_err), hipMemcpyDeviceToHost));
-  if (sort_err) err |= kErrSortWait;
   if (err) {
     std::string m = "device error:";
-    if (err & kErrSortWait) m += " radix-sort look-back exceeded its wait bound;";
     if (err & kErrRefitWalk) m += " refit walk left the tree;";
     if (err & kErrTraversal) m += " traversal exceeded its step bound;";
     set_error(m);
@@ -740,7 +736,6 @@ int order_queries(rts_index* ix, const void* queries, uint64_t nq, bool points, 
   uint32_t* vals_b = keys_b + words;
   SortScratch ss;
   sort_scratch_carve(sort_base, nq, &ss);
-  ss.error = ix->error;  // a look-back that gives up is reported by the index's error word
   if (f64) {
     RTS_HIP(launch_morton64(queries, points, (uint32_t)nq, ix->scene, keys, stream));
   } else if (points) {
@@ -1217,23 +1212,29 @@ int rts_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* k
       (reinterpret_cast<uintptr_t>(vb + n) + 255) & ~uintptr_t(255));
   SortScratch ss;
   sort_scratch_carve(sbase, n, &ss);
-  RTS_HIP(hipMemcpyAsync(keys_out, keys_in, n * sizeof(uint32_t), hipMemcpyDefault, stream));
-  if (vals_in)
-    RTS_HIP(hipMemcpyAsync(vals_out, vals_in, n * sizeof(uint32_t), hipMemcpyDefault, stream));
-  bool in_b = false;
-  RTS_HIP(radix_sort_pairs(keys_out, vals_out, kb, vb, (uint32_t)n, key_bits, vals_in == nullptr, ss,
-                           stream, &in_b));
-  if (in_b) {
-    RTS_HIP(hipMemcpyAsync(keys_out, kb, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream));
-    RTS_HIP(hipMemcpyAsync(vals_out, vb, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream));
+  // The first pass reads device input where it lies. Host input is copied
+  // first, and so is input that is also an output, to the array the first
+  // pass does not write.
+  const bool odd = radix_sort_passes(key_bits) % 2 == 1;
+  auto direct = [&](const uint32_t* p) {
+    hipPointerAttribute_t at{};
+    const bool dev = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice;
+    if (!dev) (void)hipGetLastError();  // an unknown pointer is host memory
+    return dev && p != keys_out && p != vals_out;
+  };
+  if (!direct(keys_in)) {
+    uint32_t* to = odd ? kb : keys_out;
+    RTS_HIP(hipMemcpyAsync(to, keys_in, n * sizeof(uint32_t), hipMemcpyDefault, stream));
+    keys_in = to;
   }
-  uint32_t err = 0;
-  RTS_HIP(hipMemcpyAsync(&err, ss.error, sizeof(err), hipMemcpyDeviceToHost, stream));
+  if (vals_in && !direct(vals_in)) {
+    uint32_t* to = odd ? vb : vals_out;
+    RTS_HIP(hipMemcpyAsync(to, vals_in, n * sizeof(uint32_t), hipMemcpyDefault, stream));
+    vals_in = to;
+  }
+  RTS_HIP(radix_sort_into(keys_in, vals_in, keys_out, vals_out, kb, vb, (uint32_t)n, key_bits, ss,
+                          stream));
   RTS_HIP(hipStreamSynchronize(stream));
-  if (err) {
-    set_error("rts_sort_pairs: look-back exceeded its wait bound");
-    return RTS_ERR_DEVICE;
-  }
   return RTS_OK;
 }
 

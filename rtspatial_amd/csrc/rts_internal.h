@@ -27,15 +27,19 @@ struct SinkArgs {
 
 // sort.hip
 struct SortScratch {
-  uint32_t* hist;      // 4 x 256
-  uint32_t* offsets;   // 4 x 256
-  uint32_t* status;    // 4 x tiles x 256
-  uint32_t* tickets;   // 4
-  uint32_t* error;     // 1
-  uint32_t tiles_cap;  // tiles the status array holds per pass
+  uint32_t* totals;    // keys of each digit
+  uint32_t* counts;    // per digit and tile
+  uint32_t tiles_cap;  // tiles the counts hold
 };
 size_t sort_scratch_bytes(uint64_t n);
 void sort_scratch_carve(void* base, uint64_t n, SortScratch* s);
+int radix_sort_passes(int key_bits);
+// Sorts (keys_in, vals_in) on bits [0, key_bits) into the out arrays; vals_in
+// null means the values 0..n-1. The tmp arrays are scratch. The input may be
+// the out arrays when the passes are even, and the tmp arrays when odd.
+hipError_t radix_sort_into(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
+                           uint32_t* vals_out, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t n,
+                           int key_bits, const SortScratch& s, hipStream_t stream);
 // Sorts (keys, vals) on bits [0, key_bits). keys_a/vals_a hold the input
 // (with identity_vals the values 0..n-1 are generated and vals_a is only a
 // buffer); keys_b/vals_b are ping-pong buffers. `*in_b` tells whether the

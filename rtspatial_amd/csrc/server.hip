@@ -435,7 +435,6 @@ int record_slot_work(Engine& E, Slot& s, size_t up_bytes, size_t n_req) {
   sort.keys_b = s.d_sort + 2 * maxq;
   sort.vals_b = s.d_sort + 3 * maxq;
   sort_scratch_carve(s.d_sort + 4 * maxq, maxq, &sort.ss);
-  sort.ss.error = E.ix->error;  // a look-back that gives up is reported after the run
   sort.scene = E.ix->scene;
   sort.n = wave_tiles >= E.cfg.sort_min_tiles ? wave_tiles : 0;
   const BatchExtArgs ea{reinterpret_cast<uint32_t*>(s.d_ext + 64),

@@ -357,7 +357,7 @@ def pack_updates(ids, envelopes, coord_t=torch.float32):
 
 
 def sort_pairs(keys, vals=None, key_bits=32, stream=None):
-    """Stable onesweep radix sort of uint32 keys (int32 tensors) with uint32
+    """Stable radix sort of uint32 keys (int32 tensors) with uint32
     values (identity when vals is None). Returns (sorted_keys, sorted_vals)."""
     n = keys.numel()
     ko = torch.empty_like(keys)

@@ -16,8 +16,8 @@
 // wave tile's (range_log.h), a scan turns the numbers into exclusive offsets
 // into the slot's result arena, and the write pass emits the logged results
 // (a lane tile's walk is cheap and taken again) at the query's offset. Per
-// request, the batch reports its first slot, its slots and its results. Every
-// launch reads the batch's sizes from device memory.
+// request, the batch reports its first slot and its results. Every launch reads
+// the batch's sizes from device memory.
 #include <algorithm>
 
 #include "batch.h"
@@ -103,10 +103,9 @@ struct TileSource {
 };
 struct TileCount {
   uint32_t* counts;
-  uint32_t* exact;
   __device__ void hits(bool, uint64_t, uint32_t, uint32_t, uint32_t) const {}
   __device__ void finish(uint32_t i, uint32_t found) const {
-    if ((lane_id() & 7u) == 0) counts[i] = exact[i] = found;
+    if ((lane_id() & 7u) == 0) counts[i] = found;
   }
 };
 struct TileWrite {
@@ -133,24 +132,15 @@ __device__ __forceinline__ void run_tile(const TreeView& t, const BatchArgs& a,
   if (WRITE && skip_giants && wave && local < r.n &&
       a.counts[r.qbase + local] >= giant_min(kGiantBuckets - 1))
     return;
-  // A request whose slots run past the arena is launched again: its pairs
-  // would be dropped, so its walks are skipped (a one-query request still
-  // runs, for its exact count).
-  if (WRITE && r.n > 1 && a.ranges[3 * ri] + a.ranges[3 * ri + 1] > a.arena_cap) {
-    if (wave) {
-      if (local < r.n && lane_id() == 0) a.exact[r.qbase + local] = 0;
-    } else {
-      const uint32_t q = local * kWave + lane_id();
-      if (q < r.n) a.exact[r.qbase + q] = 0;
-    }
-    return;
-  }
+  // A request whose results run past the arena is launched again: its pairs
+  // would be dropped.
+  if (WRITE && a.ranges[2 * ri] + a.ranges[2 * ri + 1] > a.arena_cap) return;
   if (t.n == 0) {
     if (wave) {
-      if (local < r.n && lane_id() == 0) a.counts[r.qbase + local] = a.exact[r.qbase + local] = 0;
+      if (local < r.n && lane_id() == 0) a.counts[r.qbase + local] = 0;
     } else {
       const uint32_t q = local * kWave + lane_id();
-      if (q < r.n) a.counts[r.qbase + q] = a.exact[r.qbase + q] = 0;
+      if (q < r.n) a.counts[r.qbase + q] = 0;
     }
     return;
   }
@@ -174,7 +164,7 @@ __device__ __forceinline__ void run_tile(const TreeView& t, const BatchArgs& a,
       const uint64_t c = wide_walk<0, false, false, true>(t, qb, local, NoEmit{}, lds.wide, &lg);
       log_commit(lc, a.log, g, lg);
       if (lane_id() == 0) {
-        a.counts[g] = a.exact[g] = (uint32_t)c;
+        a.counts[g] = (uint32_t)c;
         // Giants are listed as they are counted (rare: one atomic each).
         if (a.giants && c >= giant_min(kGiantBuckets - 1)) {
           int b = kGiantBuckets - 1;
@@ -195,7 +185,7 @@ __device__ __forceinline__ void run_tile(const TreeView& t, const BatchArgs& a,
       TileWrite sink{a.offsets + r.qbase, a.arena, a.arena_cap, r.qid_base};
       oct_walk<0, false, false, QueryRT>(t, stack, first, last, src, sink);
     } else {
-      TileCount sink{a.counts + r.qbase, a.exact + r.qbase};
+      TileCount sink{a.counts + r.qbase};
       oct_walk<0, false, true, QueryRT>(t, stack, first, last, src, sink);
     }
   }
@@ -326,85 +316,18 @@ __global__ void __launch_bounds__(kThreads) k_seg_apply(const BatchArgs a) {
   }
 }
 
-// Per request: first arena slot and slots (the sum of its bounds).
+// Per request: first arena slot and results.
 __global__ void __launch_bounds__(kThreads) k_request_ranges(const BatchArgs a) {
   const BatchHeader h = *a.header;
   for (uint32_t r = blockIdx.x * kThreads + threadIdx.x; r < h.n_requests;
        r += gridDim.x * kThreads) {
     const BatchRequest q = a.requests[r];
-    const uint64_t start = q.n ? a.offsets[q.qbase] : 0;
+    // (A request without queries has a place too, and no results.)
+    const uint64_t start = q.qbase < h.n_queries ? a.offsets[q.qbase] : a.total[0];
     const uint64_t end = (q.qbase + q.n < h.n_queries) ? a.offsets[q.qbase + q.n] : a.total[0];
-    a.ranges[3 * r] = start;
-    a.ranges[3 * r + 1] = q.n ? end - start : 0;
-    a.ranges[3 * r + 2] = 0;  // results: summed by k_request_exact
+    a.ranges[2 * r] = start;
+    a.ranges[2 * r + 1] = end - start;
   }
-}
-
-// Request of global query q: the last request whose qbase <= q (requests are
-// laid out in query order).
-__device__ __forceinline__ uint32_t request_of_query(const BatchRequest* reqs, uint32_t nreq,
-                                                     uint64_t q) {
-  uint32_t lo = 0, hi = nreq - 1;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi + 1) >> 1;
-    if (reqs[mid].qbase <= q) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-// After the write pass: each request's results, the sum of its queries'
-// exact counts, added into ranges[3r + 2]. A wavefront sums a block of
-// kExactBlock counts: with one atomic when the block lies in one request
-// (requests are contiguous in query space), else lane by lane, each lane
-// over its own run of the block, one atomic per request it meets. (One
-// atomic per query from the write pass, on one address per request, made
-// that pass twice as slow.)
-constexpr uint32_t kExactPerLane = 16;
-constexpr uint32_t kExactBlock = kWave * kExactPerLane;
-
-__global__ void __launch_bounds__(kThreads) k_request_exact(const BatchArgs a) {
-  const BatchHeader h = *a.header;
-  if (h.n_requests == 0) return;
-  const uint32_t lane = lane_id();
-  const uint64_t waves = (uint64_t)gridDim.x * kWaves;
-  for (uint64_t w = (uint64_t)blockIdx.x * kWaves + threadIdx.x / kWave;
-       w * kExactBlock < h.n_queries; w += waves) {
-    const uint64_t b0 = w * kExactBlock;
-    const uint64_t b1 = b0 + kExactBlock < h.n_queries ? b0 + kExactBlock : h.n_queries;
-    const uint32_t r0 = request_of_query(a.requests, h.n_requests, b0);
-    const uint32_t r1 = request_of_query(a.requests, h.n_requests, b1 - 1);
-    if (r0 == r1) {
-      uint64_t s = 0;
-      for (uint64_t i = b0 + lane; i < b1; i += kWave) s += a.exact[i];
-      s = wave_sum_u64(s);
-      if (lane == 0 && s) atomicAdd(reinterpret_cast<unsigned long long*>(&a.ranges[3 * r0 + 2]), s);
-    } else {
-      uint64_t i = b0 + (uint64_t)lane * kExactPerLane;
-      const uint64_t e = i + kExactPerLane < b1 ? i + kExactPerLane : b1;
-      if (i < e) {
-        uint32_t r = request_of_query(a.requests, h.n_requests, i);
-        uint64_t r_end = r + 1 < h.n_requests ? a.requests[r + 1].qbase : h.n_queries;
-        uint64_t s = 0;
-        for (; i < e; i++) {
-          while (i >= r_end) {
-            if (s) atomicAdd(reinterpret_cast<unsigned long long*>(&a.ranges[3 * r + 2]), s);
-            s = 0;
-            r++;
-            r_end = r + 1 < h.n_requests ? a.requests[r + 1].qbase : h.n_queries;
-          }
-          s += a.exact[i];
-        }
-        if (s) atomicAdd(reinterpret_cast<unsigned long long*>(&a.ranges[3 * r + 2]), s);
-      }
-    }
-  }
-}
-
-__global__ void __launch_bounds__(kThreads) k_copy_u32(const uint32_t* __restrict__ src,
-                                                       uint32_t* __restrict__ dst, uint64_t n) {
-  for (uint64_t i = blockIdx.x * (uint64_t)kThreads + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * kThreads)
-    dst[i] = src[i];
 }
 
 __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
@@ -459,7 +382,7 @@ void launch_seg_scan(const BatchArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSort& sort,
-                        const BatchExt* ext, size_t n_ext, const BatchExtArgs& ea, bool collect,
+                        const BatchExt* ext, size_t n_ext, const BatchExtArgs& ea,
                         hipStream_t stream) {
   BatchArgs a = a_in;
   a.order = nullptr;
@@ -484,7 +407,7 @@ hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSor
                      kTileCounterWords);
   launch_batch_kernel<false>(t, a, stream);
   // Requests the batch kernel does not walk: one count launch each, into the
-  // same counts (so the scan below covers them). Their counts are exact.
+  // same counts (so the scan below covers them).
   for (size_t i = 0; i < n_ext; i++) {
     const BatchExt& x = ext[i];
     hipError_t e;
@@ -495,11 +418,6 @@ hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSor
       e = launch_query_wave(x.ql, wa, kPhaseCount, stream);
     }
     if (e != hipSuccess) return e;
-    if (x.ql.n) {
-      const uint32_t blocks = (uint32_t)std::min<uint64_t>((x.ql.n + kThreads - 1) / kThreads, 1024);
-      hipLaunchKernelGGL(k_copy_u32, dim3(blocks), dim3(kThreads), 0, stream, a.counts + x.qbase,
-                         a.exact + x.qbase, (uint64_t)x.ql.n);
-    }
   }
   launch_seg_scan(a, stream);
   hipLaunchKernelGGL(k_request_ranges, dim3(16), dim3(kThreads), 0, stream, a);
@@ -517,16 +435,6 @@ hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSor
     if (e != hipSuccess) return e;
   }
   phase_end(ph, stream);
-  // Per request results, and the compacted offsets for requests that copy
-  // their pairs out.
-  hipLaunchKernelGGL(k_request_exact, dim3(1024), dim3(kThreads), 0, stream, a);
-  if (collect) {
-    BatchArgs x = a;
-    x.counts = a.exact;
-    x.offsets = a.exact_offsets;
-    x.total = a.total + 2;
-    launch_seg_scan(x, stream);
-  }
   return hipGetLastError();
 }
 
@@ -534,87 +442,43 @@ size_t batch_seg_sums_words() { return kScanBlocks; }
 
 namespace {
 
-// hashes[r] += pair_hash over request r's pairs. The queries' slot ranges
-// [offsets[q], + counts[q]) tile the arena's [0, total), and query q's pairs
-// are the first exact[q] slots of its range. A wavefront takes blocks of
-// kHashBlock consecutive slots (lanes interleaved, so loads coalesce); each
-// lane finds the query of its first slot, then follows the ranges forward,
-// keeping a running sum that it adds to hashes[] when its request changes.
-// Where the whole wave ends a block in one request, one wave-reduced atomic
-// suffices.
+// hashes[r] += pair_hash over request r's pairs, arena[start, start + results).
+// A wavefront takes blocks of kHashBlock consecutive slots and goes through the
+// requests that have pairs there; each costs it one atomic. (Finding each
+// slot's query as well, when a query's slots were a bound on its results, took
+// 3.2 ms per batch of 64 served requests, 40M pairs.)
 constexpr uint32_t kHashBlock = kWave * 256;
 
-__device__ __forceinline__ uint64_t query_of_slot(const uint64_t* offsets, uint64_t nq,
-                                                  uint64_t i) {
-  uint64_t lo = 0, hi = nq - 1;
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi + 1) >> 1;
-    if (offsets[mid] <= i) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-__global__ void __launch_bounds__(kThreads) k_hash_queries(const BatchArgs a,
-                                                           unsigned long long* __restrict__ hashes) {
+__global__ void __launch_bounds__(kThreads) k_hash_requests(const BatchArgs a,
+                                                            unsigned long long* __restrict__ hashes) {
   const BatchHeader h = *a.header;
-  const uint64_t nq = h.n_queries;
   const uint64_t hi = a.total[0] < a.arena_cap ? a.total[0] : a.arena_cap;
-  if (h.n_requests == 0 || nq == 0 || hi == 0) return;
+  if (h.n_requests == 0 || h.n_queries == 0 || hi == 0) return;
   const uint32_t lane = lane_id();
   const uint64_t waves = (uint64_t)gridDim.x * kWaves;
   const uint64_t w0 = (uint64_t)blockIdx.x * kWaves + threadIdx.x / kWave;
   for (uint64_t b0 = w0 * kHashBlock; b0 < hi; b0 += waves * kHashBlock) {
     const uint64_t b1 = b0 + kHashBlock < hi ? b0 + kHashBlock : hi;
-    uint64_t i = b0 + lane;
-    uint64_t q = query_of_slot(a.offsets, nq, i < b1 ? i : b0);
-    uint64_t q_end = a.offsets[q] + a.counts[q];
-    uint64_t v_end = a.offsets[q] + a.exact[q];
-    uint32_t r = request_of_query(a.requests, h.n_requests, q);
-    uint64_t r_end = r + 1 < h.n_requests ? a.requests[r + 1].qbase : nq;
-    uint64_t hs = 0;
-    for (; i < b1; i += kWave) {
-      while (i >= q_end && q + 1 < nq) {
-        q++;
-        q_end = a.offsets[q] + a.counts[q];
-        v_end = a.offsets[q] + a.exact[q];
-        while (q >= r_end) {
-          if (hs) atomicAdd(&hashes[r], (unsigned long long)hs);
-          hs = 0;
-          r++;
-          r_end = r + 1 < h.n_requests ? a.requests[r + 1].qbase : nq;
-        }
-      }
-      if (i < v_end && i >= a.offsets[q]) {
+    // The last request that starts at or before b0; earlier ones that start
+    // there too are empty.
+    uint32_t lo = 0, end = h.n_requests;
+    while (end - lo > 1) {
+      const uint32_t mid = (lo + end) >> 1;
+      if (a.ranges[2 * mid] <= b0) lo = mid; else end = mid;
+    }
+    for (uint32_t r = lo; r < h.n_requests; r++) {
+      const uint64_t s0 = a.ranges[2 * r], s1 = s0 + a.ranges[2 * r + 1];
+      if (s0 >= b1) break;
+      const uint64_t i0 = s0 > b0 ? s0 : b0, i1 = s1 < b1 ? s1 : b1;
+      if (i0 >= i1) continue;
+      uint64_t hs = 0;
+      for (uint64_t i = i0 + lane; i < i1; i += kWave) {
         const rts_pair p = a.arena[i];
         hs += pair_hash(p.query_id, p.geom_id);
       }
-    }
-    const uint32_t r0 = readlane_u32(r, 0);
-    if (__all(r == r0)) {
       hs = wave_sum_u64(hs);
-      if (lane == 0 && hs) atomicAdd(&hashes[r0], (unsigned long long)hs);
-    } else if (hs) {
-      atomicAdd(&hashes[r], (unsigned long long)hs);
+      if (lane == 0 && hs) atomicAdd(&hashes[r], (unsigned long long)hs);
     }
-  }
-}
-
-// Pairs of queries [q0, q0 + n) to out[0, take), in query order: one
-// wavefront per query.
-__global__ void __launch_bounds__(kThreads) k_copy_queries(const BatchArgs a, uint64_t q0,
-                                                           uint64_t n, rts_pair* __restrict__ out,
-                                                           uint64_t take) {
-  const uint32_t lane = lane_id();
-  const uint64_t waves = (uint64_t)gridDim.x * kWaves;
-  const uint64_t base = a.exact_offsets[q0];
-  for (uint64_t j = (uint64_t)blockIdx.x * kWaves + threadIdx.x / kWave; j < n; j += waves) {
-    const uint64_t q = q0 + j;
-    const uint64_t d = a.exact_offsets[q] - base;
-    if (d >= take) continue;
-    const uint64_t e = a.exact[q];
-    const uint64_t m = d + e < take ? e : take - d;
-    const uint64_t o = a.offsets[q];
-    for (uint64_t i = lane; i < m && o + i < a.arena_cap; i += kWave) out[d + i] = a.arena[o + i];
   }
 }
 
@@ -641,18 +505,9 @@ __global__ void __launch_bounds__(kThreads) k_rebase_hash_span(rts_pair* __restr
 
 }  // namespace
 
-hipError_t launch_hash_queries(const BatchArgs& a, unsigned long long* hashes,
-                               hipStream_t stream) {
-  hipLaunchKernelGGL(k_hash_queries, dim3(4096), dim3(kThreads), 0, stream, a, hashes);
-  return hipGetLastError();
-}
-
-hipError_t launch_copy_queries(const BatchArgs& a, uint64_t q0, uint64_t n, rts_pair* out,
-                               uint64_t take, hipStream_t stream) {
-  if (n == 0 || take == 0) return hipSuccess;
-  const uint64_t blocks = std::min<uint64_t>((n + kWaves - 1) / kWaves, 4096);
-  hipLaunchKernelGGL(k_copy_queries, dim3((uint32_t)blocks), dim3(kThreads), 0, stream, a, q0, n,
-                     out, take);
+hipError_t launch_hash_requests(const BatchArgs& a, unsigned long long* hashes,
+                                hipStream_t stream) {
+  hipLaunchKernelGGL(k_hash_requests, dim3(4096), dim3(kThreads), 0, stream, a, hashes);
   return hipGetLastError();
 }
 

@@ -58,10 +58,10 @@ __host__ __device__ inline int tile_class(uint32_t flags) {
 constexpr int kGiantBuckets = 3;
 __host__ __device__ constexpr uint32_t giant_min(int b) { return 1u << (20 - 2 * b); }
 
-// Tile counters of a batch, each on its own 64-byte line, zeroed by the
+// Tile counters of a batch, 256 bytes apart (traverse.h), zeroed by the
 // batch's first launch: for each pass (count, write), class and XCD one tile
 // counter, then per giant bucket an append and a take counter.
-constexpr uint32_t kCounterStride = 16;
+constexpr uint32_t kCounterStride = 64;
 constexpr uint32_t kTileCounterWords = (2 * kClasses * 8 + 2 * kGiantBuckets) * kCounterStride;
 constexpr uint32_t kGiantCounterOff = 2 * kClasses * 8 * kCounterStride;
 
@@ -125,6 +125,7 @@ struct BatchExt {
 };
 struct BatchExtArgs {
   uint32_t* tickets;     // kWaveTicketWords words
+  uint32_t* heavy;       // wave_heavy_words(the batch's queries) words
   const uint64_t* zero;  // a device 0 (queue base of the arena)
   const void* arena_queue;  // device rts_dev_queue over the slot's arena
 };

@@ -650,7 +650,8 @@ struct QueryScratch {
   uint64_t* offsets = nullptr;      //                exclusive scan of counts
   uint64_t* total = nullptr;        //                [0] total, [1] queue base
   void* scan_tmp = nullptr;
-  uint32_t* tickets = nullptr;      // wave traversal: per-XCD query tickets
+  uint32_t* tickets = nullptr;      // wave traversal: counters
+  uint32_t* heavy = nullptr;        //                 queries left to whole waves
   RangeLogArgs log;                 // wave two-pass: the count walks' range logs
 };
 
@@ -663,7 +664,7 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
                   QueryScratch* qs, size_t* order_off, size_t* sort_off, char* ext = nullptr,
                   size_t ext_bytes = 0, char** base_out = nullptr) {
   size_t off = 0;
-  size_t o_keys = 0, o_sort = 0, o_counts = 0, o_offsets = 0, o_total = 0, o_scan = 0, o_tk = 0;
+  size_t o_keys = 0, o_sort = 0, o_counts = 0, o_offsets = 0, o_total = 0, o_scan = 0, o_tk = 0, o_heavy = 0;
   size_t o_log = 0, o_log_off = 0, o_log_n = 0;
   // Range logs: not in a caller's static scratch.
   const bool logs = two_pass && !ext;
@@ -671,6 +672,8 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
   if (wave) {
     o_tk = off;
     off = align_up(off + kWaveTicketWords * sizeof(uint32_t));
+    o_heavy = off;
+    off = align_up(off + wave_heavy_words(nq) * sizeof(uint32_t));
   }
   if (sort) {
     o_keys = off;
@@ -706,7 +709,10 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
     b = qs->block.get();
   }
   if (base_out) *base_out = b;
-  if (wave) qs->tickets = reinterpret_cast<uint32_t*>(b + o_tk);
+  if (wave) {
+    qs->tickets = reinterpret_cast<uint32_t*>(b + o_tk);
+    qs->heavy = reinterpret_cast<uint32_t*>(b + o_heavy);
+  }
   if (two_pass) {
     qs->counts = reinterpret_cast<uint32_t*>(b + o_counts);
     qs->offsets = reinterpret_cast<uint64_t*>(b + o_offsets);
@@ -857,12 +863,12 @@ int run_plan(rts_index* ix, const Plan& plan, int pred, const void* queries, uin
         RTS_HIP(launch_query(ql, stream));
         phase_end(ph, stream);
       } else if (!two_pass) {
-        WaveArgs wa{nullptr, nullptr, nullptr, qs.tickets};
+        WaveArgs wa{nullptr, nullptr, nullptr, qs.tickets, qs.heavy, {}};
         PhaseToken ph = phase_begin(RTS_PHASE_TRAVERSE, stream);
         RTS_HIP(launch_query_wave(ql, wa, staged ? kPhaseWriteStaged : kPhaseCountSink, stream));
         phase_end(ph, stream);
       } else {
-        WaveArgs wa{qs.counts, qs.offsets, qs.total + 1, qs.tickets, qs.log};
+        WaveArgs wa{qs.counts, qs.offsets, qs.total + 1, qs.tickets, qs.heavy, qs.log};
         PhaseToken ph = phase_begin(RTS_PHASE_QUERY_COUNT, stream);
         RTS_HIP(launch_query_wave(ql, wa, kPhaseCount, stream));
         RTS_HIP(launch_exclusive_scan(qs.counts, m, qs.offsets, qs.total, qs.scan_tmp, stream));

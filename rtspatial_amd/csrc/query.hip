@@ -16,6 +16,8 @@
 // slots with one atomic per ~1000 pairs, in place of the reference's one
 // atomic per result (utils/queue.h:22-27); a wave kernel counts, scans and
 // then writes each query's pairs contiguously.
+#include <algorithm>
+
 #include "rts_internal.h"
 #include "range_log.h"
 #include "rtspatial/device/traverse.h"
@@ -168,17 +170,223 @@ __global__ void __launch_bounds__(kOctThreads)
 }
 
 // ----------------------------------------------------------------- wave ----
-// Per-request wave traversal (wide.h wide_walk): kWaveCount writes the
-// query's result count to counts[query]; kWaveCountSink adds it to the
-// counting handler's counter; kWaveWrite writes the pairs at queue slot
+// Wavefront calls. A counting kernel writes each query's result count to
+// counts[query], logging the results (range_log.h), or adds them to the
+// counting handler's counter; the write kernel emits the logs at queue slot
 // base + offsets[query] (offsets from the scan of the counts), so the queue
-// holds each query's pairs contiguously, in query order. kWaveStaged
-// collects in one pass, for walks whose count pass would cost as much as
-// the write (segments: no subtree lies inside a segment): each wavefront
-// stages its pairs in LDS and flushes them with one device atomic per
-// kStageWave pairs; a query's pairs may then be split over flushes.
-enum { kWaveCount = 0, kWaveCountSink = 1, kWaveWrite = 2, kWaveStaged = 3 };
+// holds each query's pairs contiguously, in query order. The staged kernel
+// collects segment walks in one pass where there is no room for logs: each
+// wavefront stages its pairs in LDS and flushes them with one device atomic
+// per kStageWave pairs; a query's pairs may then be split over flushes.
+//
+// Large calls run twice per pass. First the octets of a wave take one query
+// each, kGroup queries per ticket, which answers those of a few leaf blocks
+// eight at a time; the others are listed (one atomic per ticket), and the
+// second launch's waves walk or write them one by one. A wave half of whose
+// queries turn out heavy lists kSkip tickets without trying. 1M within queries
+// of 20 results count in 0.51 and write in 0.31 ms (1.58 and 1.22 ms a wave
+// each; 3.3 and 2.6 ms on the binary tree); on the 10M x 1M join, whose
+// queries are heavy, the trial costs 0.3 of 5 ms. (Having the same wave walk
+// its heavy queries made the join with 200k queries 1.7x slower: sixteen long
+// walks in a row on some waves, none on others.)
+constexpr uint32_t kGroup = 16;
+constexpr uint32_t kSkip = 7;
+constexpr uint32_t kHeavyGroup = 2;
 constexpr uint32_t kStageWave = 512;
+
+__device__ __forceinline__ uint32_t* wave_counters(uint32_t* tickets, uint32_t kind) {
+  return tickets + kind * kXcds * kTicketStride;
+}
+static_assert(kTicketStride == kTicketWords && kXcds == kTicketXcds, "counter layout");
+__device__ __forceinline__ unsigned long long* sum_slot(uint32_t* tickets, uint32_t i) {
+  return reinterpret_cast<unsigned long long*>(tickets +
+                                               (kTicketKinds * kXcds + i) * kTicketStride);
+}
+
+// Counts of the waves are spread over kSumSlots words and added up by
+// k_sum_counts: one atomic per query on the handler's counter made the 10M x
+// 1M join wait for it (1M atomics on one address, 14 ns each).
+__device__ __forceinline__ void add_sum(uint32_t* tickets, uint64_t sum) {
+  if (lane_id() == 0 && sum)
+    atomicAdd(sum_slot(tickets, blockIdx.x % kSumSlots), (unsigned long long)sum);
+}
+
+// The octets' count pass. One wavefront per workgroup, so that a wave's LDS is
+// released by itself (here and below).
+template <int PRED, bool POINTS, bool LOG, bool F64>
+__global__ void __launch_bounds__(kWave) k_light_count(const QueryLaunch q, const WaveArgs a,
+                                                       const uint32_t group) {
+  __shared__ uint32_t s_stack[kWave / kFan][kOctStack];
+  __shared__ uint2 s_log[LOG ? kWave / kFan : 1][LOG ? kOctLog : 1];
+  const TreeView t = q.tree;
+  const OctSource<PRED, POINTS, F64> src{q.queries, q.order};
+  const uint32_t lane = lane_id(), oct = lane / kFan;
+  SliceTickets tickets =
+      slice_tickets(wave_counters(a.tickets, kTicketsLight), wave_counters(a.tickets, kFlagsLight),
+                    slice_size(q.n), group);
+  const uint32_t per = slice_length(q.n);
+  LogCursor lc = LOG ? log_cursor(a.log) : LogCursor{};
+  uint64_t sum = 0;  // octet-uniform: without LOG
+  uint32_t skip = 0;
+  // Every iteration takes a query or finds none left.
+  for (uint32_t it = 0; it <= q.n; it++) {
+    uint32_t lin, end;
+    bool late;
+    if (!next_items(tickets, group, &lin, &end, &late)) break;
+    const uint32_t m = end - lin;
+    lin += tickets.slice * per;
+    uint32_t todo = (1u << m) - 1u;
+    if (m < (uint32_t)kFan || skip) {
+      skip -= skip ? 1u : 0u;
+    } else {
+      auto commit = [&](bool done, uint32_t i, uint32_t found, uint32_t n, const uint2* log) {
+        if (LOG) {
+          const uint32_t qi = q.order && done ? q.order[i] : i;
+          if (!log_commit_octets(lc, a.log, done, qi, n, log)) return false;
+          if (done && (lane & 7u) == 0) a.counts[qi] = found;
+        } else if (done) {
+          sum += found;
+        }
+        return true;
+      };
+      todo = oct_count<PRED, POINTS, LOG, query_t<PRED, F64>>(
+          t, s_stack[oct], s_log[LOG ? oct : 0], lin, lin + m, src, commit);
+      if (2u * (uint32_t)__popc(todo) >= m) skip = kSkip;
+    }
+    if (todo) {  // onto the slice's list
+      uint32_t at = 0;
+      if (lane == 0)
+        at = atomicAdd(wave_counters(a.tickets, kHeavyCount) + tickets.slice * kTicketStride,
+                       (uint32_t)__popc(todo));
+      at = readlane_u32(at, 0);
+      if (lane < m && ((todo >> lane) & 1u))
+        a.heavy[tickets.slice * per + at + (uint32_t)__popc(todo & ((1u << lane) - 1u))] =
+            q.order ? q.order[lin + lane] : lin + lane;
+    }
+  }
+  if (!LOG) add_sum(a.tickets, wave_sum_u64((lane & 7u) == 0 ? sum : 0));
+}
+
+// Queries of a wave-by-wave launch: those the octets listed (LISTED), or all.
+struct WaveQueries {
+  SliceTickets tickets;
+  uint32_t per;
+};
+template <bool LISTED>
+__device__ __forceinline__ WaveQueries wave_queries(const QueryLaunch& q, const WaveArgs& a,
+                                                    uint32_t group) {
+  const uint32_t size =
+      LISTED ? wave_counters(a.tickets, kHeavyCount)[lane_id() % kXcds * kTicketStride]
+             : slice_size(q.n);
+  return WaveQueries{slice_tickets(wave_counters(a.tickets, kTicketsHeavy),
+                                   wave_counters(a.tickets, kFlagsHeavy), size, group),
+                     slice_length(q.n)};
+}
+template <bool LISTED>
+__device__ __forceinline__ uint32_t wave_query_id(const QueryLaunch& q, const WaveArgs& a,
+                                                  uint32_t at) {
+  return LISTED ? a.heavy[at] : (q.order ? q.order[at] : at);
+}
+
+template <int PRED, bool POINTS, bool LOG, bool F64, bool LISTED>
+__global__ void __launch_bounds__(kWave) k_wave_count(const QueryLaunch q, const WaveArgs a,
+                                                      const uint32_t group) {
+  __shared__ WideLds s_lds;
+  const TreeView t = q.tree;
+  WaveQueries w = wave_queries<LISTED>(q, a, group);
+  LogCursor lc = LOG ? log_cursor(a.log) : LogCursor{};
+  uint64_t sum = 0;  // wave-uniform: without LOG
+  uint32_t want = group;
+  for (uint32_t it = 0; it <= q.n; it++) {
+    uint32_t lin, end;
+    bool late;
+    if (!next_items(w.tickets, want, &lin, &end, &late)) break;
+    want = late ? 1u : group;
+    for (; lin < end; lin++) {
+      const uint32_t qi =
+          readlane_u32(wave_query_id<LISTED>(q, a, w.tickets.slice * w.per + lin), 0);
+      query_t<PRED, F64> qb;
+      load_q(q.queries, POINTS, qi, qb);
+      if (LOG) {
+        RangeLog lg = log_for_count(lc);
+        const uint64_t all = wide_walk<PRED, POINTS, false, true>(t, qb, 0, NoEmit{}, s_lds, &lg);
+        log_commit(lc, a.log, qi, lg);
+        if (lane_id() == 0) a.counts[qi] = (uint32_t)all;
+      } else {
+        sum += wide_walk<PRED, POINTS, false, false>(t, qb, 0, NoEmit{}, s_lds);
+      }
+    }
+  }
+  if (!LOG) add_sum(a.tickets, sum);
+}
+
+// The octets' write pass: every query whose log an octet made.
+__global__ void __launch_bounds__(kWave) k_light_write(const QueryLaunch q, const WaveArgs a,
+                                                       const uint32_t group) {
+  const TreeView t = q.tree;
+  const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
+  rts_pair* out = dq->data;
+  const uint64_t cap = dq->capacity;
+  const uint32_t lane = lane_id();
+  SliceTickets tickets =
+      slice_tickets(wave_counters(a.tickets, kTicketsLight), wave_counters(a.tickets, kFlagsLight),
+                    slice_size(q.n), group);
+  const uint32_t per = slice_length(q.n);
+  for (uint32_t it = 0; it <= q.n; it++) {
+    uint32_t lin, end;
+    bool late;
+    if (!next_items(tickets, group, &lin, &end, &late)) break;
+    const uint32_t m = end - lin;  // at most kWave
+    lin += tickets.slice * per;
+    // Lane l: query lin + l.
+    uint32_t qi = 0, n = 0, off = 0;
+    uint64_t slot = 0;
+    if (lane < m) {
+      qi = q.order ? q.order[lin + lane] : lin + lane;
+      n = a.log.n[qi];
+      off = a.log.off[qi];
+      slot = a.base[0] + a.offsets[qi];
+      if (n & kLogWave) n = 0;
+    }
+    if (!ballot(n != 0)) continue;
+    for (uint32_t b = 0; b < m; b += kWave / kFan) {
+      const int l = (int)(b + lane / kFan);
+      const uint32_t ln = (uint32_t)__shfl((int)n, l, 64), lo = (uint32_t)__shfl((int)off, l, 64);
+      const uint32_t lq = (uint32_t)__shfl((int)qi, l, 64);
+      const uint64_t ls = __shfl(slot, l, 64);
+      oct_replay(t, a.log.entries + lo, ln, out, cap, ls, lq + q.qid_base);
+    }
+  }
+}
+
+template <int PRED, bool POINTS, bool F64, bool LISTED>
+__global__ void __launch_bounds__(kWave) k_wave_write(const QueryLaunch q, const WaveArgs a,
+                                                      const uint32_t group) {
+  __shared__ WideLds s_lds;
+  const TreeView t = q.tree;
+  const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
+  WaveQueries w = wave_queries<LISTED>(q, a, group);
+  uint32_t want = group;
+  for (uint32_t it = 0; it <= q.n; it++) {
+    uint32_t lin, end;
+    bool late;
+    if (!next_items(w.tickets, want, &lin, &end, &late)) break;
+    want = late ? 1u : group;
+    for (; lin < end; lin++) {
+      const uint32_t qi =
+          readlane_u32(wave_query_id<LISTED>(q, a, w.tickets.slice * w.per + lin), 0);
+      const QueueEmit emit{dq->data, dq->capacity, a.base[0] + a.offsets[qi]};
+      const RangeLog lg = log_for_write(a.log, qi);
+      if (lg.n_in != kLogOverflow) {
+        wide_replay(t, lg, qi + q.qid_base, emit);
+      } else {
+        query_t<PRED, F64> qb;
+        load_q(q.queries, POINTS, qi, qb);
+        wide_walk<PRED, POINTS, true, false>(t, qb, qi + q.qid_base, emit, s_lds);
+      }
+    }
+  }
+}
 
 struct StagedEmit {
   rts_pair* stage;  // LDS, kStageWave pairs
@@ -207,71 +415,40 @@ struct StagedEmit {
   }
 };
 
-// One wavefront per workgroup, so that a wave's LDS is released by itself.
-template <int PRED, bool POINTS, int MODE, bool F64>
-__global__ void __launch_bounds__(kWave) k_query_wave(const QueryLaunch q, const WaveArgs a) {
+template <int PRED, bool POINTS, bool F64>
+__global__ void __launch_bounds__(kWave) k_wave_staged(const QueryLaunch q, const WaveArgs a,
+                                                       const uint32_t group) {
   __shared__ WideLds s_lds;
-  __shared__ rts_pair s_stage[MODE == kWaveStaged ? kStageWave : 1];
+  __shared__ rts_pair s_stage[kStageWave];
   const TreeView t = q.tree;
-  StagedEmit se{s_stage, nullptr, nullptr, 0};
-  if (MODE == kWaveStaged) {
-    const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
-    se.counter = dq->counter;
-    se.out = dq->data;
-    se.cap = dq->capacity;
-  }
-  uint32_t slice = blockIdx.x % kXcds;
-  LogCursor lc = MODE == kWaveCount ? log_cursor(a.log) : LogCursor{};
-  uint64_t sum = 0;  // wave-uniform: kWaveCountSink
-  // Every iteration takes a ticket or finds none left: q.n + 1 iterations
-  // bound the loop.
+  const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
+  StagedEmit se{s_stage, dq->counter, dq->data, dq->capacity};
+  WaveQueries w = wave_queries<false>(q, a, group);
+  uint32_t want = group;
   for (uint32_t it = 0; it <= q.n; it++) {
-    uint32_t lin, lin_end;
-    grab_queries(a.tickets, q.n, slice, &lin, &lin_end);
-    if (lin >= lin_end) break;
-    for (; lin < lin_end; lin++) {
-      const uint32_t qi = q.order ? readlane_u32(q.order[lin], 0) : lin;
-      if (MODE == kWaveWrite) {
-        // The count walk's log is emitted; a query whose log did not fit is
-        // walked again.
-        const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
-        const QueueEmit emit{dq->data, dq->capacity, a.base[0] + a.offsets[qi]};
-        const RangeLog lg = log_for_write(a.log, qi);
-        if (lg.n_in != kLogOverflow) {
-          wide_replay(t, lg, qi + q.qid_base, emit);
-          continue;
-        }
-      }
+    uint32_t lin, end;
+    bool late;
+    if (!next_items(w.tickets, want, &lin, &end, &late)) break;
+    want = late ? 1u : group;
+    for (; lin < end; lin++) {
+      const uint32_t qi =
+          readlane_u32(wave_query_id<false>(q, a, w.tickets.slice * w.per + lin), 0);
       query_t<PRED, F64> qb;
       load_q(q.queries, POINTS, qi, qb);
-      if (MODE == kWaveWrite) {
-        const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
-        wide_walk<PRED, POINTS, true, false>(
-            t, qb, qi + q.qid_base, QueueEmit{dq->data, dq->capacity, a.base[0] + a.offsets[qi]},
-            s_lds);
-      } else if (MODE == kWaveStaged) {
-        wide_walk<PRED, POINTS, true, false>(t, qb, qi + q.qid_base, se, s_lds);
-      } else if (MODE == kWaveCount) {
-        RangeLog lg = log_for_count(lc);
-        const uint64_t all = wide_walk<PRED, POINTS, false, true>(t, qb, 0, NoEmit{}, s_lds, &lg);
-        log_commit(lc, a.log, qi, lg);
-        if (lane_id() == 0) a.counts[qi] = (uint32_t)all;
-      } else {
-        sum += wide_walk<PRED, POINTS, false, false>(t, qb, 0, NoEmit{}, s_lds);
-      }
+      wide_walk<PRED, POINTS, true, false>(t, qb, qi + q.qid_base, se, s_lds);
     }
   }
-  if (MODE == kWaveStaged) se.flush();
-  // Counts of the waves are spread over kSumSlots words and added up by
-  // k_sum_counts: one atomic per query on the handler's counter made the
-  // 10M x 1M join wait for it (1M atomics on one address, 14 ns each).
-  if (MODE == kWaveCountSink && lane_id() == 0 && sum)
-    atomicAdd(wave_sums(a.tickets) + blockIdx.x % kSumSlots, (unsigned long long)sum);
+  se.flush();
 }
 
-__global__ void __launch_bounds__(kWave) k_sum_counts(const unsigned long long* __restrict__ sums,
+__global__ void __launch_bounds__(256) k_clear_counters(uint32_t* p, uint32_t lines) {
+  for (uint32_t i = threadIdx.x; i < lines * kXcds; i += 256)
+    p[i / kXcds * kTicketStride + i % kXcds] = 0;
+}
+
+__global__ void __launch_bounds__(kWave) k_sum_counts(uint32_t* tickets,
                                                       unsigned long long* counter) {
-  const uint64_t s = wave_sum_u64(sums[threadIdx.x]);
+  const uint64_t s = wave_sum_u64(threadIdx.x < kSumSlots ? *sum_slot(tickets, threadIdx.x) : 0);
   if (threadIdx.x == 0 && s) atomicAdd(counter, (unsigned long long)s);
 }
 
@@ -285,41 +462,107 @@ uint32_t device_cus() {
   return cus;
 }
 
-// Persistent grid: 32 single-wave workgroups per CU, the most waves a CU
-// holds. Occupancy (VGPRs, LDS) admits fewer at once; the rest start as
-// waves finish and exit as soon as they find every slice drained.
-template <int PRED, bool POINTS, int MODE, bool F64>
-hipError_t launch_wave_mode(const QueryLaunch& q, const WaveArgs& a_in, hipStream_t stream) {
-  hipError_t e = launch_fill_u32(a_in.tickets, 0u, kWaveTicketWords, stream);
-  if (e != hipSuccess) return e;
-  const uint32_t resident = device_cus() * 32;
-  uint32_t blocks = resident < q.n ? resident : q.n;
-  blocks = (blocks + kXcds - 1) / kXcds * kXcds;  // whole rounds over the XCDs
-  WaveArgs a = a_in;
-  if (blocks) a.log.per_wave = (uint32_t)(a.log.n_entries / blocks);
-  hipLaunchKernelGGL((k_query_wave<PRED, POINTS, MODE, F64>), dim3(blocks), dim3(kWave), 0, stream,
-                     q, a);
-  if (MODE == kWaveCountSink)
-    hipLaunchKernelGGL(k_sum_counts, dim3(1), dim3(kSumSlots), 0, stream, wave_sums(a.tickets),
-                       static_cast<unsigned long long*>(const_cast<void*>(q.sink.arg)));
-  return hipGetLastError();
+// The single-wave workgroups of `kernel` that the device holds at once.
+template <typename K>
+uint32_t resident_waves(K kernel) {
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kWave, 0) != hipSuccess ||
+      per_cu <= 0)
+    per_cu = 24;
+  return device_cus() * (uint32_t)per_cu;
+}
+
+// A persistent grid for n queries, `group` to a ticket, in whole rounds over
+// the XCDs.
+template <typename K>
+void launch_persistent(K kernel, uint32_t resident, uint32_t group, const QueryLaunch& q,
+                       WaveArgs a, uint64_t log_first, uint64_t log_entries, hipStream_t stream) {
+  uint32_t blocks = std::min((q.n + group - 1) / group, resident);
+  blocks = (blocks + kXcds - 1) / kXcds * kXcds;
+  a.log.first = (uint32_t)log_first;
+  a.log.per_wave = (uint32_t)(log_entries / blocks);
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWave), 0, stream, q, a, group);
+}
+
+// Calls of at least kOctetTickets queries per wave run the octets first, 8 to a
+// ticket, and 16 once every wave gets one; smaller ones leave each wave up to
+// kFewQueries queries of its own, without tickets. (20k intersects queries of
+// 1000 results: 0.30 ms so, 0.36 with octets; 30k within queries of 20: 0.16
+// without octets, 0.09 with them.)
+constexpr uint32_t kFewQueries = 4;
+constexpr uint32_t kOctetTickets = 3;
+uint32_t octet_group(uint32_t n) {
+  const uint32_t waves = device_cus() * 32;
+  return n >= kGroup * waves ? kGroup : n >= kOctetTickets * waves ? 8u : 0u;
+}
+
+template <int PRED, bool POINTS, bool LOG, bool F64>
+void launch_count(const QueryLaunch& q, const WaveArgs& a, hipStream_t stream) {
+  auto* all = &k_wave_count<PRED, POINTS, LOG, F64, false>;
+  auto* listed = &k_wave_count<PRED, POINTS, LOG, F64, true>;
+  auto* light = &k_light_count<PRED, POINTS, LOG, F64>;
+  static const uint32_t r_all = resident_waves(all), r_listed = resident_waves(listed),
+                        r_light = resident_waves(light);
+  const uint32_t group = octet_group(q.n);
+  if (!group) {
+    const uint32_t few = std::max(1u, std::min(kFewQueries, (q.n + r_all - 1) / r_all));
+    launch_persistent(all, r_all, few, q, a, 0, a.log.n_entries, stream);
+    return;
+  }
+  // An octet's query logs at most kOctLog entries.
+  const uint64_t first = std::min<uint64_t>((uint64_t)q.n * kOctLog, a.log.n_entries / 4);
+  launch_persistent(light, r_light, group, q, a, 0, first, stream);
+  launch_persistent(listed, r_listed, kHeavyGroup, q, a, first, a.log.n_entries - first, stream);
 }
 
 template <int PRED, bool POINTS, bool F64>
 hipError_t launch_wave_f(const QueryLaunch& q, const WaveArgs& a, int phase, hipStream_t stream) {
   switch (phase) {
-    case kWaveCount:
-      return launch_wave_mode<PRED, POINTS, kWaveCount, F64>(q, a, stream);
-    case kWaveCountSink:
-      return launch_wave_mode<PRED, POINTS, kWaveCountSink, F64>(q, a, stream);
-    case kWaveStaged:
+    case kPhaseCount:
+    case kPhaseCountSink:
+      hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, stream, a.tickets,
+                         kTicketKinds * kXcds + kSumSlots);
+      if (phase == kPhaseCount) {
+        launch_count<PRED, POINTS, true, F64>(q, a, stream);
+      } else {
+        launch_count<PRED, POINTS, false, F64>(q, a, stream);
+        hipLaunchKernelGGL(k_sum_counts, dim3(1), dim3(kWave), 0, stream, a.tickets,
+                           static_cast<unsigned long long*>(const_cast<void*>(q.sink.arg)));
+      }
+      break;
+    case kPhaseWriteStaged: {
       // Only segment walks are staged.
-      if constexpr (PRED == kPredLine)
-        return launch_wave_mode<PRED, POINTS, kWaveStaged, F64>(q, a, stream);
+      if constexpr (PRED == kPredLine) {
+        auto* k = &k_wave_staged<PRED, POINTS, F64>;
+        static const uint32_t resident = resident_waves(k);
+        hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, stream, a.tickets,
+                           kTicketKinds * kXcds);
+        launch_persistent(k, resident, 1, q, a, 0, 0, stream);
+        break;
+      }
       return hipErrorInvalidValue;
-    default:
-      return launch_wave_mode<PRED, POINTS, kWaveWrite, F64>(q, a, stream);
+    }
+    default: {
+      auto* all = &k_wave_write<PRED, POINTS, F64, false>;
+      auto* listed = &k_wave_write<PRED, POINTS, F64, true>;
+      static const uint32_t r_all = resident_waves(all), r_listed = resident_waves(listed),
+                            r_light = resident_waves(&k_light_write);
+      // The count pass's tickets are taken: new ones, but its list of heavy
+      // queries stays.
+      const uint32_t group = octet_group(q.n);
+      hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, stream, a.tickets,
+                         kHeavyCount * kXcds);
+      if (!group || !a.log.entries) {
+        const uint32_t few = std::max(1u, std::min(kFewQueries, (q.n + r_all - 1) / r_all));
+        launch_persistent(all, r_all, few, q, a, 0, 0, stream);
+      } else {
+        launch_persistent(&k_light_write, r_light, group, q, a, 0, 0, stream);
+        launch_persistent(listed, r_listed, kHeavyGroup, q, a, 0, 0, stream);
+      }
+      break;
+    }
   }
+  return hipGetLastError();
 }
 
 template <int PRED, bool POINTS>

@@ -23,6 +23,9 @@ namespace rts {
 constexpr uint32_t kLogQueryMax = 4096;
 constexpr uint32_t kLogOverflow = 0xFFFFFFFFu;
 constexpr uint32_t kLogRange = 0x80000000u;
+// A header's entry count carries this bit when a wave walked the query (its log
+// is then written by a wave too).
+constexpr uint32_t kLogWave = 0x40000000u;
 
 // Log entries bypass the caches both ways (written once, read once), so
 // that they do not evict the nodes and leaf data the walks re-read.
@@ -54,7 +57,7 @@ struct LogCursor {
 __device__ __forceinline__ LogCursor log_cursor(const RangeLogArgs& la) {
   LogCursor c;
   if (la.entries) {
-    c.base = blockIdx.x * la.per_wave;
+    c.base = la.first + blockIdx.x * la.per_wave;
     c.region = la.entries + c.base;
     c.room = la.per_wave;
   }
@@ -79,10 +82,34 @@ __device__ __forceinline__ void log_commit(LogCursor& c, const RangeLogArgs& la,
   if (!c.region) return;
   const bool fit = lg.logged <= lg.cap;
   if (lane_id() == 0) {
-    la.n[g] = fit ? lg.logged : kLogOverflow;
+    la.n[g] = fit ? lg.logged | kLogWave : kLogOverflow;
     la.off[g] = c.base + c.fill;
   }
   if (fit) c.fill += lg.logged;
+}
+
+// After octets completed queries (`done`, octet-uniform, as are g, n and the
+// n entries in `log`, in LDS): their entries and headers. Called by the whole
+// wave. False: they do not fit the wave's region and are not logged.
+__device__ __forceinline__ bool log_commit_octets(LogCursor& c, const RangeLogArgs& la, bool done,
+                                                  uint64_t g, uint32_t n, const uint2* log) {
+  if (!c.region) return true;
+  const uint32_t lane = lane_id(), j = lane & 7u;
+  const uint32_t mine = done && j == 0 ? n : 0u;
+  const uint32_t inc = wave_inclusive_sum(mine);
+  const uint32_t total = readlane_u32(inc, kWave - 1);
+  if (total > c.room - c.fill) return false;
+  // Lane 8o's inclusive sum less its own is octet o's place.
+  const uint32_t at = c.fill + (uint32_t)__shfl((int)(inc - mine), (int)(lane & ~7u), 64);
+  if (done) {
+    for (uint32_t k = j; k < n; k += 8) log_store(c.region + at + k, log[k].x, log[k].y);
+    if (j == 0) {
+      la.n[g] = n;
+      la.off[g] = c.base + at;
+    }
+  }
+  c.fill += total;
+  return true;
 }
 
 // The log a writing walk of query g replays (n_in = kLogOverflow: none).
@@ -91,6 +118,7 @@ __device__ __forceinline__ RangeLog log_for_write(const RangeLogArgs& la, uint64
   if (la.entries) {
     // Wave-uniform values, kept in scalar registers.
     lg.n_in = readlane_u32(la.n[g], 0);
+    if (lg.n_in != kLogOverflow) lg.n_in &= ~kLogWave;
     lg.cap = kLogQueryMax;
     lg.entries = la.entries + readlane_u32(la.off[g], 0);
   }

@@ -164,7 +164,8 @@ hipError_t launch_query(const QueryLaunch& q, hipStream_t stream);
 struct RangeLogArgs {
   uint2* entries = nullptr;  // null: no logs (both passes walk the tree)
   uint64_t n_entries = 0;    // below 2^32
-  uint32_t per_wave = 0;     // entries of one wave's region: set by the launch (n_entries / grid)
+  uint32_t first = 0;        // a launch's regions start here,
+  uint32_t per_wave = 0;     // with this many entries each (set by the launch)
   uint32_t* off = nullptr;   // per query: first entry
   uint32_t* n = nullptr;     // per query: entries, or kLogOverflow
 };
@@ -173,20 +174,22 @@ struct RangeLogArgs {
 constexpr uint64_t kLogPerQuery = 512;
 constexpr uint64_t kLogMaxEntries = 1ull << 29;
 
+// Counters of wave calls, on lines of 256 bytes: per kind one for each XCD (a
+// counter, or flags), then the counting launches' kSumSlots partial sums.
+enum { kTicketsLight = 0, kFlagsLight, kTicketsHeavy, kFlagsHeavy, kHeavyCount, kTicketKinds };
+constexpr uint32_t kTicketXcds = 8;
+constexpr uint32_t kTicketWords = 64;
+constexpr uint32_t kSumSlots = 32;
+constexpr uint32_t kWaveTicketWords = (kTicketKinds * kTicketXcds + kSumSlots) * kTicketWords;
 struct WaveArgs {
   uint32_t* counts;
   const uint64_t* offsets;
   const uint64_t* base;
-  uint32_t* tickets;  // kWaveTicketWords words, cleared by the launch
+  uint32_t* tickets;  // kWaveTicketWords words
+  uint32_t* heavy;    // queries the octets left to the waves (room for wave_heavy_words(n))
   RangeLogArgs log;   // two-pass calls: the count walks' range logs
 };
-// Tickets (one 64-byte line per XCD), then the counting launches' kSumSlots
-// partial sums.
-constexpr uint32_t kSumSlots = 64;
-constexpr uint32_t kWaveTicketWords = 8 * 16 + 2 * kSumSlots;
-__host__ __device__ inline unsigned long long* wave_sums(uint32_t* tickets) {
-  return reinterpret_cast<unsigned long long*>(tickets + 8 * 16);
-}
+inline uint64_t wave_heavy_words(uint64_t n) { return n + kTicketXcds; }
 // Wave-per-query traversal. phase 0: per-query counts -> a.counts;
 // 1: counts added to the counting handler's counter; 2: pairs written at
 // queue slot a.base[0] + a.offsets[query]; 3: pairs collected in one pass

@@ -149,6 +149,7 @@ struct Slot {
   Scratch block;                         // the device buffers below
   char* d_desc = nullptr;
   uint32_t* d_counters = nullptr;
+  uint32_t* d_heavy = nullptr;   // extension requests: wave_heavy_words(max_batch_queries)
   uint32_t* d_giants = nullptr;  // kGiantBuckets x max_batch_queries tile ids
   uint2* d_log = nullptr;        // range-log entries (kServeLogPerQuery per query)
   uint32_t* d_log_off = nullptr; // per query: first range-log entry
@@ -421,7 +422,7 @@ int record_slot_work(Engine& E, Slot& s, size_t up_bytes, size_t n_req) {
   sort_scratch_carve(s.d_sort + 4 * maxq, maxq, &sort.ss);
   sort.scene = E.ix->scene;
   sort.n = wave_tiles >= E.cfg.sort_min_tiles ? wave_tiles : 0;
-  const BatchExtArgs ea{reinterpret_cast<uint32_t*>(s.d_ext + 64),
+  const BatchExtArgs ea{reinterpret_cast<uint32_t*>(s.d_ext + 64), s.d_heavy,
                         reinterpret_cast<const uint64_t*>(s.d_ext + 32), s.d_ext};
   SRV_HIP(launch_batch(reinterpret_cast<const TreeView*>(s.d_desc + kViewOff), a, sort,
                        s.ext.data(), s.ext.size(), ea, s.stream));
@@ -458,6 +459,7 @@ int slot_init(Engine& E, Slot& s) {
     carve(&s.d_desc, E.desc_bytes);
     carve(&s.d_counters, kTileCounterWords * sizeof(uint32_t));
     carve(&s.d_giants, kGiantBuckets * maxq * sizeof(uint32_t));
+    carve(&s.d_heavy, wave_heavy_words(maxq) * sizeof(uint32_t));
     carve(&s.d_log, serve_log_entries(maxq) * sizeof(uint2));
     carve(&s.d_log_off, maxq * sizeof(uint32_t));
     carve(&s.d_log_n, maxq * sizeof(uint32_t));

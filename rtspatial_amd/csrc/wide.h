@@ -51,46 +51,97 @@ __device__ __forceinline__ bool leaf_test(const TreeView&, uint32_t, const float
 }
 
 // -------------------------------------------------------------- tickets ----
-// Wave kernels take queries from per-XCD ticket counters as grab_query
-// (traverse.h) does, but the first three quarters of a slice kTicketQueries at
-// a time: a counter answers one atomic per ~14 ns, which at one query each
-// bounds a pass over 1M queries at 1.7 ms. The last quarter goes singly, so
-// that a heavy group is not left to one wave at the end.
-constexpr uint32_t kTicketQueries = 4;
+// Persistent waves take work from one counter per XCD, as traverse.h
+// describes, with the counters spared: an atomic or a coherent load takes
+// ~14 ns per address, and per memory channel (so counters lie 256 bytes
+// apart), whichever wave sends it. 8192 waves asking eight drained counters 64
+// bytes apart once more held the end of a pass for 0.2 ms, reading them 0.1
+// ms, and one query per ticket bounds a pass over 1M queries at 1.7 ms.
+//   - A wave's first items follow from its number, without an atomic.
+//   - Tickets are for `want` consecutive items of a slice.
+//   - A wave that finds a slice drained sets a flag of its XCD, in that XCD's
+//     L2, and goes on to a slice without one. The flags only spare attempts:
+//     a slice is drained when its counter says so.
+// Counters and flags (a line of kXcds words per XCD) are zero at the start;
+// the grid is whole rounds over the XCDs.
+struct SliceTickets {
+  uint32_t* counters;
+  uint32_t* flags;   // this XCD's
+  uint32_t size;     // lane l: items of slice l % kXcds
+  uint32_t given;    // items of each slice taken without tickets
+  uint32_t slice;    // slice to take from
+  uint32_t drained;  // slices known to be drained
+  bool first;
+};
 
-// The next queries [*begin, *end) for this wave; empty when every slice is
-// drained. `slice` is the slice to try first; it becomes the one taken from.
-__device__ __forceinline__ void grab_queries(uint32_t* tickets, uint32_t n, uint32_t& slice,
-                                             uint32_t* begin, uint32_t* end) {
-  const uint32_t per = (n + kXcds - 1) / kXcds;
-  uint32_t b = 0, e = 0, from = slice;
-  if (lane_id() == 0) {
-    for (uint32_t k = 0; k < kXcds; k++) {
-      const uint32_t x = (slice + k) % kXcds;
-      const uint32_t lo = x * per;
-      const uint32_t hi = lo + per < n ? lo + per : n;
-      if (lo >= hi) continue;
-      const uint32_t m = hi - lo;
-      const uint32_t groups = m / 4 * 3 / kTicketQueries;
-      const uint32_t v = atomicAdd(tickets + x * kTicketStride, 1u);
-      if (v < groups) {
-        b = lo + v * kTicketQueries;
-        e = b + kTicketQueries;
-        from = x;
-        break;
-      }
-      const uint32_t single = groups * kTicketQueries + (v - groups);
-      if (single < m) {
-        b = lo + single;
-        e = b + 1;
-        from = x;
-        break;
-      }
+__device__ __forceinline__ SliceTickets slice_tickets(uint32_t* counters, uint32_t* flags,
+                                                      uint32_t size, uint32_t first_want) {
+  SliceTickets q;
+  q.counters = counters;
+  q.flags = flags + blockIdx.x % kXcds * kTicketStride;
+  q.size = size;
+  q.given = gridDim.x / kXcds * first_want;
+  q.slice = blockIdx.x % kXcds;
+  q.drained = 0;
+  q.first = true;
+  return q;
+}
+
+// Slices of n consecutive items.
+__device__ __forceinline__ uint32_t slice_length(uint32_t n) { return (n + kXcds - 1) / kXcds; }
+__device__ __forceinline__ uint32_t slice_size(uint32_t n) {
+  const uint32_t per = slice_length(n), lo = lane_id() % kXcds * per;
+  return lo >= n ? 0u : (n - lo < per ? n - lo : per);
+}
+
+// The next items [*begin, *end) of slice q.slice, or false when every slice is
+// drained. `late`: the slice is three quarters drained.
+__device__ __forceinline__ bool next_items(SliceTickets& q, uint32_t want, uint32_t* begin,
+                                           uint32_t* end, bool* late) {
+  uint32_t at;
+  if (q.first) {
+    q.first = false;
+    at = blockIdx.x / kXcds * want;
+    const uint32_t m = readlane_u32(q.size, q.slice);
+    if (at < m) {
+      *begin = at;
+      *end = at + (m - at < want ? m - at : want);
+      *late = false;
+      return true;
     }
   }
-  slice = readlane_u32(from, 0);
-  *begin = readlane_u32(b, 0);
-  *end = readlane_u32(e, 0);
+  // Each turn returns, marks a slice drained, or ends.
+  for (uint32_t turn = 0; turn <= 2 * kXcds; turn++) {
+    const uint32_t m = readlane_u32(q.size, q.slice);
+    if (!((q.drained >> q.slice) & 1u) && q.given < m) {
+      uint32_t v = 0;
+      if (lane_id() == 0) v = atomicAdd(q.counters + q.slice * kTicketStride, want);
+      at = q.given + readlane_u32(v, 0);
+      if (at < m) {
+        *begin = at;
+        *end = at + (m - at < want ? m - at : want);
+        *late = at > m / 4 * 3;
+        return true;
+      }
+    }
+    q.drained |= 1u << q.slice;
+    const uint32_t x = lane_id() % kXcds;
+    const bool open = !((q.drained >> x) & 1u) && q.given < q.size;
+    if (!ballot(open)) return false;
+    // Workgroup scope: past the L1, to the XCD's L2.
+    if (lane_id() == 0)
+      __hip_atomic_store(q.flags + q.slice, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    const bool flagged =
+        __hip_atomic_load(q.flags + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0;
+    const uint32_t all = (1u << kXcds) - 1u;
+    q.drained |= (uint32_t)ballot(flagged) & all;
+    const uint32_t mask = (uint32_t)ballot(open && !flagged) & all;
+    if (mask == 0) return false;
+    // The next open slice after this one.
+    const uint32_t turned = ((mask >> q.slice) | (mask << (kXcds - q.slice))) & all;
+    q.slice = (q.slice + (uint32_t)__builtin_ctz(turned)) % kXcds;
+  }
+  return false;
 }
 
 // Level of heap index i, and the leaves below node i: 8^(D - level) of them
@@ -187,6 +238,114 @@ __device__ void oct_walk(const TreeView& t, uint32_t* stack, uint32_t first, uin
     }
     lds_fence();
   }
+}
+
+// Counts queries [first, last) (at most 32), one per octet at a time, as far as
+// they are light: one that holds a whole node of 64 or more leaves, logs more
+// than kOctLog - 8 entries or takes more than kOctSteps steps is left to
+// wide_walk, and its bit (i - first) set in the result. (A query of hundreds of
+// results shows such a node after some six steps, before much is wasted on it.) `commit(done, i, found, n, log)` is called by the whole wave
+// when octets complete queries: `done` and the rest are octet-uniform, `n`
+// entries being in `log`, the octet's, in LDS. It returns (wave-uniform)
+// whether it kept them; if not, they are left to wide_walk as well. Without LOG subtrees inside the
+// query are counted from their live counts and nothing is logged.
+constexpr uint32_t kOctLog = 32;
+constexpr uint32_t kOctSteps = 32;
+
+template <int PRED, bool POINTS, bool LOG, typename Q, typename Src, typename Commit>
+__device__ uint32_t oct_count(const TreeView& t, uint32_t* stack, uint2* log, uint32_t first,
+                              uint32_t last, const Src& src, Commit&& commit) {
+  const uint32_t lane = lane_id(), j = lane & 7u, oct = lane >> 3;
+  uint32_t i = first + oct;
+  bool have = i < last;
+  Q q{}, qn{};
+  if (have) src(i, q);
+  if (i + kFan < last) src(i + kFan, qn);
+  // Octet-uniform:
+  uint32_t sp = have ? 1u : 0u, found = 0, n = 0, steps = 0;
+  bool whole = false;  // octet-uniform: a node of 64 leaves lies inside the query
+  uint32_t heavy = 0;  // wave-uniform
+  if (have && j == 0) stack[0] = 0;
+  lds_fence();
+  while (ballot(have)) {
+    const uint32_t e = have ? stack[sp - 1] : 0u;
+    const uint32_t child = kFan * e + 1u + j;
+    const bool at_leaf = child >= t.leaf0;  // octet-uniform
+    const uint32_t leaf = child - t.leaf0;
+    const bool ok = have && (!at_leaf || leaf < t.n);
+    float4 b = nan_box();
+    if (ok) b = *(at_leaf ? t.leaf_boxes + leaf : t.wide + child);
+    bool hit = false;
+    if (ok) hit = at_leaf ? leaf_test<PRED, POINTS>(t, leaf, b, q) : node_test<PRED, POINTS>(b, q);
+    if (!POINTS) {
+      const bool inside = hit && !at_leaf && inside_test<PRED, POINTS>(b, q);
+      const uint64_t in = ballot(inside);
+      if (in) {
+        // A node whose children are leaves holds at most 8.
+        const uint32_t in8 = (uint32_t)(in >> (8u * oct)) & 0xFFu;
+        whole = in8 && kFan * child + 1u < t.leaf0;
+        uint32_t live = inside ? t.wide_live[child] : 0u;
+        uint32_t rf = 0, rn = 0;
+        bool take = inside && !whole;
+        if (LOG && take) {
+          wide_leaves(t, child, &rf, &rn);
+          take = live == rn;  // otherwise a deleted box lies below: descend
+        }
+        if (take) hit = false;
+        uint32_t add = take ? live : 0u;
+        add += __shfl_xor(add, 1, 64);
+        add += __shfl_xor(add, 2, 64);
+        add += __shfl_xor(add, 4, 64);
+        found += add;
+        if (LOG) {
+          const uint32_t m8 = (uint32_t)(ballot(take) >> (8u * oct)) & 0xFFu;
+          if (take) log[n + (uint32_t)__popc(m8 & ((1u << j) - 1u))] = make_uint2(rf, (1u << rn) - 1u);
+          n += (uint32_t)__popc(m8);
+        }
+      }
+    }
+    const uint64_t hits = ballot(hit);
+    const uint32_t m8 = (uint32_t)(hits >> (8u * oct)) & 0xFFu;
+    if (have) {
+      sp--;
+      steps++;
+    }
+    if (at_leaf) {
+      found += (uint32_t)__popc(m8);
+      if (LOG && m8) {
+        if (j == 0) log[n] = make_uint2(leaf, m8);
+        n++;
+      }
+    } else {
+      if (hit) stack[sp + (uint32_t)__popc(m8 & ((1u << j) - 1u))] = child;
+      sp += (uint32_t)__popc(m8);
+    }
+    const bool done = have && sp == 0 && !whole;
+    const bool leave =
+        have && !done && (whole || (LOG && n + kFan > kOctLog) || steps >= kOctSteps);
+    lds_fence();
+    if (ballot(done || leave)) {
+      const bool kept = commit(done, i, found, n, log);
+      uint64_t lm = ballot((leave || (done && !kept)) && j == 0);
+      while (lm) {
+        const int l = __builtin_ctzll(lm);
+        lm &= lm - 1;
+        heavy |= 1u << (readlane_u32(i, l) - first);
+      }
+      if (done || leave) {
+        i += kFan;
+        have = i < last;
+        q = qn;
+        found = n = steps = 0;
+        whole = false;
+        sp = have ? 1u : 0u;
+        if (have && j == 0) stack[0] = 0;
+        if (i + kFan < last) src(i + kFan, qn);
+      }
+      lds_fence();
+    }
+  }
+  return heavy;
 }
 
 // ----------------------------------------------------------------- wave ----
@@ -314,6 +473,30 @@ __device__ uint64_t wide_walk(const TreeView& t, const Q& q, const uint32_t qid,
   }
   if (LOG) log->logged = nlog;
   return WRITE ? emitted : emitted + wave_sum_u64(inside_live);
+}
+
+// Emits the logged results of up to eight queries, one per octet: octet-uniform
+// n entries (leaf blocks all, oct_count's), the first result at `slot`.
+__device__ __forceinline__ void oct_replay(const TreeView& t, const uint2* entries, uint32_t n,
+                                           rts_pair* out, uint64_t cap, uint64_t slot,
+                                           const uint32_t qid) {
+  const uint32_t j = lane_id() & 7u;
+  for (uint32_t k = 0; k < n; k += 4) {
+    uint2 en[4];
+    uint32_t gid[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++)
+      en[u] = k + u < n ? log_load(entries + k + u) : make_uint2(0u, 0u);
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++)
+      gid[u] = (en[u].y >> j) & 1u ? t.leaf_ids[en[u].x + j] : 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) {
+      const uint64_t at = slot + (uint32_t)__popc(en[u].y & ((1u << j) - 1u));
+      if (((en[u].y >> j) & 1u) && at < cap) store_pair(out + at, gid[u], qid);
+      slot += (uint32_t)__popc(en[u].y);
+    }
+  }
 }
 
 // Emits the logged results of one query and returns their number. Blocks are

@@ -78,3 +78,48 @@ def test_every_box_deleted(n):
     ix.Update((dev(np.arange(3, dtype=np.int64)), dev(new)))
     assert count(ix, P.kWithin, np.float32([[-9, -9, 9, 9]])) == 3
     ix.Sync()
+
+
+@pytest.mark.parametrize("nq", [24_575, 24_576, 131_071, 131_077])
+@pytest.mark.parametrize("heavy", [0.0, 0.02, 0.9])
+def test_light_and_heavy_queries_together(oracle, nq, heavy):
+    # Around the sizes at which octets take the queries first (8, then 16 to a
+    # ticket), with none, few or most of them too heavy for an octet: windows
+    # of thousands of boxes, and thin ones that meet many blocks.
+    log(f"light and heavy queries nq={nq} heavy={heavy}")
+    rng = np.random.default_rng(nq + int(heavy * 100))
+    n = 60_000
+    b = _boxes(rng, n)
+    c = rng.random((nq, 2)).astype(np.float32)
+    h = (rng.random((nq, 2)) * 2.0 / np.sqrt(n)).astype(np.float32)
+    big = rng.random(nq) < heavy
+    if heavy < 0.5:
+        h[big] = (rng.random((int(big.sum()), 2)) * 0.06).astype(np.float32)
+        h[big[:] & (np.arange(nq) % 2 == 0), 1] = 1e-4  # thin
+    else:
+        h[big] = np.float32(0.02)
+    q = np.ascontiguousarray(np.concatenate([c - h, c + h], 1))
+    tree = oracle.RTree(b)
+    ix = make_index(b, traversal=N.RTS_TRAVERSAL_WAVE)
+    for pred in (P.kIntersects, P.kWithin):
+        want = tree.pairs(int(pred), q)
+        assert count(ix, pred, q) == want.shape[0]
+        got, k = collect(ix, pred, q, capacity=want.shape[0] + 1)
+        assert k == want.shape[0] and np.array_equal(got, want)
+    ix.Sync()
+
+
+def test_large_windows_outgrow_their_log(oracle):
+    # Some 5000 partly covered blocks per query: more than a query's log holds.
+    log("windows that outgrow their logs")
+    rng = np.random.default_rng(77)
+    n = 2_000_000
+    b = _boxes(rng, n)
+    b[:, 2:] = b[:, :2]  # points, so that a thin window meets no whole node
+    q = np.float32([[-1, y, 2, y + 0.004] for y in (0.1, 0.35, 0.6, 0.85)] + [[-1, -1, 2, 2]])
+    tree = oracle.RTree(b)
+    ix = make_index(b)
+    want = tree.pairs(oracle.INTERSECTS, q)
+    got, k = collect(ix, P.kIntersects, q, capacity=want.shape[0] + 1)
+    assert k == want.shape[0] and np.array_equal(got, want)
+    ix.Sync()

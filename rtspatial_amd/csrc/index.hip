@@ -657,6 +657,10 @@ struct QueryScratch {
 
 size_t align_up(size_t x) { return (x + 255) & ~size_t(255); }
 
+// Of the sort's four arrays of nq words two are free once it is done: room
+// for the list of heavy queries.
+bool sort_holds_heavy(bool sort, uint64_t nq) { return sort && wave_heavy_words(nq) <= 2 * nq; }
+
 // Carves the scratch of a query call over nq queries. With `ext` (the
 // allocation-free entry point) the block is ext's first ext_bytes bytes, and
 // a call needing more is an error; otherwise it is leased for `stream`.
@@ -672,8 +676,12 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
   if (wave) {
     o_tk = off;
     off = align_up(off + kWaveTicketWords * sizeof(uint32_t));
-    o_heavy = off;
-    off = align_up(off + wave_heavy_words(nq) * sizeof(uint32_t));
+    // An ordered call's list takes the place of the sort's buffers
+    // (order_queries), so that it adds nothing to the largest call's scratch.
+    if (!sort_holds_heavy(sort, nq)) {
+      o_heavy = off;
+      off = align_up(off + wave_heavy_words(nq) * sizeof(uint32_t));
+    }
   }
   if (sort) {
     o_keys = off;
@@ -711,7 +719,7 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
   if (base_out) *base_out = b;
   if (wave) {
     qs->tickets = reinterpret_cast<uint32_t*>(b + o_tk);
-    qs->heavy = reinterpret_cast<uint32_t*>(b + o_heavy);
+    if (!sort_holds_heavy(sort, nq)) qs->heavy = reinterpret_cast<uint32_t*>(b + o_heavy);
   }
   if (two_pass) {
     qs->counts = reinterpret_cast<uint32_t*>(b + o_counts);
@@ -731,10 +739,10 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
 }
 
 // Morton-orders the queries for traversal coherence; the permutation lands in
-// the scratch block.
+// the scratch block. *spare (optional): 2 nq words of it that are free again.
 int order_queries(rts_index* ix, const void* queries, uint64_t nq, bool points, bool f64,
                   char* keys_base, char* sort_base, hipStream_t stream,
-                  const uint32_t** order_out) {
+                  const uint32_t** order_out, uint32_t** spare = nullptr) {
   const size_t words = (size_t)nq;
   uint32_t* keys = reinterpret_cast<uint32_t*>(keys_base);
   uint32_t* vals = keys + words;
@@ -755,6 +763,7 @@ int order_queries(rts_index* ix, const void* queries, uint64_t nq, bool points, 
   RTS_HIP(radix_sort_pairs(keys, vals, keys_b, vals_b, (uint32_t)nq, kMortonBits, true, ss, stream,
                            &in_b));
   *order_out = in_b ? vals_b : vals;
+  if (spare) *spare = in_b ? keys : keys_b;
   return RTS_OK;
 }
 
@@ -835,10 +844,12 @@ int run_plan(rts_index* ix, const Plan& plan, int pred, const void* queries, uin
     if (rc) return rc;
     if (sort) {
       PhaseToken ph = phase_begin(RTS_PHASE_QUERY_ORDER, stream);
+      uint32_t* spare = nullptr;
       rc = order_queries(ix, qp, m, points, f64, base + o_keys, base + o_sort, stream,
-                         &qs.order);
+                         &qs.order, &spare);
       phase_end(ph, stream);
       if (rc) return rc;
+      if (sort_holds_heavy(sort, m)) qs.heavy = spare;
     }
     QueryLaunch ql;
     ql.queries = qp;
@@ -1013,8 +1024,8 @@ namespace {
 
 // Scratch of rts_index_query_static: one array per GPU in the library's device
 // image, held until the process ends. kStaticMaxQueries queries under any plan
-// need at most ~29.2 MiB of it (Morton keys and values 16 MiB, radix-sort
-// status 1 MiB, counts 4 MiB, offsets 8 MiB, scan tiles and tickets); a call
+// need at most ~29.3 MiB of it (Morton keys and values 16 MiB, the sort's digit
+// counts 1 MiB, counts 4 MiB, offsets 8 MiB, scan tiles and tickets); a call
 // that would need more is refused before anything is launched. In host code
 // `scratch` names a host-side stand-in, so kernels are only ever given the
 // device address hipGetSymbolAddress returns for the current device.

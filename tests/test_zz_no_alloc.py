@@ -104,6 +104,24 @@ def test_static_equals_allocating_two_calls(oracle, index, name, pred, kind):
     ix.Sync()
 
 
+@pytest.mark.parametrize("pred", [P.kIntersects, P.kWithin])
+def test_static_takes_its_largest_call(index, pred):
+    """1048576 ordered wavefront queries, collected: the call that needs the
+    most of the static scratch. One query in sixteen is heavy."""
+    ix, boxes, rng, means = index
+    n = 1 << 20
+    q = np.concatenate([W.mixture_boxes(rng, means, n - n // 16, np.log(1e-4)),
+                        W.mixture_boxes(rng, means, n // 16, np.log(1e-3))])
+    dq = dev(q)
+    log(f"static query {pred!r}: {n} queries")
+    want = _count(ix, "alloc", pred, KIND_ENVELOPES, dq)
+    got_a, na = _pairs(ix, "alloc", pred, KIND_ENVELOPES, dq, want + 16)
+    got_s, ns = _pairs(ix, "static", pred, KIND_ENVELOPES, dq, want + 16)
+    assert na == ns == want
+    assert np.array_equal(got_s, got_a)
+    ix.Sync()
+
+
 def test_static_limits_refused(index):
     ix, boxes, rng, means = index
     L = N.lib()

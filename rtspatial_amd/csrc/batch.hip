@@ -153,7 +153,7 @@ __device__ __forceinline__ void run_tile(const TreeView& t, const BatchArgs& a,
       const RangeLog lg = log_for_write(a.log, g);
       const QueueEmit emit{a.arena, a.arena_cap, a.offsets[g]};
       if (lg.n_in != kLogOverflow) {
-        wide_replay(t, lg, local + r.qid_base, emit);
+        wide_replay(t, lg, 0, 0xFFFFFFFFu, local + r.qid_base, emit);
       } else {
         const QueryRT qb{load_query(r.queries, points, local), pred};
         wide_walk<0, false, true, false>(t, qb, local + r.qid_base, emit, lds.wide);
@@ -414,7 +414,7 @@ hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSor
     if (x.none) {
       e = launch_fill_u32(a.counts + x.qbase, 0u, x.ql.n, stream);
     } else {
-      const WaveArgs wa{a.counts + x.qbase, a.offsets + x.qbase, ea.zero, ea.tickets, ea.heavy, {}};
+      const WaveArgs wa{a.counts + x.qbase, a.offsets + x.qbase, ea.zero, nullptr, ea.tickets, ea.heavy, {}};
       e = launch_query_wave(x.ql, wa, kPhaseCount, stream);
     }
     if (e != hipSuccess) return e;
@@ -430,7 +430,7 @@ hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSor
     QueryLaunch ql = x.ql;
     ql.sink.mode = RTS_HANDLER_COLLECT;
     ql.sink.arg = ea.arena_queue;
-    const WaveArgs wa{a.counts + x.qbase, a.offsets + x.qbase, ea.zero, ea.tickets, ea.heavy, {}};
+    const WaveArgs wa{a.counts + x.qbase, a.offsets + x.qbase, ea.zero, nullptr, ea.tickets, ea.heavy, {}};
     const hipError_t e = launch_query_wave(ql, wa, kPhaseWrite, stream);
     if (e != hipSuccess) return e;
   }

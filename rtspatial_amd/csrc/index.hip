@@ -672,7 +672,7 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
   size_t o_log = 0, o_log_off = 0, o_log_n = 0;
   // Range logs: not in a caller's static scratch.
   const bool logs = two_pass && !ext;
-  const uint64_t log_entries = std::min<uint64_t>(nq * kLogPerQuery, kLogMaxEntries);
+  const uint64_t log_entries = std::min<uint64_t>(std::max(nq * kLogPerQuery, std::min(nq * kLogQueryMax, kLogMinEntries)), kLogMaxEntries);
   if (wave) {
     o_tk = off;
     off = align_up(off + kWaveTicketWords * sizeof(uint32_t));
@@ -874,12 +874,12 @@ int run_plan(rts_index* ix, const Plan& plan, int pred, const void* queries, uin
         RTS_HIP(launch_query(ql, stream));
         phase_end(ph, stream);
       } else if (!two_pass) {
-        WaveArgs wa{nullptr, nullptr, nullptr, qs.tickets, qs.heavy, {}};
+        WaveArgs wa{nullptr, nullptr, nullptr, nullptr, qs.tickets, qs.heavy, {}};
         PhaseToken ph = phase_begin(RTS_PHASE_TRAVERSE, stream);
         RTS_HIP(launch_query_wave(ql, wa, staged ? kPhaseWriteStaged : kPhaseCountSink, stream));
         phase_end(ph, stream);
       } else {
-        WaveArgs wa{qs.counts, qs.offsets, qs.total + 1, qs.tickets, qs.heavy, qs.log};
+        WaveArgs wa{qs.counts, qs.offsets, qs.total + 1, qs.total, qs.tickets, qs.heavy, qs.log};
         PhaseToken ph = phase_begin(RTS_PHASE_QUERY_COUNT, stream);
         RTS_HIP(launch_query_wave(ql, wa, kPhaseCount, stream));
         RTS_HIP(launch_exclusive_scan(qs.counts, m, qs.offsets, qs.total, qs.scan_tmp, stream));

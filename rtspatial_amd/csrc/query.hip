@@ -179,16 +179,15 @@ __global__ void __launch_bounds__(kOctThreads)
 // wavefront stages its pairs in LDS and flushes them with one device atomic
 // per kStageWave pairs; a query's pairs may then be split over flushes.
 //
-// Large calls run twice per pass. First the octets of a wave take one query
-// each, kGroup queries per ticket, which answers those of a few leaf blocks
-// eight at a time; the others are listed (one atomic per ticket), and the
-// second launch's waves walk or write them one by one. A wave half of whose
-// queries turn out heavy lists kSkip tickets without trying. 1M within queries
-// of 20 results count in 0.51 and write in 0.31 ms (1.58 and 1.22 ms a wave
-// each; 3.3 and 2.6 ms on the binary tree); on the 10M x 1M join, whose
-// queries are heavy, the trial costs 0.3 of 5 ms. (Having the same wave walk
-// its heavy queries made the join with 200k queries 1.7x slower: sixteen long
-// walks in a row on some waves, none on others.)
+// Large calls count twice. First the octets of a wave take one query each,
+// kGroup queries per ticket, which answers those of a few leaf blocks eight at
+// a time; the others are listed (one atomic per ticket), and the second
+// launch's waves walk them one by one. A wave half of whose queries turn out
+// heavy lists kSkip tickets without trying. 1M within queries of 20 results
+// count in 0.51 ms (1.58 a wave each; 3.3 on the binary tree); on the 10M x 1M
+// join, whose queries are heavy, the trial costs 0.3 of 5 ms. (Having the same
+// wave walk its heavy queries made the join with 200k queries 1.7x slower:
+// sixteen long walks in a row on some waves, none on others.)
 constexpr uint32_t kGroup = 16;
 constexpr uint32_t kSkip = 7;
 constexpr uint32_t kHeavyGroup = 2;
@@ -320,52 +319,14 @@ __global__ void __launch_bounds__(kWave) k_wave_count(const QueryLaunch q, const
   if (!LOG) add_sum(a.tickets, sum);
 }
 
-// The octets' write pass: every query whose log an octet made.
-__global__ void __launch_bounds__(kWave) k_light_write(const QueryLaunch q, const WaveArgs a,
-                                                       const uint32_t group) {
-  const TreeView t = q.tree;
-  const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
-  rts_pair* out = dq->data;
-  const uint64_t cap = dq->capacity;
-  const uint32_t lane = lane_id();
-  SliceTickets tickets =
-      slice_tickets(wave_counters(a.tickets, kTicketsLight), wave_counters(a.tickets, kFlagsLight),
-                    slice_size(q.n), group);
-  const uint32_t per = slice_length(q.n);
-  for (uint32_t it = 0; it <= q.n; it++) {
-    uint32_t lin, end;
-    bool late;
-    if (!next_items(tickets, group, &lin, &end, &late)) break;
-    const uint32_t m = end - lin;  // at most kWave
-    lin += tickets.slice * per;
-    // Lane l: query lin + l.
-    uint32_t qi = 0, n = 0, off = 0;
-    uint64_t slot = 0;
-    if (lane < m) {
-      qi = q.order ? q.order[lin + lane] : lin + lane;
-      n = a.log.n[qi];
-      off = a.log.off[qi];
-      slot = a.base[0] + a.offsets[qi];
-      if (n & kLogWave) n = 0;
-    }
-    if (!ballot(n != 0)) continue;
-    for (uint32_t b = 0; b < m; b += kWave / kFan) {
-      const int l = (int)(b + lane / kFan);
-      const uint32_t ln = (uint32_t)__shfl((int)n, l, 64), lo = (uint32_t)__shfl((int)off, l, 64);
-      const uint32_t lq = (uint32_t)__shfl((int)qi, l, 64);
-      const uint64_t ls = __shfl(slot, l, 64);
-      oct_replay(t, a.log.entries + lo, ln, out, cap, ls, lq + q.qid_base);
-    }
-  }
-}
-
-template <int PRED, bool POINTS, bool F64, bool LISTED>
+// The write pass without logs: every query is walked again.
+template <int PRED, bool POINTS, bool F64>
 __global__ void __launch_bounds__(kWave) k_wave_write(const QueryLaunch q, const WaveArgs a,
                                                       const uint32_t group) {
   __shared__ WideLds s_lds;
   const TreeView t = q.tree;
   const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
-  WaveQueries w = wave_queries<LISTED>(q, a, group);
+  WaveQueries w = wave_queries<false>(q, a, group);
   uint32_t want = group;
   for (uint32_t it = 0; it <= q.n; it++) {
     uint32_t lin, end;
@@ -374,11 +335,100 @@ __global__ void __launch_bounds__(kWave) k_wave_write(const QueryLaunch q, const
     want = late ? 1u : group;
     for (; lin < end; lin++) {
       const uint32_t qi =
-          readlane_u32(wave_query_id<LISTED>(q, a, w.tickets.slice * w.per + lin), 0);
-      const QueueEmit emit{dq->data, dq->capacity, a.base[0] + a.offsets[qi]};
-      const RangeLog lg = log_for_write(a.log, qi);
-      if (lg.n_in != kLogOverflow) {
-        wide_replay(t, lg, qi + q.qid_base, emit);
+          readlane_u32(wave_query_id<false>(q, a, w.tickets.slice * w.per + lin), 0);
+      query_t<PRED, F64> qb;
+      load_q(q.queries, POINTS, qi, qb);
+      wide_walk<PRED, POINTS, true, false>(
+          t, qb, qi + q.qid_base, QueueEmit{dq->data, dq->capacity, a.base[0] + a.offsets[qi]},
+          s_lds);
+    }
+  }
+}
+
+// The write pass from the logs. A wave owns a window of the output, not some
+// queries: query i takes the units [offsets[i] + kWindowCost i, offsets[i + 1]
+// + kWindowCost (i + 1)), its results and kWindowCost more for having been
+// looked at, and every wave an equal share of all units. So a query of 1e5
+// results is written by many waves, each skipping to its share of the log, and
+// 1e5 queries without results are skipped by many too. A query that overflowed
+// its log is walked again by the wave whose window it starts in. Queries that
+// octets logged are written by octets, 8 at a time.
+// Bound by the stores and by latency (log, leaf ids, store). A wave per query,
+// octets per light query, by tickets: 20k queries of 1000 results 188 us, now
+// 80 (160 MB); 1M of 20, 302 and 195; 100 of 1000, 152 and 15. The last two
+// also by the longer logs and the octets' plain stores.
+constexpr uint32_t kWindowCost = 4;
+constexpr uint32_t kWindowMin = 32;
+
+template <int PRED, bool POINTS, bool F64>
+__global__ void __launch_bounds__(kWave) k_window_write(const QueryLaunch q, const WaveArgs a) {
+  __shared__ WideLds s_lds;
+  const TreeView t = q.tree;
+  const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
+  const uint32_t lane = lane_id();
+  const uint64_t units = a.total[0] + (uint64_t)kWindowCost * q.n;
+  uint64_t per = (units + gridDim.x - 1) / gridDim.x;
+  if (per < kWindowMin) per = kWindowMin;
+  // Neighbouring windows on one XCD.
+  const uint64_t m0 = (uint64_t)(blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds) * per;
+  if (m0 >= units) return;
+  const uint64_t m1 = m0 + per;
+  // The last query that starts at m0 or before, 64 probes at a time.
+  uint32_t first = 0, len = q.n;
+  while (len > 1) {
+    const uint32_t step = (len + kWave - 1) / kWave, at = lane * step;
+    const bool before =
+        at < len && a.offsets[first + at] + (uint64_t)kWindowCost * (first + at) <= m0;
+    const uint32_t k = (uint32_t)__popcll(ballot(before)) - 1u;  // query `first` is one
+    first += k * step;
+    len = len - k * step < step ? len - k * step : step;
+  }
+  const uint64_t base = a.base[0], cap = dq->capacity;
+  for (uint32_t b = first; b < q.n; b += kWave) {
+    // Lane l: query b + l and its results [lo, hi) that are this window's.
+    const uint32_t i = b + lane;
+    uint64_t slot = 0, at = ~0ull;
+    if (i < q.n) {
+      slot = a.offsets[i];
+      at = slot + (uint64_t)kWindowCost * i;
+      slot += base;
+    }
+    const bool in = at < m1;
+    if (!ballot(in)) break;
+    uint32_t c = 0, n = 0, off = 0, lo = 0, hi = 0;
+    if (in) {
+      c = a.counts[i];
+      n = a.log.n[i];
+      off = a.log.off[i];
+      lo = at >= m0 ? 0u : (m0 - at < c ? (uint32_t)(m0 - at) : c);
+      hi = m1 - at < c ? (uint32_t)(m1 - at) : c;
+      if (n == kLogOverflow) hi = at >= m0 ? c : 0u;
+    }
+    const bool some = lo < hi;
+    const uint64_t light = ballot(some && !(n & kLogWave));
+    for (uint32_t g = 0; g < (uint32_t)kWave; g += kFan) {
+      if (!((light >> g) & 0xFFu)) continue;
+      const int l = (int)(g + lane / kFan);
+      const uint32_t en = (uint32_t)__shfl((int)n, l, 64), eo = (uint32_t)__shfl((int)off, l, 64);
+      const uint32_t elo = (uint32_t)__shfl((int)lo, l, 64), ehi = (uint32_t)__shfl((int)hi, l, 64);
+      const uint64_t es = __shfl(slot, l, 64);
+      const bool mine = (light >> l) & 1u;
+      oct_replay(t, a.log.entries + eo, mine ? en : 0u, dq->data, cap, es, elo, ehi,
+                 b + (uint32_t)l + q.qid_base);
+    }
+    uint64_t heavy = ballot(some && (n & kLogWave));
+    while (heavy) {
+      const int l = __builtin_ctzll(heavy);
+      heavy &= heavy - 1;
+      const uint32_t qi = b + (uint32_t)l, ln = readlane_u32(n, l);
+      const QueueEmit emit{dq->data, cap,
+                           (uint64_t)readlane_u32((uint32_t)(slot >> 32), l) << 32 |
+                               readlane_u32((uint32_t)slot, l)};
+      if (ln != kLogOverflow) {
+        RangeLog lg;
+        lg.entries = a.log.entries + readlane_u32(off, l);
+        lg.n_in = ln & ~kLogWave;
+        wide_replay(t, lg, readlane_u32(lo, l), readlane_u32(hi, l), qi + q.qid_base, emit);
       } else {
         query_t<PRED, F64> qb;
         load_q(q.queries, POINTS, qi, qb);
@@ -543,22 +593,22 @@ hipError_t launch_wave_f(const QueryLaunch& q, const WaveArgs& a, int phase, hip
       return hipErrorInvalidValue;
     }
     default: {
-      auto* all = &k_wave_write<PRED, POINTS, F64, false>;
-      auto* listed = &k_wave_write<PRED, POINTS, F64, true>;
-      static const uint32_t r_all = resident_waves(all), r_listed = resident_waves(listed),
-                            r_light = resident_waves(&k_light_write);
-      // The count pass's tickets are taken: new ones, but its list of heavy
-      // queries stays.
-      const uint32_t group = octet_group(q.n);
-      hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, stream, a.tickets,
-                         kHeavyCount * kXcds);
-      if (!group || !a.log.entries) {
-        const uint32_t few = std::max(1u, std::min(kFewQueries, (q.n + r_all - 1) / r_all));
-        launch_persistent(all, r_all, few, q, a, 0, 0, stream);
-      } else {
-        launch_persistent(&k_light_write, r_light, group, q, a, 0, 0, stream);
-        launch_persistent(listed, r_listed, kHeavyGroup, q, a, 0, 0, stream);
+      if (a.log.entries) {
+        auto* k = &k_window_write<PRED, POINTS, F64>;
+        static const uint32_t resident = resident_waves(k);
+        uint32_t blocks = q.n < resident ? std::min(resident, 512 + 4 * q.n) : resident;
+        blocks = (blocks + kXcds - 1) / kXcds * kXcds;
+        hipLaunchKernelGGL(k, dim3(blocks), dim3(kWave), 0, stream, q, a);
+        break;
       }
+      auto* k = &k_wave_write<PRED, POINTS, F64>;
+      static const uint32_t resident = resident_waves(k);
+      // The count pass's tickets are taken: new ones.
+      hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(256), 0, stream, a.tickets,
+                         kTicketKinds * kXcds);
+      launch_persistent(k, resident,
+                        std::max(1u, std::min(kFewQueries, (q.n + resident - 1) / resident)), q, a,
+                        0, 0, stream);
       break;
     }
   }

@@ -20,7 +20,6 @@
 
 namespace rts {
 
-constexpr uint32_t kLogQueryMax = 4096;
 constexpr uint32_t kLogOverflow = 0xFFFFFFFFu;
 constexpr uint32_t kLogRange = 0x80000000u;
 // A header's entry count carries this bit when a wave walked the query (its log

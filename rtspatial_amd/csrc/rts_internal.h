@@ -169,9 +169,14 @@ struct RangeLogArgs {
   uint32_t* off = nullptr;   // per query: first entry
   uint32_t* n = nullptr;     // per query: entries, or kLogOverflow
 };
-// Range-log entries (8 bytes each) of a two-pass query call: 512 per query,
-// at most 2^29 (4 GiB).
+// Range-log entries (8 bytes each) of a two-pass query call: 512 per query, at
+// most 2^29 (4 GiB); in calls of up to 32768 queries, whose waves have few
+// queries to even out long logs, up to kLogQueryMax per query but at most 2^24
+// (128 MiB). With 512 the waves of 10k double queries of 1000 results walked
+// the longest again: 0.23 ms for the write pass, 0.05 with 1600.
+constexpr uint32_t kLogQueryMax = 4096;  // longest log of a query
 constexpr uint64_t kLogPerQuery = 512;
+constexpr uint64_t kLogMinEntries = 1ull << 24;
 constexpr uint64_t kLogMaxEntries = 1ull << 29;
 
 // Counters of wave calls, on lines of 256 bytes: per kind one for each XCD (a
@@ -185,9 +190,10 @@ struct WaveArgs {
   uint32_t* counts;
   const uint64_t* offsets;
   const uint64_t* base;
-  uint32_t* tickets;  // kWaveTicketWords words
-  uint32_t* heavy;    // queries the octets left to the waves (room for wave_heavy_words(n))
-  RangeLogArgs log;   // two-pass calls: the count walks' range logs
+  const uint64_t* total;  // sum of the counts
+  uint32_t* tickets;      // kWaveTicketWords words
+  uint32_t* heavy;        // queries the octets left to the waves (wave_heavy_words(n) words)
+  RangeLogArgs log;       // two-pass calls: the count walks' range logs
 };
 inline uint64_t wave_heavy_words(uint64_t n) { return n + kTicketXcds; }
 // Wave-per-query traversal. phase 0: per-query counts -> a.counts;

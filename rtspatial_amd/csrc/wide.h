@@ -475,12 +475,15 @@ __device__ uint64_t wide_walk(const TreeView& t, const Q& q, const uint32_t qid,
   return WRITE ? emitted : emitted + wave_sum_u64(inside_live);
 }
 
-// Emits the logged results of up to eight queries, one per octet: octet-uniform
-// n entries (leaf blocks all, oct_count's), the first result at `slot`.
+// Emits the logged results [lo, hi) of up to eight queries, one per octet: all
+// octet-uniform, n entries (leaf blocks all, oct_count's), result 0 at `slot`.
+// Ordinary stores: an octet's three pairs or so are part of a line, which the
+// L2 puts together (1M queries of 20 results: 0.19 ms, 0.29 with store_pair).
 __device__ __forceinline__ void oct_replay(const TreeView& t, const uint2* entries, uint32_t n,
-                                           rts_pair* out, uint64_t cap, uint64_t slot,
-                                           const uint32_t qid) {
+                                           rts_pair* out, uint64_t cap, uint64_t slot, uint32_t lo,
+                                           uint32_t hi, const uint32_t qid) {
   const uint32_t j = lane_id() & 7u;
+  uint32_t first = 0;  // result of the next entry
   for (uint32_t k = 0; k < n; k += 4) {
     uint2 en[4];
     uint32_t gid[4];
@@ -492,29 +495,36 @@ __device__ __forceinline__ void oct_replay(const TreeView& t, const uint2* entri
       gid[u] = (en[u].y >> j) & 1u ? t.leaf_ids[en[u].x + j] : 0u;
 #pragma unroll
     for (uint32_t u = 0; u < 4; u++) {
-      const uint64_t at = slot + (uint32_t)__popc(en[u].y & ((1u << j) - 1u));
-      if (((en[u].y >> j) & 1u) && at < cap) store_pair(out + at, gid[u], qid);
-      slot += (uint32_t)__popc(en[u].y);
+      const uint32_t r = first + (uint32_t)__popc(en[u].y & ((1u << j) - 1u));
+      if (((en[u].y >> j) & 1u) && r >= lo && r < hi && slot + r < cap)
+        out[slot + r] = rts_pair{gid[u], qid};
+      first += (uint32_t)__popc(en[u].y);
     }
   }
 }
 
-// Emits the logged results of one query and returns their number. Blocks are
-// taken 8 at a time, one per octet: each lane stores the result its mask bit
-// names, and the wave's stores of a round are consecutive pairs. Runs of
-// leaves are copied 64 (4 x 64 while they last) at a time.
+// Emits the logged results [lo, hi) of one query. Blocks are taken 8 at a time,
+// one per octet: each lane stores the result its mask bit names, and the
+// wave's stores of a round are consecutive pairs. Runs of leaves are copied 64
+// (4 x 64 while they last) at a time. The next 64 entries are in flight while
+// these are emitted.
 template <typename Emit>
-__device__ uint64_t wide_replay(const TreeView& t, const RangeLog& lg, const uint32_t qid,
-                                const Emit& emit) {
+__device__ void wide_replay(const TreeView& t, const RangeLog& lg, uint32_t lo, uint32_t hi,
+                            const uint32_t qid, const Emit& emit) {
   const uint32_t lane = lane_id(), j = lane & 7u, oct = lane >> 3;
-  uint64_t emitted = 0;  // wave-uniform
-  for (uint32_t b0 = 0; b0 < lg.n_in; b0 += kWave) {
+  uint32_t first = 0;  // wave-uniform: result of the next entry
+  uint2 next = lane < lg.n_in ? log_load(lg.entries + lane) : make_uint2(0u, 0u);
+  for (uint32_t b0 = 0; b0 < lg.n_in && first < hi; b0 += kWave) {
     const uint32_t m = lg.n_in - b0 < (uint32_t)kWave ? lg.n_in - b0 : (uint32_t)kWave;
-    const uint2 en = lane < m ? log_load(lg.entries + b0 + lane) : make_uint2(0u, 0u);
+    const uint2 en = next;
+    next = b0 + kWave + lane < lg.n_in ? log_load(lg.entries + b0 + kWave + lane)
+                                       : make_uint2(0u, 0u);
     const bool run = en.x & kLogRange;
     const uint32_t cnt = run ? en.y : (uint32_t)__popc(en.y);
     const uint32_t inc = wave_inclusive_sum(cnt);
-    const uint32_t off = inc - cnt;
+    const uint32_t off = first + inc - cnt;
+    first += readlane_u32(inc, kWave - 1);
+    if (first <= lo) continue;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       if ((uint32_t)(h * 32) >= m) break;
@@ -526,21 +536,22 @@ __device__ uint64_t wide_replay(const TreeView& t, const RangeLog& lg, const uin
         const uint32_t x = (uint32_t)__shfl((int)en.x, s, 64);
         const uint32_t y = (uint32_t)__shfl((int)en.y, s, 64);
         at[r] = (uint32_t)__shfl((int)off, s, 64) + (uint32_t)__popc(y & ((1u << j) - 1u));
-        const bool hit = !(x & kLogRange) && ((y >> j) & 1u);
+        const bool hit = !(x & kLogRange) && ((y >> j) & 1u) && at[r] >= lo && at[r] < hi;
         hm |= (hit ? 1u : 0u) << r;
         gid[r] = hit ? t.leaf_ids[x + j] : 0u;
       }
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        if ((hm >> r) & 1u) emit(emitted + at[r], gid[r], qid);
+        if ((hm >> r) & 1u) emit(at[r], gid[r], qid);
     }
-    uint64_t rm = ballot(run);
+    uint64_t rm = ballot(run && off < hi && off + cnt > lo);
     while (rm) {
       const int l = __builtin_ctzll(rm);
       rm &= rm - 1;
-      const uint32_t f = readlane_u32(en.x, l) & ~kLogRange, n = readlane_u32(en.y, l);
-      const uint64_t at = emitted + readlane_u32(off, l);
-      uint32_t k = 0;
+      const uint32_t f = readlane_u32(en.x, l) & ~kLogRange, at = readlane_u32(off, l);
+      const uint32_t c = readlane_u32(cnt, l);
+      uint32_t k = lo > at ? lo - at : 0u;
+      const uint32_t n = hi - at < c ? hi - at : c;
       for (; k + 4 * kWave <= n; k += 4 * kWave) {
         uint32_t gid[4];
 #pragma unroll
@@ -551,9 +562,7 @@ __device__ uint64_t wide_replay(const TreeView& t, const RangeLog& lg, const uin
       for (; k < n; k += kWave)
         if (k + lane < n) emit(at + k + lane, t.leaf_ids[f + k + lane], qid);
     }
-    emitted += readlane_u32(inc, kWave - 1);
   }
-  return emitted;
 }
 
 }  // namespace rts

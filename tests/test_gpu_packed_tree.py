@@ -13,7 +13,7 @@ if not torch.cuda.is_available():
 
 import rtspatial_amd as R  # noqa: E402
 from rtspatial_amd import _native as N  # noqa: E402
-from gpu_util import collect, count, dev, log, make_index  # noqa: E402
+from gpu_util import canon, collect, count, dev, log, make_index  # noqa: E402
 
 P = R.Predicate
 SIZES = [1, 2, 7, 8, 9, 63, 64, 65, 511, 512, 513, 4095, 4096, 4097, 32767, 32769, 262145]
@@ -122,4 +122,40 @@ def test_large_windows_outgrow_their_log(oracle):
     want = tree.pairs(oracle.INTERSECTS, q)
     got, k = collect(ix, P.kIntersects, q, capacity=want.shape[0] + 1)
     assert k == want.shape[0] and np.array_equal(got, want)
+    ix.Sync()
+
+
+@pytest.mark.parametrize("nq,giants", [(1, [0]), (5, [4]), (3000, [0, 1499, 1500, 2999]),
+                                       (40_000, [7, 39_999]), (40_000, [])])
+def test_write_windows(oracle, nq, giants):
+    # Waves write windows of the output: queries of 1e5 results that take many
+    # windows, long stretches of queries without results, and the rest of a few
+    # results; each query's pairs together, in query order; into a queue with
+    # room for all and for some.
+    log(f"write windows nq={nq} giants={giants}")
+    rng = np.random.default_rng(nq)
+    n = 120_000
+    b = _boxes(rng, n)
+    c = rng.random((nq, 2)).astype(np.float32)
+    c[nq // 3: nq // 2] += 5  # off the boxes
+    h = np.full((nq, 2), 1.5 / np.sqrt(n), np.float32)
+    h[giants] = 0.45
+    c[giants] = 0.5
+    q = np.ascontiguousarray(np.concatenate([c - h, c + h], 1))
+    want = oracle.RTree(b).pairs(oracle.INTERSECTS, q)
+    ix = make_index(b)
+    queue = R.Queue(want.shape[0] + 8)
+    ix.Query(P.kIntersects, dev(q), queue)
+    assert queue.size() == want.shape[0]
+    assert np.array_equal(canon(queue.pairs()), want)
+    ids = queue.pairs()[:, 1].cpu().numpy()
+    assert (np.diff(ids.astype(np.int64)) >= 0).all()
+    some = R.Queue(want.shape[0] // 2 + 1)
+    ix.Query(P.kIntersects, dev(q), some)
+    assert some.size() == want.shape[0]
+    # The slots of the first half of the results, each written once.
+    assert np.array_equal(some.pairs()[:, 1].cpu().numpy(), ids[:some.capacity()])
+    a, b = canon(some.pairs()).astype(np.uint64), want.astype(np.uint64)
+    a, b = a[:, 0] << np.uint64(32) | a[:, 1], b[:, 0] << np.uint64(32) | b[:, 1]
+    assert np.unique(a).size == a.size and np.isin(a, b).all()
     ix.Sync()

@@ -14,10 +14,10 @@
 //
 // Two passes: the count pass writes each query's number of results and logs a
 // wave tile's (range_log.h), a scan turns the numbers into exclusive offsets
-// into the slot's result arena, and the write pass emits the logged results
-// (a lane tile's walk is cheap and taken again) at the query's offset. Per
-// request, the batch reports its first slot and its results. Every launch reads
-// the batch's sizes from device memory.
+// into the slot's result arena, and the write pass emits the logged results by
+// windows of the arena (write_window), whatever their queries, and walks the
+// lane tiles again (cheap). Per request, the batch reports its first slot and
+// its results. Every launch reads the batch's sizes from device memory.
 #include <algorithm>
 
 #include "batch.h"
@@ -46,24 +46,25 @@ __device__ __forceinline__ uint32_t find_request(const BatchRequest* reqs, uint3
 
 // Tile slices: class c's tiles [lo_c, hi_c) are cut into kXcds contiguous
 // slices, one counter each. Wave w on XCD x first drains its own XCD's slices
-// class by class (heaviest first: neighbouring Morton-ordered queries then
-// share that XCD's L2), then steals, heaviest class first, from the other
-// XCDs. Counters only grow, so a slice found drained stays drained: `pos`
-// (wave-uniform) walks the 5 x 8 slice positions of this wave's order once.
-constexpr uint32_t kSlicePositions = kClasses * kXcds;
-
+// class by class from class FIRST on (heaviest first: neighbouring
+// Morton-ordered queries then share that XCD's L2), then steals, heaviest class
+// first, from the other XCDs. Counters only grow, so a slice found drained stays
+// drained: `pos` (wave-uniform) walks the slice positions of this wave's order
+// once.
+template <int FIRST>
 __device__ __forceinline__ uint32_t grab_tile(uint32_t* counters, const uint32_t* class_end,
                                               uint32_t xcd, uint32_t& pos) {
+  constexpr uint32_t kTaken = kClasses - FIRST, kSlicePositions = kTaken * kXcds;
   uint32_t got = 0xFFFFFFFFu, at = kSlicePositions;
   if (lane_id() == 0) {
     for (uint32_t p = pos; p < kSlicePositions; p++) {
       uint32_t c, x;
-      if (p < kClasses) {
-        c = p;
+      if (p < kTaken) {
+        c = FIRST + p;
         x = xcd;
       } else {
-        c = (p - kClasses) / (kXcds - 1);
-        x = (xcd + 1 + (p - kClasses) % (kXcds - 1)) % kXcds;
+        c = FIRST + (p - kTaken) / (kXcds - 1);
+        x = (xcd + 1 + (p - kTaken) % (kXcds - 1)) % kXcds;
       }
       const uint32_t lo = c == 0 ? 0u : class_end[c - 1];
       const uint32_t n = class_end[c] - lo;
@@ -88,9 +89,6 @@ union TileLds {
   uint32_t oct[kWave / kFan][kOctStack];
 };
 
-// One tile of the batch: a wave tile's one query (by the whole wave) or a
-// lane tile's 64 queries. With skip_giants a wave tile whose query is on a
-// giant list is left to that list.
 // Queries and results of a lane tile's octet walk.
 struct TileSource {
   const void* queries;
@@ -108,6 +106,11 @@ struct TileCount {
     if ((lane_id() & 7u) == 0) counts[i] = found;
   }
 };
+// A request whose results run past the arena is launched again: its pairs would
+// be dropped.
+__device__ __forceinline__ bool past_arena(const BatchArgs& a, uint32_t ri) {
+  return a.ranges[2 * ri] + a.ranges[2 * ri + 1] > a.arena_cap;
+}
 struct TileWrite {
   const uint64_t* offsets;
   rts_pair* arena;
@@ -121,74 +124,66 @@ struct TileWrite {
   __device__ void finish(uint32_t, uint32_t) const {}
 };
 
-template <bool WRITE>
-__device__ __forceinline__ void run_tile(const TreeView& t, const BatchArgs& a,
-                                         const BatchHeader& h, uint32_t tile, bool skip_giants,
-                                         LogCursor& lc, TileLds& lds) {
-  const uint32_t ri = find_request(a.requests, h.n_requests, tile);
-  const BatchRequest r = a.requests[ri];
+__device__ __forceinline__ int request_pred(const BatchRequest& r) {
+  return r.flags & kReqPoints ? (int)RTS_CONTAINS : (int)((r.flags >> kReqPredShift) & 3u);
+}
+
+// Counts one tile of the batch: a wave tile's one query (by the whole wave) or
+// a lane tile's 64 queries.
+__device__ __forceinline__ void count_tile(const TreeView& t, const BatchArgs& a,
+                                           const BatchHeader& h, uint32_t tile, LogCursor& lc,
+                                           TileLds& lds) {
+  const BatchRequest r = a.requests[find_request(a.requests, h.n_requests, tile)];
   const uint32_t local = tile - r.tbase;
-  const bool wave = r.flags & kReqWaveTiles;
-  if (WRITE && skip_giants && wave && local < r.n &&
-      a.counts[r.qbase + local] >= giant_min(kGiantBuckets - 1))
-    return;
-  // A request whose results run past the arena is launched again: its pairs
-  // would be dropped.
-  if (WRITE && a.ranges[2 * ri] + a.ranges[2 * ri + 1] > a.arena_cap) return;
+  const bool wave = r.flags & kReqWaveTiles, points = r.flags & kReqPoints;
   if (t.n == 0) {
-    if (wave) {
-      if (local < r.n && lane_id() == 0) a.counts[r.qbase + local] = 0;
-    } else {
-      const uint32_t q = local * kWave + lane_id();
-      if (q < r.n) a.counts[r.qbase + q] = 0;
-    }
+    // An empty index (no boxes inserted, or cleared) has no tree: zero results.
+    const uint32_t q = wave ? local : local * kWave + lane_id();
+    if (q < r.n && (!wave || lane_id() == 0)) a.counts[r.qbase + q] = 0;
     return;
   }
-  const bool points = r.flags & kReqPoints;
-  const int pred = points ? (int)RTS_CONTAINS : (int)((r.flags >> kReqPredShift) & 3u);
   if (wave) {
     if (local >= r.n) return;
     const uint64_t g = r.qbase + local;
-    if (WRITE) {
-      const RangeLog lg = log_for_write(a.log, g);
-      const QueueEmit emit{a.arena, a.arena_cap, a.offsets[g]};
-      if (lg.n_in != kLogOverflow) {
-        wide_replay(t, lg, 0, 0xFFFFFFFFu, local + r.qid_base, emit);
-      } else {
-        const QueryRT qb{load_query(r.queries, points, local), pred};
-        wide_walk<0, false, true, false>(t, qb, local + r.qid_base, emit, lds.wide);
-      }
-    } else {
-      const QueryRT qb{load_query(r.queries, points, local), pred};
-      RangeLog lg = log_for_count(lc);
-      const uint64_t c = wide_walk<0, false, false, true>(t, qb, local, NoEmit{}, lds.wide, &lg);
-      log_commit(lc, a.log, g, lg);
-      if (lane_id() == 0) {
-        a.counts[g] = (uint32_t)c;
-        // Giants are listed as they are counted (rare: one atomic each).
-        if (a.giants && c >= giant_min(kGiantBuckets - 1)) {
-          int b = kGiantBuckets - 1;
-          while (b > 0 && c >= giant_min(b - 1)) b--;
-          const uint32_t at =
-              atomicAdd(&a.tile_counters[kGiantCounterOff + 2 * b * kCounterStride], 1u);
-          if (at < a.giant_cap) a.giants[(uint64_t)b * a.giant_cap + at] = tile;
-        }
-      }
-    }
+    const QueryRT qb{load_query(r.queries, points, local), request_pred(r)};
+    RangeLog lg = log_for_count(lc);
+    const uint64_t c = wide_walk<0, false, false, true>(t, qb, local, NoEmit{}, lds.wide, &lg);
+    log_commit(lc, a.log, g, lg);
+    if (lane_id() == 0) a.counts[g] = (uint32_t)c;
   } else {
     const uint32_t first = local * kWave;
     if (first >= r.n) return;
     const uint32_t last = first + kWave < r.n ? first + kWave : r.n;
-    const TileSource src{r.queries, points, pred};
-    uint32_t* stack = lds.oct[lane_id() / kFan];
-    if (WRITE) {
-      TileWrite sink{a.offsets + r.qbase, a.arena, a.arena_cap, r.qid_base};
-      oct_walk<0, false, false, QueryRT>(t, stack, first, last, src, sink);
-    } else {
-      TileCount sink{a.counts + r.qbase};
-      oct_walk<0, false, true, QueryRT>(t, stack, first, last, src, sink);
-    }
+    TileCount sink{a.counts + r.qbase};
+    oct_walk<0, false, true, QueryRT>(t, lds.oct[lane_id() / kFan], first, last,
+                                      TileSource{r.queries, points, request_pred(r)}, sink);
   }
+}
+
+// Writes one lane tile.
+__device__ __forceinline__ void write_tile(const TreeView& t, const BatchArgs& a,
+                                           const BatchHeader& h, uint32_t tile, TileLds& lds) {
+  const uint32_t ri = find_request(a.requests, h.n_requests, tile);
+  const BatchRequest r = a.requests[ri];
+  const uint32_t first = (tile - r.tbase) * kWave;
+  if ((r.flags & kReqWaveTiles) || first >= r.n || past_arena(a, ri)) return;
+  const uint32_t last = first + kWave < r.n ? first + kWave : r.n;
+  TileWrite sink{a.offsets + r.qbase, a.arena, a.arena_cap, r.qid_base};
+  oct_walk<0, false, false, QueryRT>(
+      t, lds.oct[lane_id() / kFan], first, last,
+      TileSource{r.queries, (r.flags & kReqPoints) != 0, request_pred(r)}, sink);
+}
+
+// The request of global query i: the last of the n that starts at i or before
+// (earlier ones that start there too are empty).
+__device__ __forceinline__ uint32_t request_of_query(const BatchRequest* reqs, uint32_t n,
+                                                     uint64_t i) {
+  uint32_t lo = 0, end = n;
+  while (end - lo > 1) {
+    const uint32_t mid = (lo + end) >> 1;
+    if (reqs[mid].qbase <= i) lo = mid; else end = mid;
+  }
+  return lo;
 }
 
 // One kernel per pass answers every tile of the batch. A request's predicate
@@ -196,57 +191,59 @@ __device__ __forceinline__ void run_tile(const TreeView& t, const BatchArgs& a,
 // walk and one lane walk. The tree view is read from device memory so that
 // the launch does not depend on the index's state. One wavefront per
 // workgroup: a workgroup's slot is freed as soon as its one wave runs out of
-// tiles (four-wave workgroups held theirs until the slowest wave ended). The
-// write pass first takes the giant tiles, largest bucket first.
-template <bool WRITE>
-__global__ void __launch_bounds__(kWave) k_batch(const TreeView* tv, const BatchArgs a) {
+// work (four-wave workgroups held theirs until the slowest wave ended).
+__global__ void __launch_bounds__(kWave) k_batch_count(const TreeView* tv, const BatchArgs a) {
   __shared__ TileLds s_lds;
   const TreeView t = *tv;
   const BatchHeader h = *a.header;
   if (h.n_tiles == 0 || h.n_requests == 0) return;
-  // An empty index (no boxes inserted, or cleared) has no tree: the count
-  // pass still writes every query's count (zero), the write pass has nothing
-  // to write.
-  if (WRITE && t.n == 0) return;
-  uint32_t* counters = a.tile_counters + (WRITE ? kClasses * kXcds * kCounterStride : 0u);
-  const uint32_t xcd = blockIdx.x % kXcds;
   const uint32_t wave_end = h.class_end[kClassWavePoints];
-  // The giant lists are used only when every one of them held its tiles
-  // (a batch never has more wave tiles than the lists' capacity).
-  uint32_t* gc = a.tile_counters + kGiantCounterOff;
-  bool giants = false;
-  if (WRITE && a.giants) {
-    giants = true;
-    for (int b = 0; b < kGiantBuckets; b++) giants &= gc[2 * b * kCounterStride] <= a.giant_cap;
-  }
-  int bucket = giants ? 0 : kGiantBuckets;  // wave-uniform: list being drained
-  LogCursor lc = WRITE ? LogCursor{} : log_cursor(a.log);
+  LogCursor lc = log_cursor(a.log);
   uint32_t pos = 0;
-  // Every iteration takes a tile, from a list or the queue, or finds none
-  // left; listed tiles are wave tiles, so 2 * n_tiles + 1 iterations bound
-  // the loop.
-  for (uint64_t it = 0; it <= 2ull * h.n_tiles; it++) {
-    uint32_t tile = 0xFFFFFFFFu;
-    for (; bucket < kGiantBuckets; bucket++) {
-      uint32_t k = 0;
-      if (lane_id() == 0) k = atomicAdd(&gc[(2 * bucket + 1) * kCounterStride], 1u);
-      k = readlane_u32(k, 0);
-      if (k < gc[2 * bucket * kCounterStride]) {
-        tile = a.giants[(uint64_t)bucket * a.giant_cap + k];
-        break;
-      }
-    }
-    const bool listed = tile != 0xFFFFFFFFu;
-    if (!listed) {
-      // class_end from device memory: indexing the local copy by a run-time
-      // class would put that copy in private memory.
-      tile = grab_tile(counters, a.header->class_end, xcd, pos);
-      if (tile >= h.n_tiles) break;
-      // Wave tiles are Morton-ordered within their class (the sort keys
-      // lead with the class).
-      if (a.order && tile < wave_end) tile = a.order[tile];
-    }
-    run_tile<WRITE>(t, a, h, tile, giants && !listed, lc, s_lds);
+  // Every iteration takes a tile or finds none left.
+  for (uint32_t it = 0; it <= h.n_tiles; it++) {
+    // class_end from device memory: indexing the local copy by a run-time
+    // class would put that copy in private memory.
+    uint32_t tile = grab_tile<0>(a.tile_counters, a.header->class_end, blockIdx.x % kXcds, pos);
+    if (tile >= h.n_tiles) break;
+    // Wave tiles are Morton-ordered within their class (the sort keys lead
+    // with the class).
+    if (a.order && tile < wave_end) tile = a.order[tile];
+    count_tile(t, a, h, tile, lc, s_lds);
+  }
+}
+
+// A wave's window of the wave tiles' results, then lane tiles. (With a wave to
+// a query, the largest first from lists, a batch of 40M pairs was written in
+// 0.71 ms: a query of 1e5 results held its wave past the others' end. Now 0.20.)
+__global__ void __launch_bounds__(kWave) k_batch_write(const TreeView* tv, const BatchArgs a) {
+  __shared__ TileLds s_lds;
+  const TreeView t = *tv;
+  const BatchHeader h = *a.header;
+  if (h.n_tiles == 0 || h.n_requests == 0 || t.n == 0) return;
+  const Windows w{a.offsets,   a.counts, a.log,      a.arena,
+                  a.arena_cap, 0,        a.total[0], (uint32_t)h.n_queries};
+  write_window(
+      t, w,
+      [&](uint32_t i, uint32_t* qid) {
+        const uint32_t ri = request_of_query(a.requests, h.n_requests, i);
+        const BatchRequest r = a.requests[ri];
+        *qid = i - (uint32_t)r.qbase + r.qid_base;
+        return !(r.flags & kReqExt) && (r.flags & kReqWaveTiles) && !past_arena(a, ri);
+      },
+      [&](uint32_t i, uint32_t qid, const QueueEmit& emit) {
+        const BatchRequest r = a.requests[request_of_query(a.requests, h.n_requests, i)];
+        const QueryRT qb{load_query(r.queries, r.flags & kReqPoints, i - (uint32_t)r.qbase),
+                         request_pred(r)};
+        wide_walk<0, false, true, false>(t, qb, qid, emit, s_lds.wide);
+      });
+  uint32_t* counters = a.tile_counters + kClasses * kXcds * kCounterStride;
+  uint32_t pos = 0;
+  for (uint32_t it = 0; it <= h.n_tiles; it++) {
+    const uint32_t tile =
+        grab_tile<kClassLane>(counters, a.header->class_end, blockIdx.x % kXcds, pos);
+    if (tile >= h.n_tiles) break;
+    write_tile(t, a, h, tile, s_lds);
   }
 }
 
@@ -330,8 +327,9 @@ __global__ void __launch_bounds__(kThreads) k_request_ranges(const BatchArgs a) 
   }
 }
 
-__global__ void k_zero_u32(uint32_t* p, uint32_t n) {
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
+__global__ void __launch_bounds__(kThreads) k_clear_counters(uint32_t* p) {
+  for (uint32_t i = threadIdx.x; i < kTileCounterWords / kCounterStride; i += kThreads)
+    p[i * kCounterStride] = 0;
 }
 
 }  // namespace
@@ -349,12 +347,15 @@ uint32_t persistent_blocks(K kernel, int threads) {
   return (blocks + kXcds - 1) / kXcds * kXcds;
 }
 
-template <bool WRITE>
-void launch_batch_kernel(const TreeView* t, const BatchArgs& a_in, hipStream_t stream) {
-  static const uint32_t blocks = persistent_blocks(k_batch<WRITE>, kWave);
+void launch_batch_count(const TreeView* t, const BatchArgs& a_in, hipStream_t stream) {
+  static const uint32_t blocks = persistent_blocks(k_batch_count, kWave);
   BatchArgs a = a_in;
   a.log.per_wave = (uint32_t)(a.log.n_entries / blocks);
-  hipLaunchKernelGGL((k_batch<WRITE>), dim3(blocks), dim3(kWave), 0, stream, t, a);
+  hipLaunchKernelGGL(k_batch_count, dim3(blocks), dim3(kWave), 0, stream, t, a);
+}
+void launch_batch_write(const TreeView* t, const BatchArgs& a, hipStream_t stream) {
+  static const uint32_t blocks = persistent_blocks(k_batch_write, kWave);
+  hipLaunchKernelGGL(k_batch_write, dim3(blocks), dim3(kWave), 0, stream, t, a);
 }
 
 // Sort keys of the wave tiles [0, n): class in the top 2 bits (the wave
@@ -403,9 +404,8 @@ hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSor
   (void)hipStreamIsCapturing(stream, &cap);
   const bool timed = cap == hipStreamCaptureStatusNone;
   PhaseToken ph = timed ? phase_begin(RTS_PHASE_BATCH_COUNT, stream) : PhaseToken{-1, nullptr};
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, stream, a.tile_counters,
-                     kTileCounterWords);
-  launch_batch_kernel<false>(t, a, stream);
+  hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(kThreads), 0, stream, a.tile_counters);
+  launch_batch_count(t, a, stream);
   // Requests the batch kernel does not walk: one count launch each, into the
   // same counts (so the scan below covers them).
   for (size_t i = 0; i < n_ext; i++) {
@@ -423,7 +423,7 @@ hipError_t launch_batch(const TreeView* t, const BatchArgs& a_in, const BatchSor
   hipLaunchKernelGGL(k_request_ranges, dim3(16), dim3(kThreads), 0, stream, a);
   phase_end(ph, stream);
   ph = timed ? phase_begin(RTS_PHASE_BATCH_WRITE, stream) : PhaseToken{-1, nullptr};
-  launch_batch_kernel<true>(t, a, stream);
+  launch_batch_write(t, a, stream);
   for (size_t i = 0; i < n_ext; i++) {
     const BatchExt& x = ext[i];
     if (x.none) continue;
@@ -443,22 +443,28 @@ size_t batch_seg_sums_words() { return kScanBlocks; }
 namespace {
 
 // hashes[r] += pair_hash over request r's pairs, arena[start, start + results).
-// A wavefront takes blocks of kHashBlock consecutive slots and goes through the
-// requests that have pairs there; each costs it one atomic. (Finding each
-// slot's query as well, when a query's slots were a bound on its results, took
-// 3.2 ms per batch of 64 served requests, 40M pairs.)
-constexpr uint32_t kHashBlock = kWave * 256;
+// A workgroup takes a block of kHashBlock consecutive slots, a wave a quarter of
+// it, and goes through the requests that have pairs there; each costs the block
+// one atomic (14 ns each, as the hashes share lines). (Finding each slot's query
+// as well, when a query's slots were a bound on its results, took 3.2 ms per
+// batch of 64 served requests, 40M pairs. A wave to 16384 slots, one load in
+// flight, took 0.18 ms per 33M pairs; a wave to 2048 slots, eight loads in
+// flight, an atomic each, 0.17; now 0.07.)
+constexpr uint32_t kHashUnroll = 8;
+constexpr uint32_t kHashBlock = kWaves * kWave * kHashUnroll * 8;
 
 __global__ void __launch_bounds__(kThreads) k_hash_requests(const BatchArgs a,
                                                             unsigned long long* __restrict__ hashes) {
+  __shared__ uint64_t s_sum[kWaves];
   const BatchHeader h = *a.header;
   const uint64_t hi = a.total[0] < a.arena_cap ? a.total[0] : a.arena_cap;
   if (h.n_requests == 0 || h.n_queries == 0 || hi == 0) return;
-  const uint32_t lane = lane_id();
-  const uint64_t waves = (uint64_t)gridDim.x * kWaves;
-  const uint64_t w0 = (uint64_t)blockIdx.x * kWaves + threadIdx.x / kWave;
-  for (uint64_t b0 = w0 * kHashBlock; b0 < hi; b0 += waves * kHashBlock) {
+  const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
+  for (uint64_t b0 = (uint64_t)blockIdx.x * kHashBlock; b0 < hi;
+       b0 += (uint64_t)gridDim.x * kHashBlock) {
     const uint64_t b1 = b0 + kHashBlock < hi ? b0 + kHashBlock : hi;
+    const uint64_t w0 = b0 + wave * (kHashBlock / kWaves);
+    const uint64_t w1 = w0 + kHashBlock / kWaves < b1 ? w0 + kHashBlock / kWaves : b1;
     // The last request that starts at or before b0; earlier ones that start
     // there too are empty.
     uint32_t lo = 0, end = h.n_requests;
@@ -466,18 +472,43 @@ __global__ void __launch_bounds__(kThreads) k_hash_requests(const BatchArgs a,
       const uint32_t mid = (lo + end) >> 1;
       if (a.ranges[2 * mid] <= b0) lo = mid; else end = mid;
     }
-    for (uint32_t r = lo; r < h.n_requests; r++) {
+    for (uint32_t r = lo; r < h.n_requests; r++) {  // the same for every wave
       const uint64_t s0 = a.ranges[2 * r], s1 = s0 + a.ranges[2 * r + 1];
       if (s0 >= b1) break;
-      const uint64_t i0 = s0 > b0 ? s0 : b0, i1 = s1 < b1 ? s1 : b1;
-      if (i0 >= i1) continue;
-      uint64_t hs = 0;
-      for (uint64_t i = i0 + lane; i < i1; i += kWave) {
+      if (s1 <= b0 || s0 == s1) continue;
+      const uint64_t i0 = s0 > w0 ? s0 : w0, i1 = s1 < w1 ? s1 : w1;
+      uint64_t hs = 0, i = i0 + lane;
+      for (; i - lane + kHashUnroll * kWave <= i1; i += kHashUnroll * kWave) {
+        rts_pair p[kHashUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kHashUnroll; u++) p[u] = a.arena[i + u * kWave];
+        // The hash factors: mostly all of one query's.
+        const uint32_t q = readlane_u32(p[0].query_id, 0);
+        bool same = true;
+#pragma unroll
+        for (uint32_t u = 0; u < kHashUnroll; u++) same &= p[u].query_id == q;
+        if (ballot(!same) == 0) {
+          uint64_t g = 0;
+#pragma unroll
+          for (uint32_t u = 0; u < kHashUnroll; u++) g += ghash(p[u].geom_id);
+          hs += qmult(q) * g;
+        } else {
+#pragma unroll
+          for (uint32_t u = 0; u < kHashUnroll; u++) hs += pair_hash(p[u].query_id, p[u].geom_id);
+        }
+      }
+      for (; i < i1; i += kWave) {
         const rts_pair p = a.arena[i];
         hs += pair_hash(p.query_id, p.geom_id);
       }
       hs = wave_sum_u64(hs);
-      if (lane == 0 && hs) atomicAdd(&hashes[r], (unsigned long long)hs);
+      if (lane == 0) s_sum[wave] = hs;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        for (int w = 1; w < kWaves; w++) hs += s_sum[w];
+        if (hs) atomicAdd(&hashes[r], (unsigned long long)hs);
+      }
+      __syncthreads();
     }
   }
 }
@@ -507,7 +538,7 @@ __global__ void __launch_bounds__(kThreads) k_rebase_hash_span(rts_pair* __restr
 
 hipError_t launch_hash_requests(const BatchArgs& a, unsigned long long* hashes,
                                 hipStream_t stream) {
-  hipLaunchKernelGGL(k_hash_requests, dim3(4096), dim3(kThreads), 0, stream, a, hashes);
+  hipLaunchKernelGGL(k_hash_requests, dim3(2048), dim3(kThreads), 0, stream, a, hashes);
   return hipGetLastError();
 }
 

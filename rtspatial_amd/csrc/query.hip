@@ -345,97 +345,24 @@ __global__ void __launch_bounds__(kWave) k_wave_write(const QueryLaunch q, const
   }
 }
 
-// The write pass from the logs. A wave owns a window of the output, not some
-// queries: query i takes the units [offsets[i] + kWindowCost i, offsets[i + 1]
-// + kWindowCost (i + 1)), its results and kWindowCost more for having been
-// looked at, and every wave an equal share of all units. So a query of 1e5
-// results is written by many waves, each skipping to its share of the log, and
-// 1e5 queries without results are skipped by many too. A query that overflowed
-// its log is walked again by the wave whose window it starts in. Queries that
-// octets logged are written by octets, 8 at a time.
-// Bound by the stores and by latency (log, leaf ids, store). A wave per query,
-// octets per light query, by tickets: 20k queries of 1000 results 188 us, now
-// 80 (160 MB); 1M of 20, 302 and 195; 100 of 1000, 152 and 15. The last two
-// also by the longer logs and the octets' plain stores.
-constexpr uint32_t kWindowCost = 4;
-constexpr uint32_t kWindowMin = 32;
-
+// The write pass from the logs (write_window).
 template <int PRED, bool POINTS, bool F64>
 __global__ void __launch_bounds__(kWave) k_window_write(const QueryLaunch q, const WaveArgs a) {
   __shared__ WideLds s_lds;
   const TreeView t = q.tree;
   const rts_dev_queue* dq = static_cast<const rts_dev_queue*>(q.sink.arg);
-  const uint32_t lane = lane_id();
-  const uint64_t units = a.total[0] + (uint64_t)kWindowCost * q.n;
-  uint64_t per = (units + gridDim.x - 1) / gridDim.x;
-  if (per < kWindowMin) per = kWindowMin;
-  // Neighbouring windows on one XCD.
-  const uint64_t m0 = (uint64_t)(blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds) * per;
-  if (m0 >= units) return;
-  const uint64_t m1 = m0 + per;
-  // The last query that starts at m0 or before, 64 probes at a time.
-  uint32_t first = 0, len = q.n;
-  while (len > 1) {
-    const uint32_t step = (len + kWave - 1) / kWave, at = lane * step;
-    const bool before =
-        at < len && a.offsets[first + at] + (uint64_t)kWindowCost * (first + at) <= m0;
-    const uint32_t k = (uint32_t)__popcll(ballot(before)) - 1u;  // query `first` is one
-    first += k * step;
-    len = len - k * step < step ? len - k * step : step;
-  }
-  const uint64_t base = a.base[0], cap = dq->capacity;
-  for (uint32_t b = first; b < q.n; b += kWave) {
-    // Lane l: query b + l and its results [lo, hi) that are this window's.
-    const uint32_t i = b + lane;
-    uint64_t slot = 0, at = ~0ull;
-    if (i < q.n) {
-      slot = a.offsets[i];
-      at = slot + (uint64_t)kWindowCost * i;
-      slot += base;
-    }
-    const bool in = at < m1;
-    if (!ballot(in)) break;
-    uint32_t c = 0, n = 0, off = 0, lo = 0, hi = 0;
-    if (in) {
-      c = a.counts[i];
-      n = a.log.n[i];
-      off = a.log.off[i];
-      lo = at >= m0 ? 0u : (m0 - at < c ? (uint32_t)(m0 - at) : c);
-      hi = m1 - at < c ? (uint32_t)(m1 - at) : c;
-      if (n == kLogOverflow) hi = at >= m0 ? c : 0u;
-    }
-    const bool some = lo < hi;
-    const uint64_t light = ballot(some && !(n & kLogWave));
-    for (uint32_t g = 0; g < (uint32_t)kWave; g += kFan) {
-      if (!((light >> g) & 0xFFu)) continue;
-      const int l = (int)(g + lane / kFan);
-      const uint32_t en = (uint32_t)__shfl((int)n, l, 64), eo = (uint32_t)__shfl((int)off, l, 64);
-      const uint32_t elo = (uint32_t)__shfl((int)lo, l, 64), ehi = (uint32_t)__shfl((int)hi, l, 64);
-      const uint64_t es = __shfl(slot, l, 64);
-      const bool mine = (light >> l) & 1u;
-      oct_replay(t, a.log.entries + eo, mine ? en : 0u, dq->data, cap, es, elo, ehi,
-                 b + (uint32_t)l + q.qid_base);
-    }
-    uint64_t heavy = ballot(some && (n & kLogWave));
-    while (heavy) {
-      const int l = __builtin_ctzll(heavy);
-      heavy &= heavy - 1;
-      const uint32_t qi = b + (uint32_t)l, ln = readlane_u32(n, l);
-      const QueueEmit emit{dq->data, cap,
-                           (uint64_t)readlane_u32((uint32_t)(slot >> 32), l) << 32 |
-                               readlane_u32((uint32_t)slot, l)};
-      if (ln != kLogOverflow) {
-        RangeLog lg;
-        lg.entries = a.log.entries + readlane_u32(off, l);
-        lg.n_in = ln & ~kLogWave;
-        wide_replay(t, lg, readlane_u32(lo, l), readlane_u32(hi, l), qi + q.qid_base, emit);
-      } else {
+  const Windows w{a.offsets, a.counts, a.log, dq->data, dq->capacity, a.base[0], a.total[0], q.n};
+  write_window(
+      t, w,
+      [&](uint32_t i, uint32_t* qid) {
+        *qid = i + q.qid_base;
+        return true;
+      },
+      [&](uint32_t i, uint32_t qid, const QueueEmit& emit) {
         query_t<PRED, F64> qb;
-        load_q(q.queries, POINTS, qi, qb);
-        wide_walk<PRED, POINTS, true, false>(t, qb, qi + q.qid_base, emit, s_lds);
-      }
-    }
-  }
+        load_q(q.queries, POINTS, i, qb);
+        wide_walk<PRED, POINTS, true, false>(t, qb, qid, emit, s_lds);
+      });
 }
 
 struct StagedEmit {
@@ -595,8 +522,8 @@ hipError_t launch_wave_f(const QueryLaunch& q, const WaveArgs& a, int phase, hip
     default: {
       if (a.log.entries) {
         auto* k = &k_window_write<PRED, POINTS, F64>;
-        static const uint32_t resident = resident_waves(k);
-        uint32_t blocks = q.n < resident ? std::min(resident, 512 + 4 * q.n) : resident;
+        const uint32_t most = device_cus() * kWindowWaves;
+        uint32_t blocks = q.n < most ? std::min(most, 512 + 4 * q.n) : most;
         blocks = (blocks + kXcds - 1) / kXcds * kXcds;
         hipLaunchKernelGGL(k, dim3(blocks), dim3(kWave), 0, stream, q, a);
         break;

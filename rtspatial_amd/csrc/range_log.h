@@ -41,8 +41,8 @@ __device__ __forceinline__ uint2 log_load(const uint2* p) {
 struct RangeLog {
   uint2* entries = nullptr;
   uint32_t cap = 0;
-  uint32_t logged = 0;           // counting walk (wave-uniform)
-  uint32_t n_in = kLogOverflow;  // writing walk: entries to emit (kLogOverflow: walk the tree)
+  uint32_t logged = 0;  // counting walk (wave-uniform)
+  uint32_t n_in = 0;    // replay: entries to emit
 };
 
 // A count-pass wave's place in its region.
@@ -109,19 +109,6 @@ __device__ __forceinline__ bool log_commit_octets(LogCursor& c, const RangeLogAr
   }
   c.fill += total;
   return true;
-}
-
-// The log a writing walk of query g replays (n_in = kLogOverflow: none).
-__device__ __forceinline__ RangeLog log_for_write(const RangeLogArgs& la, uint64_t g) {
-  RangeLog lg;
-  if (la.entries) {
-    // Wave-uniform values, kept in scalar registers.
-    lg.n_in = readlane_u32(la.n[g], 0);
-    if (lg.n_in != kLogOverflow) lg.n_in &= ~kLogWave;
-    lg.cap = kLogQueryMax;
-    lg.entries = la.entries + readlane_u32(la.off[g], 0);
-  }
-  return lg;
 }
 
 }  // namespace rts

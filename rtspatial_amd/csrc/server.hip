@@ -150,7 +150,6 @@ struct Slot {
   char* d_desc = nullptr;
   uint32_t* d_counters = nullptr;
   uint32_t* d_heavy = nullptr;   // extension requests: wave_heavy_words(max_batch_queries)
-  uint32_t* d_giants = nullptr;  // kGiantBuckets x max_batch_queries tile ids
   uint2* d_log = nullptr;        // range-log entries (kServeLogPerQuery per query)
   uint32_t* d_log_off = nullptr; // per query: first range-log entry
   uint32_t* d_log_n = nullptr;   // per query: range-log entries
@@ -397,8 +396,6 @@ BatchArgs slot_args(const Engine& E, const Slot& s) {
   a.arena = s.d_arena;
   a.arena_cap = E.cfg.arena_pairs;
   a.order = nullptr;
-  a.giants = s.d_giants;
-  a.giant_cap = (uint32_t)E.cfg.max_batch_queries;
   a.log.entries = s.d_log;
   a.log.n_entries = serve_log_entries(E.cfg.max_batch_queries);
   a.log.off = s.d_log_off;
@@ -458,7 +455,6 @@ int slot_init(Engine& E, Slot& s) {
     need = 0;
     carve(&s.d_desc, E.desc_bytes);
     carve(&s.d_counters, kTileCounterWords * sizeof(uint32_t));
-    carve(&s.d_giants, kGiantBuckets * maxq * sizeof(uint32_t));
     carve(&s.d_heavy, wave_heavy_words(maxq) * sizeof(uint32_t));
     carve(&s.d_log, serve_log_entries(maxq) * sizeof(uint2));
     carve(&s.d_log_off, maxq * sizeof(uint32_t));

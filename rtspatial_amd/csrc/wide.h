@@ -565,4 +565,111 @@ __device__ void wide_replay(const TreeView& t, const RangeLog& lg, uint32_t lo, 
   }
 }
 
+// -------------------------------------------------------------- windows ----
+// A write pass from the logs. A wave owns a window of the output, not some
+// queries: query i takes the units [offsets[i] + kWindowCost i, offsets[i + 1]
+// + kWindowCost (i + 1)), its results and kWindowCost more for having been
+// looked at, and every wave an equal share of all units. So a query of 1e5
+// results is written by many waves, each skipping to its share of the log, and
+// 1e5 queries without results are skipped by many too. A query that overflowed
+// its log is walked again by the wave whose window it starts in. Queries that
+// octets logged are written by octets, 8 at a time.
+// Bound by the stores and by latency (log, leaf ids, store). A wave per query,
+// octets per light query, by tickets: 20k queries of 1000 results 188 us, now
+// 80 (160 MB); 1M of 20, 302 and 195; 100 of 1000, 152 and 15. The last two
+// also by longer logs and the octets' plain stores.
+constexpr uint32_t kWindowCost = 4;
+constexpr uint32_t kWindowMin = 32;
+// Windows per CU: all of them resident in every kernel. 1M within queries: 8 341
+// us, 16 225, 24 194, 28 192, 32 236.
+constexpr uint32_t kWindowWaves = 24;
+
+struct Windows {
+  const uint64_t* offsets;
+  const uint32_t* counts;
+  RangeLogArgs log;
+  rts_pair* out;
+  uint64_t cap;      // slots of out
+  uint64_t base;     // query i's first result goes to slot base + offsets[i]
+  uint64_t results;  // of all queries
+  uint32_t n;        // queries
+};
+
+// This wave's window, one wave per workgroup (the grid is whole rounds over the
+// XCDs: neighbouring windows are on one). `ids(i, &qid)`: whether query i is
+// written here, and the id to report; called by every lane whose i < w.n.
+// `walk(i, qid, emit)`: the whole wave walks query i.
+template <typename Ids, typename Walk>
+__device__ __forceinline__ void write_window(const TreeView& t, const Windows& w, const Ids& ids,
+                                             const Walk& walk) {
+  const uint32_t lane = lane_id();
+  const uint64_t units = w.results + (uint64_t)kWindowCost * w.n;
+  uint64_t per = (units + gridDim.x - 1) / gridDim.x;
+  if (per < kWindowMin) per = kWindowMin;
+  const uint64_t m0 =
+      (uint64_t)(blockIdx.x % kXcds * (gridDim.x / kXcds) + blockIdx.x / kXcds) * per;
+  if (m0 >= units) return;
+  const uint64_t m1 = m0 + per;
+  // The last query that starts at m0 or before, 64 probes at a time.
+  uint32_t first = 0, len = w.n;
+  while (len > 1) {
+    const uint32_t step = (len + kWave - 1) / kWave, at = lane * step;
+    const bool before =
+        at < len && w.offsets[first + at] + (uint64_t)kWindowCost * (first + at) <= m0;
+    const uint32_t k = (uint32_t)__popcll(ballot(before)) - 1u;  // query `first` is one
+    first += k * step;
+    len = len - k * step < step ? len - k * step : step;
+  }
+  for (uint32_t b = first; b < w.n; b += kWave) {
+    // Lane l: query b + l and its results [lo, hi) that are this window's.
+    const uint32_t i = b + lane;
+    uint64_t slot = 0, at = ~0ull;
+    if (i < w.n) {
+      slot = w.offsets[i];
+      at = slot + (uint64_t)kWindowCost * i;
+      slot += w.base;
+    }
+    const bool in = at < m1;
+    if (!ballot(in)) break;
+    uint32_t n = 0, off = 0, lo = 0, hi = 0, qid = 0;
+    if (in && ids(i, &qid)) {
+      const uint32_t c = w.counts[i];
+      n = w.log.n[i];
+      off = w.log.off[i];
+      lo = at >= m0 ? 0u : (m0 - at < c ? (uint32_t)(m0 - at) : c);
+      hi = m1 - at < c ? (uint32_t)(m1 - at) : c;
+      if (n == kLogOverflow) hi = at >= m0 ? c : 0u;
+    }
+    const bool some = lo < hi;
+    const uint64_t light = ballot(some && !(n & kLogWave));
+    for (uint32_t g = 0; g < (uint32_t)kWave; g += kFan) {
+      if (!((light >> g) & 0xFFu)) continue;
+      const int l = (int)(g + lane / kFan);
+      const uint32_t en = (uint32_t)__shfl((int)n, l, 64), eo = (uint32_t)__shfl((int)off, l, 64);
+      const uint32_t elo = (uint32_t)__shfl((int)lo, l, 64), ehi = (uint32_t)__shfl((int)hi, l, 64);
+      const uint32_t eq = (uint32_t)__shfl((int)qid, l, 64);
+      const uint64_t es = __shfl(slot, l, 64);
+      const bool mine = (light >> l) & 1u;
+      oct_replay(t, w.log.entries + eo, mine ? en : 0u, w.out, w.cap, es, elo, ehi, eq);
+    }
+    uint64_t heavy = ballot(some && (n & kLogWave));
+    while (heavy) {
+      const int l = __builtin_ctzll(heavy);
+      heavy &= heavy - 1;
+      const uint32_t ln = readlane_u32(n, l), lq = readlane_u32(qid, l);
+      const QueueEmit emit{w.out, w.cap,
+                           (uint64_t)readlane_u32((uint32_t)(slot >> 32), l) << 32 |
+                               readlane_u32((uint32_t)slot, l)};
+      if (ln != kLogOverflow) {
+        RangeLog lg;
+        lg.entries = w.log.entries + readlane_u32(off, l);
+        lg.n_in = ln & ~kLogWave;
+        wide_replay(t, lg, readlane_u32(lo, l), readlane_u32(hi, l), lq, emit);
+      } else {
+        walk(b + (uint32_t)l, lq, emit);
+      }
+    }
+  }
+}
+
 }  // namespace rts

@@ -120,7 +120,8 @@ int ensure_tree_capacity(rts_index* ix, uint64_t n) {
   dev_free(ix->delta_wide_live);
   dev_free(ix->sort_scratch);
   dev_free(ix->partials);
-  RTS_HIP(dev_alloc(&ix->leaf_boxes, cap));
+  // (Walks load, and drop, what follows the last leaf up to a whole block.)
+  RTS_HIP(dev_alloc(&ix->leaf_boxes, cap + kFan));
   RTS_HIP(dev_alloc(&ix->leaf_ids, cap));
   RTS_HIP(dev_alloc(&ix->keys, cap));
   RTS_HIP(dev_alloc(&ix->keys_alt, cap));

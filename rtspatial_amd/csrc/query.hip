@@ -52,8 +52,9 @@ template <int PRED, bool POINTS, bool F64>
 struct OctSource {
   const void* queries;
   const uint32_t* order;
+  __device__ uint32_t id(uint32_t i) const { return order ? order[i] : i; }
   __device__ void operator()(uint32_t i, query_t<PRED, F64>& q) const {
-    load_q(queries, POINTS, order ? order[i] : i, q);
+    load_q(queries, POINTS, id(i), q);
   }
 };
 
@@ -184,7 +185,7 @@ __global__ void __launch_bounds__(kOctThreads)
 // a time; the others are listed (one atomic per ticket), and the second
 // launch's waves walk them one by one. A wave half of whose queries turn out
 // heavy lists kSkip tickets without trying. 1M within queries of 20 results
-// count in 0.51 ms (1.58 a wave each; 3.3 on the binary tree); on the 10M x 1M
+// count in 0.47 ms (1.58 a wave each; 3.3 on the binary tree); on the 10M x 1M
 // join, whose queries are heavy, the trial costs 0.3 of 5 ms. (Having the same
 // wave walk its heavy queries made the join with 200k queries 1.7x slower:
 // sixteen long walks in a row on some waves, none on others.)
@@ -224,7 +225,7 @@ __global__ void __launch_bounds__(kWave) k_light_count(const QueryLaunch q, cons
       slice_tickets(wave_counters(a.tickets, kTicketsLight), wave_counters(a.tickets, kFlagsLight),
                     slice_size(q.n), group);
   const uint32_t per = slice_length(q.n);
-  LogCursor lc = LOG ? log_cursor(a.log) : LogCursor{};
+  OctLogCursor lc = LOG ? oct_log_cursor(a.log) : OctLogCursor{};
   uint64_t sum = 0;  // octet-uniform: without LOG
   uint32_t skip = 0;
   // Every iteration takes a query or finds none left.
@@ -238,10 +239,9 @@ __global__ void __launch_bounds__(kWave) k_light_count(const QueryLaunch q, cons
     if (m < (uint32_t)kFan || skip) {
       skip -= skip ? 1u : 0u;
     } else {
-      auto commit = [&](bool done, uint32_t i, uint32_t found, uint32_t n, const uint2* log) {
+      auto commit = [&](bool done, uint32_t qi, uint32_t found, uint32_t n, const uint2* log) {
         if (LOG) {
-          const uint32_t qi = q.order && done ? q.order[i] : i;
-          if (!log_commit_octets(lc, a.log, done, qi, n, log)) return false;
+          if (!log_commit_octet(lc, a.log, done, qi, n, log)) return false;
           if (done && (lane & 7u) == 0) a.counts[qi] = found;
         } else if (done) {
           sum += found;

@@ -87,27 +87,35 @@ __device__ __forceinline__ void log_commit(LogCursor& c, const RangeLogArgs& la,
   if (fit) c.fill += lg.logged;
 }
 
-// After octets completed queries (`done`, octet-uniform, as are g, n and the
-// n entries in `log`, in LDS): their entries and headers. Called by the whole
-// wave. False: they do not fit the wave's region and are not logged.
-__device__ __forceinline__ bool log_commit_octets(LogCursor& c, const RangeLogArgs& la, bool done,
-                                                  uint64_t g, uint32_t n, const uint2* log) {
-  if (!c.region) return true;
-  const uint32_t lane = lane_id(), j = lane & 7u;
-  const uint32_t mine = done && j == 0 ? n : 0u;
-  const uint32_t inc = wave_inclusive_sum(mine);
-  const uint32_t total = readlane_u32(inc, kWave - 1);
-  if (total > c.room - c.fill) return false;
-  // Lane 8o's inclusive sum less its own is octet o's place.
-  const uint32_t at = c.fill + (uint32_t)__shfl((int)(inc - mine), (int)(lane & ~7u), 64);
-  if (done) {
-    for (uint32_t k = j; k < n; k += 8) log_store(c.region + at + k, log[k].x, log[k].y);
-    if (j == 0) {
-      la.n[g] = n;
-      la.off[g] = c.base + at;
-    }
+// An octet's place in its eighth of the wave's region (octet-uniform).
+struct OctLogCursor {
+  uint2* region = nullptr;
+  uint32_t base = 0, room = 0, fill = 0;  // as LogCursor's
+};
+__device__ __forceinline__ OctLogCursor oct_log_cursor(const RangeLogArgs& la) {
+  OctLogCursor c;
+  if (la.entries) {
+    c.room = la.per_wave / 8u;
+    c.base = la.first + blockIdx.x * la.per_wave + lane_id() / 8u * c.room;
+    c.region = la.entries + c.base;
   }
-  c.fill += total;
+  return c;
+}
+
+// After octets completed queries (`done`, octet-uniform, as are g, n and the
+// n entries in `log`, in LDS): their entries and headers. False: they do not
+// fit the octet's region and are not logged.
+__device__ __forceinline__ bool log_commit_octet(OctLogCursor& c, const RangeLogArgs& la, bool done,
+                                                 uint64_t g, uint32_t n, const uint2* log) {
+  if (!c.region) return true;
+  if (!done || n > c.room - c.fill) return false;
+  const uint32_t j = lane_id() & 7u;
+  for (uint32_t k = j; k < n; k += 8) log_store(c.region + c.fill + k, log[k].x, log[k].y);
+  if (j == 0) {
+    la.n[g] = n;
+    la.off[g] = c.base + c.fill;
+  }
+  c.fill += n;
   return true;
 }
 

@@ -241,71 +241,63 @@ __device__ void oct_walk(const TreeView& t, uint32_t* stack, uint32_t first, uin
 }
 
 // Counts queries [first, last) (at most 32), one per octet at a time, as far as
-// they are light: one that holds a whole node of 64 or more leaves, logs more
-// than kOctLog - 8 entries or takes more than kOctSteps steps is left to
+// they are light: one that holds a whole node of 64 or more leaves, fills
+// its kOctLog entries or takes more than kOctSteps steps is left to
 // wide_walk, and its bit (i - first) set in the result. (A query of hundreds of
-// results shows such a node after some six steps, before much is wasted on it.) `commit(done, i, found, n, log)` is called by the whole wave
-// when octets complete queries: `done` and the rest are octet-uniform, `n`
-// entries being in `log`, the octet's, in LDS. It returns (wave-uniform)
-// whether it kept them; if not, they are left to wide_walk as well. Without LOG subtrees inside the
-// query are counted from their live counts and nothing is logged.
+// results shows such a node after some six steps, before much is wasted on it.)
+// `src(i, q)` loads query i and `src.id(i)` its id. `commit(done, id, found, n,
+// log)` is called by the whole wave when octets complete queries: `done` and
+// the rest are octet-uniform, `n` entries being in `log`, the octet's, in LDS.
+// It returns (octet-uniform) whether it kept the query; if not, that is left to
+// wide_walk as well. Without LOG nothing is logged.
+// Bound by the vector unit. 1M queries of 20 results on 1M boxes count in 474 us.
+// Taking blocks of leaves inside the query whole (their live counts, another
+// load, held every octet's step), with ids loaded at the commit and the log's
+// places dealt out by a scan over the wave, took 527; at most 32 steps, which
+// leave more queries over, 527 too.
 constexpr uint32_t kOctLog = 32;
-constexpr uint32_t kOctSteps = 32;
+constexpr uint32_t kOctSteps = 48;
 
 template <int PRED, bool POINTS, bool LOG, typename Q, typename Src, typename Commit>
 __device__ uint32_t oct_count(const TreeView& t, uint32_t* stack, uint2* log, uint32_t first,
                               uint32_t last, const Src& src, Commit&& commit) {
   const uint32_t lane = lane_id(), j = lane & 7u, oct = lane >> 3;
-  uint32_t i = first + oct;
+  uint32_t i = first + oct, id = 0, idn = 0;
   bool have = i < last;
   Q q{}, qn{};
-  if (have) src(i, q);
-  if (i + kFan < last) src(i + kFan, qn);
+  if (have) {
+    src(i, q);
+    id = src.id(i);
+  }
+  if (i + kFan < last) {
+    src(i + kFan, qn);
+    idn = src.id(i + kFan);
+  }
   // Octet-uniform:
   uint32_t sp = have ? 1u : 0u, found = 0, n = 0, steps = 0;
-  bool whole = false;  // octet-uniform: a node of 64 leaves lies inside the query
   uint32_t heavy = 0;  // wave-uniform
+  const float4* const leaves = t.leaf_boxes - t.leaf0;
+  const uint32_t leaf_end = t.leaf0 + t.n;
   if (have && j == 0) stack[0] = 0;
   lds_fence();
   while (ballot(have)) {
     const uint32_t e = have ? stack[sp - 1] : 0u;
     const uint32_t child = kFan * e + 1u + j;
     const bool at_leaf = child >= t.leaf0;  // octet-uniform
-    const uint32_t leaf = child - t.leaf0;
-    const bool ok = have && (!at_leaf || leaf < t.n);
-    float4 b = nan_box();
-    if (ok) b = *(at_leaf ? t.leaf_boxes + leaf : t.wide + child);
+    const bool ok = have && child < leaf_end;
+    // As in wide_walk, lanes without a child load a box that exists.
+    const float4 b = (at_leaf ? leaves : t.wide)[child];
     bool hit = false;
-    if (ok) hit = at_leaf ? leaf_test<PRED, POINTS>(t, leaf, b, q) : node_test<PRED, POINTS>(b, q);
+    if (ok)
+      hit = at_leaf ? leaf_test<PRED, POINTS>(t, child - t.leaf0, b, q)
+                    : node_test<PRED, POINTS>(b, q);
+    const uint32_t m8 = (uint32_t)(ballot(hit) >> (8u * oct)) & 0xFFu;
+    bool whole = false;  // octet-uniform: a node of 64 leaves lies inside the query
     if (!POINTS) {
-      const bool inside = hit && !at_leaf && inside_test<PRED, POINTS>(b, q);
-      const uint64_t in = ballot(inside);
-      if (in) {
-        // A node whose children are leaves holds at most 8.
-        const uint32_t in8 = (uint32_t)(in >> (8u * oct)) & 0xFFu;
-        whole = in8 && kFan * child + 1u < t.leaf0;
-        uint32_t live = inside ? t.wide_live[child] : 0u;
-        uint32_t rf = 0, rn = 0;
-        bool take = inside && !whole;
-        if (LOG && take) {
-          wide_leaves(t, child, &rf, &rn);
-          take = live == rn;  // otherwise a deleted box lies below: descend
-        }
-        if (take) hit = false;
-        uint32_t add = take ? live : 0u;
-        add += __shfl_xor(add, 1, 64);
-        add += __shfl_xor(add, 2, 64);
-        add += __shfl_xor(add, 4, 64);
-        found += add;
-        if (LOG) {
-          const uint32_t m8 = (uint32_t)(ballot(take) >> (8u * oct)) & 0xFFu;
-          if (take) log[n + (uint32_t)__popc(m8 & ((1u << j) - 1u))] = make_uint2(rf, (1u << rn) - 1u);
-          n += (uint32_t)__popc(m8);
-        }
-      }
+      // A node whose children are leaves holds at most 8.
+      const uint64_t in = ballot(hit && kFan * child + 1u < t.leaf0 && inside_test<PRED, POINTS>(b, q));
+      whole = (uint32_t)(in >> (8u * oct)) & 0xFFu;
     }
-    const uint64_t hits = ballot(hit);
-    const uint32_t m8 = (uint32_t)(hits >> (8u * oct)) & 0xFFu;
     if (have) {
       sp--;
       steps++;
@@ -313,19 +305,19 @@ __device__ uint32_t oct_count(const TreeView& t, uint32_t* stack, uint2* log, ui
     if (at_leaf) {
       found += (uint32_t)__popc(m8);
       if (LOG && m8) {
-        if (j == 0) log[n] = make_uint2(leaf, m8);
+        if (j == 0) log[n] = make_uint2(child - t.leaf0, m8);
         n++;
       }
     } else {
       if (hit) stack[sp + (uint32_t)__popc(m8 & ((1u << j) - 1u))] = child;
       sp += (uint32_t)__popc(m8);
     }
-    const bool done = have && sp == 0 && !whole;
+    const bool done = have && sp == 0;
     const bool leave =
-        have && !done && (whole || (LOG && n + kFan > kOctLog) || steps >= kOctSteps);
+        have && !done && (whole || (LOG && n >= kOctLog) || steps >= kOctSteps);
     lds_fence();
     if (ballot(done || leave)) {
-      const bool kept = commit(done, i, found, n, log);
+      const bool kept = commit(done, id, found, n, log);
       uint64_t lm = ballot((leave || (done && !kept)) && j == 0);
       while (lm) {
         const int l = __builtin_ctzll(lm);
@@ -336,11 +328,14 @@ __device__ uint32_t oct_count(const TreeView& t, uint32_t* stack, uint2* log, ui
         i += kFan;
         have = i < last;
         q = qn;
+        id = idn;
         found = n = steps = 0;
-        whole = false;
         sp = have ? 1u : 0u;
         if (have && j == 0) stack[0] = 0;
-        if (i + kFan < last) src(i + kFan, qn);
+        if (i + kFan < last) {
+          src(i + kFan, qn);
+          idn = src.id(i + kFan);
+        }
       }
       lds_fence();
     }

@@ -1,4 +1,4 @@
-"""Benchmarks of the LBVH spatial index on one MI355X. Prints one JSON line.
+"""Benchmarks of the spatial index on one MI355X. Prints one JSON line.
 
 Default workload (--workload served): the served mixed stream over the 10M-box
 index the headline metric is quoted on. 10M Gaussian-mixture boxes are held
@@ -196,7 +196,7 @@ def cpu_baseline_f64(boxes, pred, queries, threads):
 
 
 def build_rate(R, ix, boxes, torch):
-    """Median LBVH build time over 3 rebuilds, phase-timed on the GPU."""
+    """Median build time over 3 rebuilds, phase-timed on the GPU."""
     R.profile_enable(True)
     ms, sort_ms = [], []
     for _ in range(3):
@@ -569,7 +569,7 @@ def run_join(args):
     traffic, traffic_src = profiled_traffic(wl) if full else (None, None)
     two_pass = prof["query_count"][0] > 0
     pname = {"c1": "contains, points", "c2": "within"}.get(wl, "intersects")
-    kernel = (f"k_query_wave<{pname}, write>" if two_pass else f"k_query_thread<{pname}>")
+    kernel = (f"k_window_write<{pname}>" if two_pass else f"k_oct_collect<{pname}>")
     if JOINS.get(wl):
         desc, _, seeds = JOINS[wl]
     else:
@@ -734,7 +734,7 @@ def run_lines(args):
         "traversals": results,
         "results_agree": bool(agree),
         "sample_check": {"segments": 200, "gpu_pairs": got_sample, "oracle_pairs": want_sample},
-        "roofline": {"bound": "hbm", "kernel": "k_query_*<segment, write> (the default plan's)",
+        "roofline": {"bound": "hbm", "kernel": "k_wave_staged<segment> (the default plan's)",
                      "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "traffic_source": traffic_src,

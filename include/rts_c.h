@@ -138,8 +138,8 @@ typedef enum rts_rebuild_policy {
 /* Traversal mode. */
 typedef enum rts_traversal {
   RTS_TRAVERSAL_AUTO = 0,
-  RTS_TRAVERSAL_THREAD = 1, /* one query per lane */
-  RTS_TRAVERSAL_WAVE = 2    /* one query per wavefront, lanes share its nodes and leaves */
+  RTS_TRAVERSAL_THREAD = 1, /* one query per octet (8 lanes) */
+  RTS_TRAVERSAL_WAVE = 2    /* one query per wavefront (light ones of a large call per octet) */
 } rts_traversal;
 
 /* Coordinate type of an index: SpatialIndex<float,2> or SpatialIndex<double,2>. */
@@ -172,7 +172,7 @@ typedef struct rts_config {
   uint32_t max_query_samples;    /* 1000 */
   uint32_t max_parallelism;      /* 512 */
   /* MI355X additions */
-  uint32_t leaf_size;            /* ranges of <= leaf_size boxes are scanned, not descended (8) */
+  uint32_t leaf_size;            /* user handlers' walks scan runs of <= leaf_size boxes (8) */
   uint32_t rebuild_policy;       /* rts_rebuild_policy (RTS_REBUILD_SAH) */
   float sah_rebuild_ratio;       /* 1.5 */
   uint32_t traversal;            /* rts_traversal (AUTO) */
@@ -352,7 +352,7 @@ int rts_index_sync(rts_index* index, rts_stream_t stream);
 typedef struct rts_index_stats {
   uint64_t n_boxes;        /* ids handed out */
   uint64_t n_tree;         /* leaves in the current tree */
-  uint64_t builds;         /* full LBVH builds */
+  uint64_t builds;         /* full tree builds */
   uint64_t refits;         /* refits after Update/Delete */
   double sah_at_build;     /* SAH-style cost right after the last build */
   double sah_current;      /* the last measured cost (after the last refit) */
@@ -542,9 +542,9 @@ int rts_serve_run(rts_index* index, const rts_serve_config* cfg, const rts_reque
  * IntersectsWhatQueryProfiling, spatial_index.cuh:566-683, times with host
  * stopwatches and stream syncs). */
 enum {
-  RTS_PHASE_BUILD_MORTON = 0,  /* scene bounds + Morton codes */
+  RTS_PHASE_BUILD_MORTON = 0,  /* scene bounds + Hilbert keys */
   RTS_PHASE_BUILD_SORT = 1,    /* radix sort of the codes */
-  RTS_PHASE_BUILD_TREE = 2,    /* leaf gather + Karras hierarchy + refit */
+  RTS_PHASE_BUILD_TREE = 2,    /* leaf gather + bounds of all levels */
   RTS_PHASE_REFIT = 3,         /* refit after Update/Delete */
   RTS_PHASE_MUTATE = 4,        /* Update/Delete scatter */
   RTS_PHASE_QUERY_ORDER = 5,   /* Morton ordering of the queries */

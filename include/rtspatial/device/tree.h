@@ -28,7 +28,7 @@ constexpr int kStackDepth = 72;           // >= max Karras depth (64) + 2
 //   live            {live leaves below the left child, ... the right child,
 //                    split (the left child's last leaf), 0}
 // parent[j] = (parent << 1) | side, for internal j in [0, n-1) and leaf k at
-// [n-1+k]. Leaves are the boxes in Morton order: leaf_boxes[k], id leaf_ids[k].
+// [n-1+k]. Leaves are the boxes in Hilbert order: leaf_boxes[k], id leaf_ids[k].
 struct __align__(64) NodeRec {
   float4 box[2];
   uint4 meta;

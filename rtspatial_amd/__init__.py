@@ -1,4 +1,4 @@
-"""rtspatial_amd: MI355X-native LBVH spatial index with the LibRTS API.
+"""rtspatial_amd: MI355X-native spatial index with the LibRTS API.
 
 The compute path is librtspatial_amd.so (hand-written HIP kernels for gfx950
 behind the C ABI in include/rts_c.h); this package is its Python host mirror.

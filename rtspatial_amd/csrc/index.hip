@@ -1,7 +1,7 @@
-// Host side of the C ABI: index state, LBVH build orchestration, mutation and
+// Host side of the C ABI: index state, tree build orchestration, mutation and
 // query entry points. Mirrors rtspatial::SpatialIndex<float, 2>
 // (reference include/rtspatial/spatial_index.cuh:62-931) with the OptiX
-// GAS/IAS machinery replaced by one LBVH over every inserted box.
+// GAS/IAS machinery replaced by one packed tree over every inserted box.
 //
 // Build policy: Insert appends boxes by id; the next query (or
 // rts_index_build) brings them into a tree once, however many Insert calls

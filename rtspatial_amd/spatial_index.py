@@ -301,7 +301,7 @@ class SpatialIndex:
     def Autotune(self, predicate, queries, collect=True, sample=32768, leaf_sizes=(4, 8, 16, 32),
                  reps=3, apply=True, stream=None):
         """Times the query over a strided sample of `queries` under every
-        plan (leaf size, per-lane or per-wavefront traversal, Morton or input
+        plan (leaf size, per-octet or per-wavefront traversal, Morton or input
         order) and, with `apply`, keeps the fastest for later queries of this
         predicate and query kind. Returns the choice and the sample timings."""
         _check_array(queries, None, self.coord_t, "Autotune")

@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(kOctThreads)
 // launch's waves walk them one by one. A wave half of whose queries turn out
 // heavy lists kSkip tickets without trying. 1M within queries of 20 results
 // count in 0.47 ms (1.58 a wave each; 3.3 on the binary tree); on the 10M x 1M
-// join, whose queries are heavy, the trial costs 0.3 of 5 ms. (Having the same
+// join, whose queries are heavy, the trial costs 0.25 of 4.4 ms. (Having the same
 // wave walk its heavy queries made the join with 200k queries 1.7x slower:
 // sixteen long walks in a row on some waves, none on others.)
 constexpr uint32_t kGroup = 16;

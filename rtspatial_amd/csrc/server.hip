@@ -150,7 +150,7 @@ struct Slot {
   char* d_desc = nullptr;
   uint32_t* d_counters = nullptr;
   uint32_t* d_heavy = nullptr;   // extension requests: wave_heavy_words(max_batch_queries)
-  uint2* d_log = nullptr;        // range-log entries (kServeLogPerQuery per query)
+  uint2* d_log = nullptr;        // range-log entries (serve_log_entries)
   uint32_t* d_log_off = nullptr; // per query: first range-log entry
   uint32_t* d_log_n = nullptr;   // per query: range-log entries
   uint32_t* d_counts = nullptr;  // per query: results

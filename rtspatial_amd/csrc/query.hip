@@ -592,7 +592,10 @@ hipError_t launch_query(const QueryLaunch& q, hipStream_t stream) {
 
 hipError_t launch_query_wave(const QueryLaunch& q, const WaveArgs& a, int phase,
                              hipStream_t stream) {
-  if (q.n == 0 || q.tree.n == 0) return hipSuccess;
+  if (q.n == 0) return hipSuccess;
+  // An empty tree: nothing to walk, but a count pass's counts are still read.
+  if (q.tree.n == 0)
+    return phase == kPhaseCount ? launch_fill_u32(a.counts, 0u, q.n, stream) : hipSuccess;
   if (q.point_queries) return launch_wave<RTS_CONTAINS, true>(q, a, phase, stream);
   switch (q.pred) {
     case RTS_INTERSECTS: return launch_wave<RTS_INTERSECTS, false>(q, a, phase, stream);

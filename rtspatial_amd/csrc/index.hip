@@ -103,6 +103,15 @@ uint64_t delta_cap(const rts_index* ix, uint64_t cap) {
   return std::min<uint64_t>(cap, cap * ix->cfg.insert_delta_pct / 100);
 }
 
+void free_binary(rts_index* ix) {
+  dev_free(ix->nodes);
+  dev_free(ix->parent);
+  dev_free(ix->node_end);
+  dev_free(ix->flags);
+  ix->bcap = 0;
+  ix->bin_valid = false;
+}
+
 int ensure_tree_capacity(rts_index* ix, uint64_t n) {
   if (n <= ix->tcap) return RTS_OK;
   RTS_HIP(hipDeviceSynchronize());
@@ -120,6 +129,7 @@ int ensure_tree_capacity(rts_index* ix, uint64_t n) {
   dev_free(ix->delta_wide_live);
   dev_free(ix->sort_scratch);
   dev_free(ix->partials);
+  free_binary(ix);
   // (Walks load, and drop, what follows the last leaf up to a whole block.)
   RTS_HIP(dev_alloc(&ix->leaf_boxes, cap + kFan));
   RTS_HIP(dev_alloc(&ix->leaf_ids, cap));
@@ -196,25 +206,19 @@ WideArgs wide_args(rts_index* ix, bool delta, bool gather) {
   return a;
 }
 
-// Brings the binary tree over the main tree's leaves up to date; there is no
-// delta tree (ensure_built with `single`).
-int ensure_binary(rts_index* ix, hipStream_t stream) {
-  if (ix->bcap < ix->n_main) {
-    RTS_HIP(hipDeviceSynchronize());
-    dev_free(ix->nodes);
-    dev_free(ix->parent);
-    dev_free(ix->node_end);
-    dev_free(ix->flags);
-    ix->bcap = 0;
-    ix->bin_valid = false;
-    RTS_HIP(dev_alloc(&ix->nodes, ix->tcap));
-    RTS_HIP(dev_alloc(&ix->parent, 2 * ix->tcap));
-    RTS_HIP(dev_alloc(&ix->node_end, ix->tcap));
-    RTS_HIP(dev_alloc(&ix->flags, ix->tcap + refit_boundary_words(ix->tcap)));
-    ix->bcap = ix->tcap;
-  }
+int alloc_binary(rts_index* ix) {
+  RTS_HIP(dev_alloc(&ix->nodes, ix->tcap));
+  RTS_HIP(dev_alloc(&ix->parent, 2 * ix->tcap));
+  RTS_HIP(dev_alloc(&ix->node_end, ix->tcap));
+  RTS_HIP(dev_alloc(&ix->flags, ix->tcap + refit_boundary_words(ix->tcap)));
+  ix->bcap = ix->tcap;
+  return RTS_OK;
+}
+
+// Queues the binary tree's hierarchy, if it is not the current leaves', and
+// its bounds.
+int build_binary(rts_index* ix, hipStream_t stream) {
   const uint32_t n = (uint32_t)ix->n_main;
-  if (ix->bin_valid && !ix->bin_refit_needed) return RTS_OK;
   PhaseToken ph = phase_begin(ix->bin_valid ? RTS_PHASE_REFIT : RTS_PHASE_BUILD_TREE, stream);
   if (!ix->bin_valid)
     RTS_HIP(launch_karras(ix->keys, n, ix->nodes, ix->parent, ix->node_end, stream));
@@ -231,8 +235,48 @@ int ensure_binary(rts_index* ix, hipStream_t stream) {
   a.boundary = ix->flags + ix->bcap;  // after the n - 1 node flags
   RTS_HIP(launch_refit(a, stream));
   phase_end(ph, stream);
-  ix->bin_valid = true;
-  ix->bin_refit_needed = false;
+  return RTS_OK;
+}
+
+// Brings the binary tree over the main tree's leaves up to date for work on
+// `stream`; there is no delta tree (ensure_built with `single`).
+int ensure_binary(rts_index* ix, hipStream_t stream) {
+  const bool captured = capturing(stream);
+  Relaxed relaxed;
+  if (ix->bcap < ix->n_main) {  // (growing the trees freed the old arrays)
+    const int rc = alloc_binary(ix);
+    if (rc) {
+      free_binary(ix);
+      return rc;
+    }
+  }
+  if (!ix->bin_valid || ix->bin_refit_needed) {
+    const bool aside = captured && !ix->tree_captured;
+    if (aside) {
+      if (!ix->bin_stream)
+        RTS_HIP(hipStreamCreateWithFlags(&ix->bin_stream, hipStreamNonBlocking));
+      RTS_HIP(hipStreamWaitEvent(ix->bin_stream, ix->tree_done, 0));
+    }
+    const hipStream_t s = aside ? ix->bin_stream : stream;
+    const int rc = build_binary(ix, s);
+    if (rc) return rc;
+    if (aside) RTS_HIP(hipStreamSynchronize(s));
+    if (!captured) RTS_HIP(hipEventRecord(ix->bin_done, s));
+    ix->bin_pending = !captured;
+    ix->bin_valid = true;
+    ix->bin_refit_needed = false;
+    return RTS_OK;
+  }
+  if (ix->bin_pending) {
+    const hipError_t e = captured ? hipEventSynchronize(ix->bin_done) : hipEventQuery(ix->bin_done);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      RTS_HIP(hipStreamWaitEvent(stream, ix->bin_done, 0));
+    } else {
+      RTS_HIP(e);
+      ix->bin_pending = false;
+    }
+  }
   return RTS_OK;
 }
 
@@ -425,15 +469,18 @@ int device_error_status(rts_index* ix) { return check_device_error(ix); }
 
 int ensure_built(rts_index* ix, hipStream_t stream, bool single) {
   poll_cost(ix);
-  if (ix->stale) return build_tree(ix, stream);
   const bool inserted = ix->n > ix->n_tree;
-  if ((inserted && !delta_ok(ix)) || (single && (ix->n_delta || inserted)))
-    return build_tree(ix, stream);  // a refit pending now is subsumed
-  if (ix->refit_needed) {
-    int rc = refit_tree(ix, stream);
-    if (rc) return rc;
+  int rc = RTS_OK;
+  if (ix->stale || (inserted && !delta_ok(ix)) || (single && (ix->n_delta || inserted))) {
+    rc = build_tree(ix, stream);  // a refit pending now is subsumed
+  } else {
+    if (!ix->refit_needed && !inserted) return RTS_OK;
+    if (ix->refit_needed) rc = refit_tree(ix, stream);
+    if (!rc && inserted) rc = build_delta(ix, stream);
   }
-  if (inserted) return build_delta(ix, stream);
+  if (rc) return rc;
+  ix->tree_captured = capturing(stream);
+  if (!ix->tree_captured) RTS_HIP(hipEventRecord(ix->tree_done, stream));
   return RTS_OK;
 }
 
@@ -497,6 +544,8 @@ int rts_index_create(const rts_config* cfg, rts_index** out) {
   RTS_HIP(hipHostMalloc(reinterpret_cast<void**>(&ix->h_cost), 4 * sizeof(double)));
   RTS_HIP(hipEventCreateWithFlags(&ix->ev_cost_build, hipEventDisableTiming));
   RTS_HIP(hipEventCreateWithFlags(&ix->ev_cost_refit, hipEventDisableTiming));
+  RTS_HIP(hipEventCreateWithFlags(&ix->tree_done, hipEventDisableTiming));
+  RTS_HIP(hipEventCreateWithFlags(&ix->bin_done, hipEventDisableTiming));
   if (ix->cfg.preallocate && ix->cfg.max_geometries) {
     int rc = ensure_id_capacity(ix, ix->cfg.max_geometries, nullptr);
     if (!rc) rc = ensure_tree_capacity(ix, ix->cfg.max_geometries);
@@ -522,10 +571,7 @@ int rts_index_destroy(rts_index* ix) {
   dev_free(ix->keys);
   dev_free(ix->keys_alt);
   dev_free(ix->vals_alt);
-  dev_free(ix->nodes);
-  dev_free(ix->parent);
-  dev_free(ix->node_end);
-  dev_free(ix->flags);
+  free_binary(ix);
   dev_free(ix->wide_mem);
   dev_free(ix->wide_live);
   dev_free(ix->delta_wide_mem);
@@ -536,6 +582,9 @@ int rts_index_destroy(rts_index* ix) {
   if (ix->h_cost) (void)hipHostFree(ix->h_cost);
   if (ix->ev_cost_build) (void)hipEventDestroy(ix->ev_cost_build);
   if (ix->ev_cost_refit) (void)hipEventDestroy(ix->ev_cost_refit);
+  if (ix->tree_done) (void)hipEventDestroy(ix->tree_done);
+  if (ix->bin_done) (void)hipEventDestroy(ix->bin_done);
+  if (ix->bin_stream) (void)hipStreamDestroy(ix->bin_stream);
   if (ix->counted) workspace_index_end(ix->device);
   delete ix;
   return RTS_OK;

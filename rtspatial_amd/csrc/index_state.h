@@ -48,10 +48,20 @@ struct rts_index {
   float4* wide() const { return wide_mem + (rts::kFan - 1); }
   float4* delta_wide() const { return delta_wide_mem + (rts::kFan - 1); }
   // Binary tree over the main tree's leaves, for caller-compiled handlers:
-  // allocated and built by the first rts_index_tree_view after a build.
+  // allocated and built by the first rts_index_tree_view after a build. A view
+  // does not queue the trees' builds again, so one taken on another stream than
+  // the binary tree was queued on waits for that (bin_done), and one taken
+  // while a graph is captured must not leave the tree to the graph's replay: it
+  // is then built at once on bin_stream, after what the trees were last built
+  // or refitted by (tree_done), unless that was captured too.
   uint64_t bcap = 0;
   bool bin_valid = false;         // it has the current leaves' hierarchy
   bool bin_refit_needed = false;  // boxes changed in place since it was fitted
+  bool bin_pending = false;       // bin_done may not have passed yet
+  bool tree_captured = false;     // the last build or refit was queued under capture
+  hipEvent_t tree_done = nullptr;
+  hipEvent_t bin_done = nullptr;
+  hipStream_t bin_stream = nullptr;
   rts::NodeRec* nodes = nullptr;
   uint32_t* parent = nullptr;
   uint32_t* node_end = nullptr;  // far end of each internal node's leaf range (refit meta)

@@ -234,6 +234,20 @@ struct Scratch {
   hipError_t lease(size_t bytes, hipStream_t stream) { return workspace_lease(bytes, stream, &l); }
   char* get() const { return static_cast<char*>(l.p); }
 };
+// Within its scope allocation and event calls are legal also while a stream is
+// captured in a mode that forbids them to threads at large.
+struct Relaxed {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  Relaxed(const Relaxed&) = delete;
+  Relaxed& operator=(const Relaxed&) = delete;
+};
+inline bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  (void)hipStreamIsCapturing(stream, &cap);
+  return cap != hipStreamCaptureStatusNone;
+}
 // An index lives on the device from _begin to _end.
 void workspace_index_begin(int dev);
 void workspace_index_end(int dev);

@@ -45,14 +45,6 @@ Device& device(int dev) {
   return all[dev];
 }
 
-// Allocation and event calls are legal while another thread captures a
-// stream in a mode that forbids them to threads at large.
-struct Relaxed {
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-  ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-};
-
 // Sizes are rounded to an eighth of their power of two (at most 64 MiB), so
 // that calls of nearly equal sizes share blocks.
 size_t rounded(size_t bytes) {
@@ -88,9 +80,7 @@ hipError_t workspace_lease(size_t bytes, hipStream_t stream, Lease* out) {
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
   out->device = dev;
   out->stream = stream;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  (void)hipStreamIsCapturing(stream, &cap);
-  if (cap != hipStreamCaptureStatusNone) {
+  if (capturing(stream)) {
     e = hipMallocAsync(&out->p, bytes, stream);
     if (e == hipSuccess) out->stream_ordered = true;
     return e;

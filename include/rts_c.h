@@ -422,6 +422,14 @@ int rts_index_autotune(rts_index* index, rts_predicate pred, const void* queries
 int rts_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
                    uint32_t* vals_out, uint64_t n, int key_bits, rts_stream_t stream);
 
+/* Gives back the device scratch that query, sort and serve calls keep between
+ * calls on the current device (at most 1/16 of its memory while an index lives
+ * on it), for a program that needs the memory elsewhere. Waits for the work
+ * that uses it. Scratch is also given back when the last index is destroyed,
+ * and when an allocation of the library's finds the device full. No reference
+ * counterpart. */
+int rts_release_scratch(void);
+
 /* Checksum of a result-pair array, for checking result sets too large to
  * compare pair by pair (no reference counterpart). For each query id q <
  * n_queries: counts[q] = pairs with that query id, gsums[q] = sum over them

@@ -13,6 +13,7 @@ from .spatial_index import (  # noqa: F401
     pack_updates,
     profile_enable,
     profile_read,
+    release_scratch,
     sort_pairs,
 )
 
@@ -26,6 +27,7 @@ __all__ = [
     "sort_pairs",
     "profile_enable",
     "profile_read",
+    "release_scratch",
     "RtsError",
     "lib",
 ]

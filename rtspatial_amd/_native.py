@@ -218,6 +218,7 @@ SIGNATURES = [
     ("rts_index_get_stats", _I32, [_VP, ctypes.POINTER(rts_index_stats)]),
     ("rts_index_memory", _I32, [_VP, ctypes.POINTER(rts_memory_usage)]),
     ("rts_sort_pairs", _I32, [_VP, _VP, _VP, _VP, _U64, _I32, _VP]),
+    ("rts_release_scratch", _I32, []),
     ("rts_tune_config_default", None, [ctypes.POINTER(rts_tune_config)]),
     ("rts_index_autotune", _I32, [_VP, _I32, _VP, _U64, _I32, _I32, ctypes.POINTER(rts_tune_config),
                                   ctypes.POINTER(rts_tune_result), _VP]),

@@ -57,7 +57,7 @@ template <typename T>
 hipError_t dev_alloc(T** p, uint64_t count) {
   *p = nullptr;
   if (count == 0) return hipSuccess;
-  return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
+  return device_alloc(reinterpret_cast<void**>(p), count * sizeof(T));
 }
 
 template <typename T>
@@ -1353,11 +1353,11 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
   for (int attempt = 0;; ++attempt) {
     if (tb.sample) RTS_HIP(hipFree(tb.sample));
     tb.sample = nullptr;
-    RTS_HIP(hipMalloc(&tb.sample, m * qbytes));
+    RTS_HIP(device_alloc(&tb.sample, m * qbytes));
     RTS_HIP(launch_gather_strided(queries, (uint32_t)qbytes, n / m, tb.sample, (uint32_t)m, stream));
     if (ix->cfg.coord == RTS_COORD_F64_AS_F32) {
       void* rounded = nullptr;
-      RTS_HIP(hipMalloc(&rounded, m * query_bytes(pts, false)));
+      RTS_HIP(device_alloc(&rounded, m * query_bytes(pts, false)));
       const hipError_t e = launch_round_queries64(tb.sample, pts, m, rounded, stream);
       (void)hipStreamSynchronize(stream);
       (void)hipFree(tb.sample);
@@ -1375,7 +1375,7 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
   void* arg = counter;
   if (handler == RTS_HANDLER_COLLECT) {
     const uint64_t cap = std::min(total, kMaxPairs) + 1;
-    RTS_HIP(hipMalloc(reinterpret_cast<void**>(&tb.pairs), cap * sizeof(rts_pair)));
+    RTS_HIP(dev_alloc(&tb.pairs, cap));
     rts_dev_queue q{tb.pairs, cap, counter};
     RTS_HIP(hipMemcpyAsync(tb.small, &q, sizeof(q), hipMemcpyHostToDevice, stream));
     arg = tb.small;
@@ -1473,7 +1473,7 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
     uint64_t cap = 0;
     if (handler == RTS_HANDLER_COLLECT) {
       cap = (uint64_t)(est_all * 1.5) + 4096;
-      RTS_HIP(hipMalloc(reinterpret_cast<void**>(&tb.all_pairs), cap * sizeof(rts_pair)));
+      RTS_HIP(dev_alloc(&tb.all_pairs, cap));
       rts_dev_queue q{tb.all_pairs, cap, counter};
       RTS_HIP(hipMemcpyAsync(tb.small + 40, &q, sizeof(q), hipMemcpyHostToDevice, stream));
       all_arg = tb.small + 40;

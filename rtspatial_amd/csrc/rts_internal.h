@@ -248,6 +248,8 @@ inline bool capturing(hipStream_t stream) {
   (void)hipStreamIsCapturing(stream, &cap);
   return cap != hipStreamCaptureStatusNone;
 }
+// hipMalloc; a device that is full gets the kept scratch back first.
+hipError_t device_alloc(void** p, size_t bytes);
 // An index lives on the device from _begin to _end.
 void workspace_index_begin(int dev);
 void workspace_index_end(int dev);

@@ -9,8 +9,10 @@
 // intersects queries 8.7 ms (1.9 ms).
 //
 // Kept blocks are bounded: 1/16 of the device's memory while an index lives on
-// it, kIdleBytes otherwise, least recently used given back first; the last
-// index's end and a failed allocation give back all that are idle. A stream
+// it, kIdleBytes otherwise, least recently used given back first (which, like
+// any free, waits for the device). The last index's end, rts_release_scratch
+// and an allocation of the library's that finds the device full
+// (device_alloc: the index's own arrays too) give back all of them. A stream
 // that is being captured gets graph-owned memory instead (stream-ordered from
 // the device's default pool), since a replay may run at any time.
 #include <algorithm>
@@ -69,6 +71,12 @@ void trim(Device& d, size_t most) {
   }
 }
 
+void give_back_all(Device& d) {
+  Relaxed relaxed;
+  std::lock_guard<std::mutex> lk(d.mu);
+  trim(d, 0);
+}
+
 }  // namespace
 
 hipError_t workspace_lease(size_t bytes, hipStream_t stream, Lease* out) {
@@ -88,7 +96,7 @@ hipError_t workspace_lease(size_t bytes, hipStream_t stream, Lease* out) {
   const size_t need = rounded(bytes);
   Relaxed relaxed;
   Device& d = device(dev);
-  std::lock_guard<std::mutex> lk(d.mu);
+  std::unique_lock<std::mutex> lk(d.mu);
   // The smallest block that fits, is not twice as large, and is free for
   // this stream.
   auto best = d.kept.end();
@@ -114,12 +122,8 @@ hipError_t workspace_lease(size_t bytes, hipStream_t stream, Lease* out) {
     d.kept.erase(best);
     return hipSuccess;
   }
-  e = hipMalloc(&out->p, need);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    trim(d, 0);
-    e = hipMalloc(&out->p, need);
-  }
+  lk.unlock();
+  e = device_alloc(&out->p, need);
   if (e != hipSuccess) {
     out->p = nullptr;
     return e;
@@ -131,6 +135,16 @@ hipError_t workspace_lease(size_t bytes, hipStream_t stream, Lease* out) {
     *out = Lease{};
   }
   return e;
+}
+
+hipError_t device_alloc(void** p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  int dev = 0;
+  if (e != hipErrorOutOfMemory || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+    return e;
+  (void)hipGetLastError();
+  give_back_all(device(dev));
+  return hipMalloc(p, bytes);
 }
 
 void workspace_return(Lease* lease) {
@@ -174,3 +188,13 @@ void workspace_index_end(int dev) {
 }
 
 }  // namespace rts
+
+extern "C" int rts_release_scratch(void) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= rts::kMaxDevices) {
+    rts::set_error("rts_release_scratch: no HIP device");
+    return RTS_ERR_MISSING;
+  }
+  rts::give_back_all(rts::device(dev));
+  return RTS_OK;
+}

@@ -368,6 +368,12 @@ def sort_pairs(keys, vals=None, key_bits=32, stream=None):
     return ko, vo
 
 
+def release_scratch():
+    """Gives back the device scratch that calls keep between them on the current
+    device (rts_release_scratch)."""
+    N.check(N.lib().rts_release_scratch(), "release_scratch")
+
+
 def profile_enable(on=True):
     """Per-phase GPU timing (HIP events on the caller's stream)."""
     N.lib().rts_profile_enable(1 if on else 0)

@@ -118,6 +118,7 @@ int ensure_tree_capacity(rts_index* ix, uint64_t n) {
   // Room for a delta tree of up to insert_delta_pct percent on top of n.
   uint64_t cap = std::max<uint64_t>(n + n * ix->cfg.insert_delta_pct / 100, ix->tcap + ix->tcap / 2);
   cap = std::max<uint64_t>(cap, 1024);
+  ix->tcap = 0;  // until all of the arrays are there
   dev_free(ix->leaf_boxes);
   dev_free(ix->leaf_ids);
   dev_free(ix->keys);

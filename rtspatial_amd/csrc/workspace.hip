@@ -138,13 +138,16 @@ hipError_t workspace_lease(size_t bytes, hipStream_t stream, Lease* out) {
 }
 
 hipError_t device_alloc(void** p, size_t bytes) {
-  const hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = hipMalloc(p, bytes);
   int dev = 0;
-  if (e != hipErrorOutOfMemory || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
-    return e;
-  (void)hipGetLastError();
-  give_back_all(device(dev));
-  return hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices) {
+    (void)hipGetLastError();
+    give_back_all(device(dev));
+    e = hipMalloc(p, bytes);
+  }
+  // The caller reports e; it is not to turn up at the program's next HIP call.
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 void workspace_return(Lease* lease) {

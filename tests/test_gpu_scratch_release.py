@@ -75,3 +75,31 @@ def test_index_grows_into_kept_scratch():
     q = np.float32([[-1, -1, 3, 3]])
     assert count(ix, P.kWithin, q) == n + 1000
     ix.Sync()
+
+
+def test_failed_growth_leaves_a_usable_index():
+    log("an index whose growth failed is cleared and used again")
+    gc.collect()
+    torch.cuda.empty_cache()
+    boxes = _boxes()
+    ix = make_index(np.concatenate([boxes] * 3))
+    assert count(ix, P.kIntersects, boxes) >= 3000
+    n = 60_000_000
+    lo = torch.rand((n, 2), device="cuda")
+    b = torch.cat([lo, lo + 1e-5], 1).contiguous()
+    del lo
+    torch.cuda.empty_cache()
+    ix.Insert(b)  # (its copy by id; the trees take another 2.4 GB)
+    R.release_scratch()
+    rest = torch.empty(_free() - GIB, dtype=torch.uint8, device="cuda")
+    try:
+        with pytest.raises(R.RtsError, match="out of memory"):
+            ix.Build()
+    finally:
+        del rest
+        torch.cuda.empty_cache()
+    # Fewer boxes than the arrays held before the growth.
+    ix.Clear()
+    ix.Insert(dev(boxes))
+    assert count(ix, P.kIntersects, boxes) >= 1000
+    ix.Sync()

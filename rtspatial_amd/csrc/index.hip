@@ -23,6 +23,7 @@
 
 #include "rts_internal.h"
 #include "index_state.h"
+#include "rules.h"
 
 namespace rts {
 
@@ -1280,15 +1281,16 @@ int rts_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* k
       (reinterpret_cast<uintptr_t>(vb + n) + 255) & ~uintptr_t(255));
   SortScratch ss;
   sort_scratch_carve(sbase, n, &ss);
-  // The first pass reads device input where it lies. Host input is copied
-  // first, and so is input that is also an output, to the array the first
-  // pass does not write.
+  // The first pass reads input where it lies if it can (sort_reads_in_place);
+  // other input is copied first, to the array the first pass does not write.
+  int device = 0;
+  RTS_HIP(hipGetDevice(&device));
   const bool odd = radix_sort_passes(key_bits) % 2 == 1;
   auto direct = [&](const uint32_t* p) {
     hipPointerAttribute_t at{};
     const bool dev = hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice;
     if (!dev) (void)hipGetLastError();  // an unknown pointer is host memory
-    return dev && p != keys_out && p != vals_out;
+    return sort_reads_in_place(dev, at.device, device, p, keys_out, vals_out, n);
   };
   if (!direct(keys_in)) {
     uint32_t* to = odd ? kb : keys_out;

@@ -1,0 +1,43 @@
+"""Host-side rules of the library that are plain arithmetic
+(rtspatial_amd/csrc/rules.h), compiled for the host and run on the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def evaluate(tmp_path, body):
+    """The integers that a C++ function body prints."""
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("no g++")
+    src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
+    src.write_text('#include <cstdio>\n#include "rules.h"\nusing namespace rts;\nint main() {\n'
+                   f"{body}\n}}\n")
+    subprocess.run([gxx, "-std=c++17", "-Wall", f"-I{ROOT}/rtspatial_amd/csrc", str(src), "-o",
+                    str(exe)], check=True)
+    out = subprocess.run([str(exe)], stdout=subprocess.PIPE, check=True).stdout.decode()
+    return [int(x) for x in out.split()]
+
+
+def test_sort_reads_only_its_own_devices_memory_in_place(tmp_path):
+    got = evaluate(tmp_path, """
+  static uint32_t m[100];
+  auto t = [&](bool dev, int owner, int device, int in, int ko, int vo) {
+    std::printf("%d ", (int)sort_reads_in_place(dev, owner, device, m + in, m + ko, m + vo, 20));
+  };
+  t(true, 0, 0, 0, 20, 40);   // device memory, apart from both outputs
+  t(true, 1, 1, 60, 20, 40);
+  t(false, 0, 0, 0, 20, 40);  // host memory
+  t(true, 1, 0, 0, 20, 40);   // another device's
+  t(true, 0, 1, 0, 20, 40);
+  t(true, 0, 0, 20, 20, 40);  // also an output
+  t(true, 0, 0, 40, 20, 40);
+  t(true, 0, 0, 25, 10, 60);  // overlapping an output's end, or its start
+  t(true, 0, 0, 25, 70, 44);
+  t(true, 0, 0, 20, 0, 40);   // next to both
+""")
+    assert got == [1, 1, 0, 0, 0, 0, 0, 0, 0, 1]

@@ -23,7 +23,6 @@
 
 #include "rts_internal.h"
 #include "index_state.h"
-#include "rules.h"
 
 namespace rts {
 
@@ -724,7 +723,7 @@ int alloc_scratch(uint64_t nq, bool sort, bool wave, bool two_pass, hipStream_t 
   size_t o_log = 0, o_log_off = 0, o_log_n = 0;
   // Range logs: not in a caller's static scratch.
   const bool logs = two_pass && !ext;
-  const uint64_t log_entries = std::min<uint64_t>(std::max(nq * kLogPerQuery, std::min(nq * kLogQueryMax, kLogMinEntries)), kLogMaxEntries);
+  const uint64_t log_entries = query_log_entries(nq);
   if (wave) {
     o_tk = off;
     off = align_up(off + kWaveTicketWords * sizeof(uint32_t));

@@ -454,8 +454,7 @@ uint32_t resident_waves(K kernel) {
 template <typename K>
 void launch_persistent(K kernel, uint32_t resident, uint32_t group, const QueryLaunch& q,
                        WaveArgs a, uint64_t log_first, uint64_t log_entries, hipStream_t stream) {
-  uint32_t blocks = std::min((q.n + group - 1) / group, resident);
-  blocks = (blocks + kXcds - 1) / kXcds * kXcds;
+  const uint32_t blocks = persistent_waves(q.n, group, resident);
   a.log.first = (uint32_t)log_first;
   a.log.per_wave = (uint32_t)(log_entries / blocks);
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWave), 0, stream, q, a, group);

@@ -9,6 +9,7 @@
 
 #include "rts_c.h"
 #include "rtspatial/device/tree.h"
+#include "rules.h"
 
 namespace rts {
 
@@ -169,20 +170,10 @@ struct RangeLogArgs {
   uint32_t* off = nullptr;   // per query: first entry
   uint32_t* n = nullptr;     // per query: entries, or kLogOverflow
 };
-// Range-log entries (8 bytes each) of a two-pass query call: 512 per query, at
-// most 2^29 (4 GiB); in calls of up to 32768 queries, whose waves have few
-// queries to even out long logs, up to kLogQueryMax per query but at most 2^24
-// (128 MiB). With 512 the waves of 10k double queries of 1000 results walked
-// the longest again: 0.23 ms for the write pass, 0.05 with 1600.
-constexpr uint32_t kLogQueryMax = 4096;  // longest log of a query
-constexpr uint64_t kLogPerQuery = 512;
-constexpr uint64_t kLogMinEntries = 1ull << 24;
-constexpr uint64_t kLogMaxEntries = 1ull << 29;
-
 // Counters of wave calls, on lines of 256 bytes: per kind one for each XCD (a
 // counter, or flags), then the counting launches' kSumSlots partial sums.
 enum { kTicketsLight = 0, kFlagsLight, kTicketsHeavy, kFlagsHeavy, kHeavyCount, kTicketKinds };
-constexpr uint32_t kTicketXcds = 8;
+constexpr uint32_t kTicketXcds = kRuleXcds;
 constexpr uint32_t kTicketWords = 64;
 constexpr uint32_t kSumSlots = 32;
 constexpr uint32_t kWaveTicketWords = (kTicketKinds * kTicketXcds + kSumSlots) * kTicketWords;

@@ -41,3 +41,17 @@ def test_sort_reads_only_its_own_devices_memory_in_place(tmp_path):
   t(true, 0, 0, 20, 0, 40);   // next to both
 """)
     assert got == [1, 1, 0, 0, 0, 0, 0, 0, 0, 1]
+
+
+def test_a_wave_with_one_query_can_log_all_of_it(tmp_path):
+    # Calls with a wave to a query, and fewer queries than fill a round of waves
+    # over the XCDs: each wave's share of the log is a query's longest log.
+    got = evaluate(tmp_path, """
+  for (uint32_t n = 1; n <= 4096; n++)
+    if (query_log_entries(n) / persistent_waves(n, 1, 8192) < kLogQueryMax) std::printf("%u ", n);
+  std::printf("0 %u %u %u", persistent_waves(1, 1, 8192), persistent_waves(8193, 4, 8192),
+              persistent_waves(1u << 26, 4, 8192));
+  std::printf(" %d %d", (int)(query_log_entries(32768) == kLogMinEntries),
+              (int)(query_log_entries(1u << 26) == kLogMaxEntries));
+""")
+    assert got == [0, 8, 2056, 8192, 1, 1]

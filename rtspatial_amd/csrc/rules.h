@@ -15,6 +15,13 @@ constexpr uint32_t persistent_waves(uint32_t n, uint32_t group, uint32_t residen
   return ((tickets < resident ? tickets : resident) + kRuleXcds - 1) / kRuleXcds * kRuleXcds;
 }
 
+// Whether heap index i of the packed tree (leaf 0 at leaf0 = (8^D - 1) / 7) lies
+// above the nodes whose children are leaves: it then holds 64 leaves or more
+// (fewer only at the end). Leaves do not: leaf0 + k reaches 1.2e9, and eight
+// times that 2^32, so the test asks where level D - 1 begins instead of where
+// i's children are.
+constexpr bool above_leaf_blocks(uint32_t i, uint32_t leaf0) { return i < (leaf0 - 1) / 8; }
+
 // Range-log entries (8 bytes each) of a two-pass query call, which its waves
 // share equally: 512 per query, at most 2^29 (4 GiB); in calls of up to 32768
 // queries, whose waves have few queries to even out long logs, up to

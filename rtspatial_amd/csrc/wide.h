@@ -295,7 +295,8 @@ __device__ uint32_t oct_count(const TreeView& t, uint32_t* stack, uint2* log, ui
     bool whole = false;  // octet-uniform: a node of 64 leaves lies inside the query
     if (!POINTS) {
       // A node whose children are leaves holds at most 8.
-      const uint64_t in = ballot(hit && kFan * child + 1u < t.leaf0 && inside_test<PRED, POINTS>(b, q));
+      const uint64_t in =
+          ballot(hit && above_leaf_blocks(child, t.leaf0) && inside_test<PRED, POINTS>(b, q));
       whole = (uint32_t)(in >> (8u * oct)) & 0xFFu;
     }
     if (have) {

@@ -15,7 +15,7 @@ def evaluate(tmp_path, body):
     if not gxx:
         pytest.skip("no g++")
     src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
-    src.write_text('#include <cstdio>\n#include "rules.h"\nusing namespace rts;\nint main() {\n'
+    src.write_text('#include <cstdio>\n#include <initializer_list>\n#include "rules.h"\nusing namespace rts;\nint main() {\n'
                    f"{body}\n}}\n")
     subprocess.run([gxx, "-std=c++17", "-Wall", f"-I{ROOT}/rtspatial_amd/csrc", str(src), "-o",
                     str(exe)], check=True)
@@ -55,3 +55,23 @@ def test_a_wave_with_one_query_can_log_all_of_it(tmp_path):
               (int)(query_log_entries(1u << 26) == kLogMaxEntries));
 """)
     assert got == [0, 8, 2056, 8192, 1, 1]
+
+
+def test_leaves_are_not_above_the_leaf_blocks(tmp_path):
+    # At every depth: nodes above level D - 1, and neither that level's nor the
+    # leaves, up to the last of 2^30 - 1.
+    got = evaluate(tmp_path, """
+  for (uint32_t d = 1; d <= 10; d++) {
+    uint64_t leaf0 = 0, last = 0;  // last: first node of level d - 1
+    for (uint32_t k = 0; k < d; k++) { last = leaf0; leaf0 = 8 * leaf0 + 1; }
+    const uint64_t n = d == 10 ? (1ull << 30) - 1 : 1ull << (3 * d);
+    uint64_t wrong = 0;
+    for (const uint64_t i : {(uint64_t)0, last - 1, last, leaf0 - 1, leaf0, leaf0 + n / 3,
+                       (uint64_t)((1ull << 29) - 1), (uint64_t)(1ull << 29),
+                       (uint64_t)((1ull << 29) + 7), leaf0 + n - 1})
+      if (i < leaf0 + n && i != ~0ull)
+        wrong += above_leaf_blocks((uint32_t)i, (uint32_t)leaf0) != (i < last);
+    std::printf("%d ", (int)wrong);
+  }
+""")
+    assert got == [0] * 10

@@ -288,12 +288,14 @@ typedef struct rts_tree_view {
 
 int rts_index_tree_view(rts_index* index, rts_stream_t stream, rts_tree_view* out);
 
-/* The plan the library runs a query call of this kind (`points`: an
- * rts_query_kind) and size under: the config's settings, else the
- * autotuner's stored plan (not for segments), else the defaults.
- * Kernels compiled by the caller follow it to run as the library's do. */
+/* The plan of a query call of this kind (`points`: an rts_query_kind) and size
+ * by kernels the caller compiles around its own result handler, which walk the
+ * tree of rts_index_tree_view: the config's settings, else what the autotuner
+ * measured of such kernels (not for segments), else the defaults. The
+ * library's own calls choose by the same settings and defaults of their own
+ * walks (octets in place of lanes, in input order). */
 typedef struct rts_query_plan {
-  uint32_t traversal;    /* RTS_TRAVERSAL_THREAD or RTS_TRAVERSAL_WAVE */
+  uint32_t traversal;    /* RTS_TRAVERSAL_THREAD (a query per lane) or RTS_TRAVERSAL_WAVE */
   uint32_t sort_queries; /* 1 = Morton-ordered, 2 = input order */
   uint32_t leaf_size;    /* leaf-range size */
   uint32_t reserved;
@@ -377,17 +379,21 @@ int rts_index_memory(rts_index* index, rts_memory_usage* out);
  * CalculateBestParallelism sampling (spatial_index.cuh:41-57,690-760) picks a
  * ray parallelism. It times the query over an evenly strided sample of
  * `queries` (shrunk until its results are at most 2^26 pairs) under every
- * candidate plan -- leaf size, one query per lane or per wavefront (per lane
+ * candidate plan -- one query per octet or per wavefront (collected per octet
  * only when the sample averages at most 256 results per query) -- with the
  * given handler, and then Morton-ordered against input-ordered queries on the
  * whole set when that is cheap (at most 4M queries and, going by the sample,
  * 2^26 results; a strided sample has none of the set's locality). The
  * ordering measured at n queries moves the size rule's threshold (65536
- * queries): calls of at least min(n, 65536) queries are ordered when it won,
- * calls of at most max(n, 65535) are not when it lost. With `apply` set, it
- * stores the fastest plan in the index for this
+ * queries per wavefront, none per octet): calls of at least min(n, threshold)
+ * queries are ordered when it won, calls of at most max(n, threshold - 1) are
+ * not when it lost. Then it times handlers' calls (rts_index_query_plan) in
+ * the same way: leaf size, one query per lane (up to 256 results) or per
+ * wavefront, order (threshold 2^19 per lane), with a handler that takes pairs
+ * for RTS_HANDLER_COLLECT and one that only counts for RTS_HANDLER_COUNT. With
+ * `apply` set, it stores the fastest plans in the index for this
  * (predicate, query kind); later queries of that kind, and the batches of
- * rts_serve_run, use it for every setting their config leaves on auto. The
+ * rts_serve_run, use them for every setting their config leaves on auto. The
  * plan survives rts_index_clear. Results are identical under every plan;
  * only the time differs. `queries` is rts_point* when `points` is 1, else
  * rts_envelope* (rts_point_d* / rts_envelope_d* for a double index), in
@@ -400,11 +406,12 @@ typedef struct rts_tune_config {
 } rts_tune_config;
 
 typedef struct rts_tune_result {
-  uint32_t leaf_size;      /* the winner */
-  uint32_t traversal;      /* RTS_TRAVERSAL_THREAD or RTS_TRAVERSAL_WAVE */
+  uint32_t leaf_size;      /* the fastest of handlers' calls */
+  uint32_t traversal;      /* the winner: RTS_TRAVERSAL_THREAD or RTS_TRAVERSAL_WAVE */
   uint32_t sort_queries;   /* 1 = Morton-ordered, 2 = input order; 0 = not tuned (the whole
                               set was too large to time), the call's size decides */
-  uint32_t plans;          /* plans timed */
+  uint32_t plans;          /* plans of handlers' calls timed (the library's own: one per
+                              traversal and order) */
   uint64_t sample;         /* queries in the sample */
   uint64_t sample_results; /* results of the sample */
   double best_ms;          /* the winner's time over the sample */

@@ -263,7 +263,7 @@ void QueryWithKind(rts_index* index, int pred, const void* queries, uint64_t n, 
 
 // Runs `queries` (n points or envelopes, floats for a float index, doubles
 // for a double one, in device or pinned memory) against `index` with handler
-// `h` on `stream`, under the plan the library would run the same call under
+// `h` on `stream`, under the index's plan for such calls
 // (rts_index_query_plan: traversal mode, Morton ordering, leaf-range size);
 // `traversal` other than RTS_TRAVERSAL_AUTO overrides its mode. Throws
 // rtspatial::Exception on a bad argument or a failed launch; rts_index_sync

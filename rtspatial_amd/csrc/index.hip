@@ -818,34 +818,49 @@ int order_queries(rts_index* ix, const void* queries, uint64_t nq, bool points, 
   return RTS_OK;
 }
 
-// How one query call runs: traversal mode, query ordering, leaf-range size.
+// How one query call runs: traversal mode, query ordering and, of handlers'
+// calls, the leaf-range size.
 struct Plan {
   int traversal;
   bool sort;
   uint32_t leaf_size;
 };
 
-// The plan of a query call. Explicit config settings win; a plan stored by
-// rts_index_autotune fills the settings left on auto; otherwise: one query
-// per wavefront where queries have many results (envelope intersects /
-// within), one per octet of lanes otherwise (points, envelope contains), and
-// Morton ordering of wavefront batches of 64K queries or more (neighbouring
-// waves, which take consecutive queries on one XCD, share that XCD's L2: the
-// 10M x 1M join counts in 4.6 ms with the order and 7.7 ms without). Octet
-// walks keep the input order: ordering 1M points costs 0.11 ms and made their
-// walk no faster at 1M (2.01 against 1.36 ms for 10M points), 10M (2.61
-// against 1.88) and 60M boxes (4.06 against 3.79); at 100M boxes it gains 3%.
 // Wavefront calls of at least this many queries are Morton-ordered unless a
 // tuning moved the threshold (TunedPlan::sort_min_n).
 constexpr uint64_t kSortMinQueries = 65536;
+// The same of handlers' calls with a query per lane. Lanes of a wave share
+// their descent, which pays for the sort from about here on: 1M points on 1M
+// boxes take 0.33 ms in order and 0.55 without, on 10M 0.56 and 0.72; 512k 0.22
+// against 0.30 and 0.36 against 0.39 (on 100k boxes 0.19 and 0.16); 256k 0.17
+// against 0.14 and 0.22 against 0.19. Data-contains-query calls alike.
+constexpr uint64_t kLaneSortMinQueries = 1ull << 19;
+// The size rule of a walk: calls of at least this many queries are ordered.
+uint64_t order_rule(int traversal, bool handler) {
+  if (traversal == RTS_TRAVERSAL_WAVE) return kSortMinQueries;
+  return handler ? kLaneSortMinQueries : UINT64_MAX;  // octets: never
+}
 // The autotuner times query ordering on the whole query set up to this size.
 constexpr uint64_t kOrderTuneQueries = 1ull << 22;
 
-Plan plan_query(const rts_index* ix, int pred, bool points, uint64_t nq) {
-  // Segment queries (kPredLine) are not tuned: they take the config or the defaults.
+// The plan of a query call: explicit config settings win, a plan stored by
+// rts_index_autotune fills the settings left on auto, then the defaults. One
+// query per wavefront where queries have many results (envelope intersects /
+// within), and one per octet of lanes otherwise (points, envelope contains).
+// Wavefront calls of kSortMinQueries are Morton-ordered (neighbouring waves,
+// which take consecutive queries on one XCD, share that XCD's L2: the 10M x 1M
+// join counts in 4.6 ms with the order and 7.7 ms without); octet walks keep
+// the input order: ordering 1M points costs 0.11 ms and made their walk no
+// faster at 1M (2.01 against 1.36 ms for 10M points), 10M (2.61 against 1.88)
+// and 60M boxes (4.06 against 3.79); at 100M boxes it gains 3%.
+// A handler's calls (`handler`: kernels compiled around it, on the binary tree)
+// go one query per lane where the library's go one per octet.
+// Segment queries (kPredLine) are not tuned: they take the config or the defaults.
+Plan plan_query(const rts_index* ix, int pred, bool points, uint64_t nq, bool handler = false) {
   static const rts_index::TunedPlan kUntuned{};
   const rts_index::TunedPlan& t =
-      pred == kPredLine ? kUntuned : ix->tuned[pred][points ? 1 : 0];
+      pred == kPredLine ? kUntuned
+                        : (handler ? ix->handler_tuned : ix->tuned)[pred][points ? 1 : 0];
   Plan p;
   if (ix->cfg.traversal == RTS_TRAVERSAL_THREAD || ix->cfg.traversal == RTS_TRAVERSAL_WAVE)
     p.traversal = (int)ix->cfg.traversal;
@@ -858,8 +873,8 @@ Plan plan_query(const rts_index* ix, int pred, bool points, uint64_t nq) {
   else if (t.valid && t.sort_tuned)
     p.sort = nq >= t.sort_min_n;
   else
-    p.sort = p.traversal == RTS_TRAVERSAL_WAVE && nq >= kSortMinQueries;
-  p.leaf_size = t.valid ? t.leaf_size : ix->cfg.leaf_size;
+    p.sort = nq >= order_rule(p.traversal, handler);
+  p.leaf_size = handler && t.valid ? t.leaf_size : ix->cfg.leaf_size;
   return p;
 }
 
@@ -919,7 +934,6 @@ int run_plan(rts_index* ix, const Plan& plan, int pred, const void* queries, uin
     for (const TreeView& tv : trees) {
       if (tv.n == 0) continue;
       ql.tree = tv;
-      ql.tree.leaf_size = plan.leaf_size;
       if (trav == RTS_TRAVERSAL_THREAD) {
         PhaseToken ph = phase_begin(RTS_PHASE_TRAVERSE, stream);
         RTS_HIP(launch_query(ql, stream));
@@ -1017,17 +1031,180 @@ struct TuneBuffers {
   void* sample = nullptr;
   rts_pair* pairs = nullptr;
   rts_pair* all_pairs = nullptr;  // results of the whole query set (ordering runs)
+  uint32_t* sink = nullptr;       // handlers' calls: a word per query
   char* small = nullptr;  // [0, 24): rts_dev_queue, [32, 40): counter, [40, 64): a second queue
   hipEvent_t ev[2] = {nullptr, nullptr};
   ~TuneBuffers() {
     if (sample) (void)hipFree(sample);
     if (pairs) (void)hipFree(pairs);
     if (all_pairs) (void)hipFree(all_pairs);
+    if (sink) (void)hipFree(sink);
     if (small) (void)hipFree(small);
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
   }
 };
+
+// The fastest of a kind of calls' plans.
+struct Tuned {
+  Plan winner{};
+  double best = 1e300, default_ms = 0;  // on the sample
+  uint32_t plans = 0;
+  bool order_tuned = false, order = false;
+};
+
+// Times the plans of one kind of calls over a sample of the queries, and with
+// `whole_set` the best of each traversal mode on all of them in both orders (a
+// sample of 32k queries does not fill the chip by lanes: 200k windows of 80
+// results take 0.46 ms so and 0.71 by wavefronts, 32k the other way round). `run(plan, all)` queues
+// a call on the sample or on all queries (all = true); `fits(&ok)` tells, after
+// a call on all queries, whether its results had room. A time is the fastest
+// of `reps` runs, after an untimed one when the traversal mode has not run yet
+// (its kernels then load and warm up); a plan whose first run is already 3x
+// slower than the best so far is not repeated.
+template <typename Run, typename Fits>
+int tune_plans(const rts_tune_config& cfg, uint32_t leaf_sizes, const Plan& base, bool try_other,
+               bool sample_is_all, bool whole_set, hipEvent_t* ev, hipStream_t stream, Run&& run,
+               Fits&& fits, Tuned* out) {
+  Tuned& t = *out;
+  bool warm[3] = {false, false, false};
+  auto time_on = [&](const Plan& p, bool all, double best, double* ms_out) -> int {
+    float ms = 0.0f;
+    double fastest = 1e300;
+    const uint32_t r0 = warm[p.traversal] ? 1u : 0u;
+    warm[p.traversal] = true;
+    for (uint32_t r = r0; r <= cfg.reps; ++r) {
+      RTS_HIP(hipEventRecord(ev[0], stream));
+      const int e = run(p, all);
+      if (e) return e;
+      RTS_HIP(hipEventRecord(ev[1], stream));
+      RTS_HIP(hipEventSynchronize(ev[1]));
+      RTS_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
+      if (r == r0 && ms > 3.0 * best) {
+        fastest = ms;
+        break;
+      }
+      if (r > 0) fastest = std::min(fastest, (double)ms);
+    }
+    *ms_out = fastest;
+    return RTS_OK;
+  };
+  int rc = time_on(base, false, t.best, &t.default_ms);
+  if (rc) return rc;
+  t.best = t.default_ms;
+  t.winner = base;
+  t.plans = 1;
+  Plan mode_plan[3]{};  // by traversal: the fastest on the sample
+  double mode_best[3] = {1e300, 1e300, 1e300};
+  mode_plan[base.traversal] = base;
+  mode_best[base.traversal] = t.default_ms;
+  // Traversal modes in the outer loop: a mode whose first plan is already 4x
+  // slower than the best is not tried with the other leaf sizes or orders.
+  // Query ordering is only tuned here when the sample is the whole query set:
+  // a strided sample has none of the set's locality, which is what Morton
+  // ordering exploits, so otherwise the order stays with the call's size rule.
+  const int other =
+      base.traversal == RTS_TRAVERSAL_WAVE ? (int)RTS_TRAVERSAL_THREAD : (int)RTS_TRAVERSAL_WAVE;
+  for (int trav : {base.traversal, other}) {
+    if (trav == other && !try_other) continue;
+    bool first = true;
+    for (uint32_t k = 0; k <= 6; ++k) {
+      if (!(leaf_sizes & (1u << k))) continue;
+      for (bool sort : {false, true}) {
+        if (!sample_is_all && sort != base.sort) continue;
+        const Plan p{trav, sort, leaf_sizes == 1u ? base.leaf_size : 1u << k};
+        if (p.traversal == base.traversal && p.sort == base.sort && p.leaf_size == base.leaf_size)
+          continue;
+        double ms = 0;
+        rc = time_on(p, false, t.best, &ms);
+        if (rc) return rc;
+        ++t.plans;
+        if (ms < t.best) {
+          t.best = ms;
+          t.winner = p;
+        }
+        if (ms < mode_best[trav]) {
+          mode_best[trav] = ms;
+          mode_plan[trav] = p;
+        }
+        if (first && ms > 4.0 * t.best) goto next_mode;
+        first = false;
+      }
+    }
+  next_mode:;
+  }
+  t.order_tuned = sample_is_all;
+  t.order = t.winner.sort;
+  if (whole_set) {
+    // Both orders of each mode that is within reach, with full repetitions.
+    Plan best_plan = t.winner;
+    double best_ms = 1e300, far = 4.0 * t.best;
+    bool ok = true;
+    for (int trav : {base.traversal, other}) {
+      if (mode_best[trav] > far) continue;
+      for (int o = 0; o < 2 && ok; ++o) {
+        Plan p = mode_plan[trav];
+        p.sort = o == 1;
+        double ms = 0;
+        rc = time_on(p, true, 1e300, &ms);
+        if (!rc) rc = fits(&ok);
+        if (rc) return rc;
+        if (ms < best_ms) {
+          best_ms = ms;
+          best_plan = p;
+        }
+      }
+    }
+    if (ok) {
+      t.winner = best_plan;
+      t.best = mode_best[best_plan.traversal];
+      t.order_tuned = true;
+      t.order = best_plan.sort;
+      t.plans += 2;
+    }
+  }
+  return RTS_OK;
+}
+
+// A tuned plan as it is stored. The ordering measured at n queries moves the
+// size rule's threshold: calls of at least min(n, the rule's size) are ordered
+// when ordering won, calls of at most max(n, ...) are not when it lost.
+rts_index::TunedPlan stored_plan(const Tuned& t, uint64_t n, bool handler) {
+  rts_index::TunedPlan p;
+  p.valid = true;
+  p.traversal = (uint32_t)t.winner.traversal;
+  p.sort_tuned = t.order_tuned;
+  const uint64_t rule = order_rule(t.winner.traversal, handler);
+  p.sort_min_n = t.order ? std::min(n, rule) : std::max(n + 1, rule);
+  p.leaf_size = t.winner.leaf_size;
+  return p;
+}
+
+// Runs one call of the handlers' kernels under `plan`, ordering included.
+int run_handler(rts_index* ix, const Plan& plan, int pred, const void* queries, uint64_t nq,
+                bool points, bool f64, bool pairs, uint32_t* sink, hipStream_t stream) {
+  Scratch block;
+  HandlerCall c{};
+  c.tree = tree_view(ix);
+  c.tree.leaf_size = plan.leaf_size;
+  c.pred = pred;
+  c.points = points;
+  c.f64 = f64;
+  c.wave = plan.traversal == RTS_TRAVERSAL_WAVE;
+  c.pairs = pairs;
+  c.queries = queries;
+  c.n = (uint32_t)nq;
+  c.sink = sink;
+  if (plan.sort) {
+    const size_t keys_bytes = align_up(4 * nq * sizeof(uint32_t));
+    RTS_HIP(block.lease(keys_bytes + sort_scratch_bytes(nq), stream));
+    const int rc = order_queries(ix, queries, nq, points, f64, block.get(),
+                                 block.get() + keys_bytes, stream, &c.order);
+    if (rc) return rc;
+  }
+  RTS_HIP(launch_handler_call(c, stream));
+  return RTS_OK;
+}
 
 }  // namespace
 
@@ -1154,8 +1331,9 @@ int rts_index_query_plan(rts_index* ix, rts_predicate pred, int points, uint64_t
   RTS_CHECK_ARG(points >= RTS_QUERY_ENVELOPES && points <= RTS_QUERY_LINES,
                 "rts_index_query_plan: unknown query kind");
   std::lock_guard<std::mutex> lk(ix->mu);
-  const Plan p = points == RTS_QUERY_LINES ? plan_query(ix, kPredLine, false, n)
-                                           : plan_query(ix, pred, points == RTS_QUERY_POINTS, n);
+  const Plan p = points == RTS_QUERY_LINES
+                     ? plan_query(ix, kPredLine, false, n, true)
+                     : plan_query(ix, pred, points == RTS_QUERY_POINTS, n, true);
   out->traversal = (uint32_t)p.traversal;
   out->sort_queries = p.sort ? 1u : 2u;
   out->leaf_size = p.leaf_size;
@@ -1383,151 +1561,92 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
     arg = tb.small;
   }
 
-  // Time one plan: the fastest of `reps` runs, after an untimed one when
-  // the plan's traversal mode has not run yet (its kernels then load and
-  // warm up). A plan whose first run is already 3x slower than the best so
-  // far is not repeated.
-  double best = 1e300;
-  bool warm[3] = {false, false, false};
-  auto time_on = [&](const Plan& p, const void* qs, uint64_t qn, void* qarg,
-                     double* ms_out) -> int {
-    float ms = 0.0f;
-    double fastest = 1e300;
-    const uint32_t r0 = warm[p.traversal] ? 1u : 0u;
-    warm[p.traversal] = true;
-    for (uint32_t r = r0; r <= cfg.reps; ++r) {
-      RTS_HIP(hipMemsetAsync(counter, 0, sizeof(*counter), stream));
-      RTS_HIP(hipEventRecord(tb.ev[0], stream));
-      int e = run_plan(ix, p, pred, qs, qn, pts, f64, handler, qarg, stream);
-      if (e) return e;
-      RTS_HIP(hipEventRecord(tb.ev[1], stream));
-      RTS_HIP(hipEventSynchronize(tb.ev[1]));
-      RTS_HIP(hipEventElapsedTime(&ms, tb.ev[0], tb.ev[1]));
-      if (r == r0 && ms > 3.0 * best) {
-        fastest = ms;
-        break;
-      }
-      if (r > 0) fastest = std::min(fastest, (double)ms);
-    }
-    *ms_out = fastest;
-    return RTS_OK;
-  };
-  auto time_plan = [&](const Plan& p, double* ms_out) -> int {
-    return time_on(p, tb.sample, m, arg, ms_out);
-  };
-
-  double default_ms = 0;
-  rc = time_plan(base, &default_ms);
-  if (rc) return rc;
-  best = default_ms;
-  Plan winner = base;
-  uint32_t plans = 1;
-  // Traversal modes in the outer loop: a mode whose first plan is already 4x
-  // slower than the best is not tried with the other leaf sizes or orders
-  // (per-lane traversal of queries with thousands of results each, say).
-  // Query ordering is only tuned when the sample is the whole query set: a
-  // strided sample has none of the set's locality, which is what Morton
-  // ordering exploits, so otherwise the order stays with the call's size rule.
-  const bool whole = m == n;
-  const int other =
-      base.traversal == RTS_TRAVERSAL_WAVE ? (int)RTS_TRAVERSAL_THREAD : (int)RTS_TRAVERSAL_WAVE;
-  // A lane emits its query's results one per step, while a wavefront scans
-  // 512 leaves per step: queries averaging more than kLaneMaxResults results
-  // are not timed one per lane (on the 10M-box index the per-lane probe of
-  // intersects queries with ~1e4 results each took 446 ms against 6 ms).
-  constexpr double kLaneMaxResults = 256.0;
-  const bool lane_hopeless = (double)total > kLaneMaxResults * (double)m;
-  for (int trav : {base.traversal, other}) {
-    if (trav == RTS_TRAVERSAL_THREAD && lane_hopeless) continue;
-    bool first = true;
-    for (uint32_t k = 1; k <= 6; ++k) {
-      if (!(cfg.leaf_sizes & (1u << k))) continue;
-      for (bool sort : {false, true}) {
-        if (!whole && sort != base.sort) continue;
-        Plan p{trav, sort, 1u << k};
-        if (p.traversal == base.traversal && p.sort == base.sort && p.leaf_size == base.leaf_size)
-          continue;
-        double ms = 0;
-        rc = time_plan(p, &ms);
-        if (rc) return rc;
-        ++plans;
-        if (ms < best) {
-          best = ms;
-          winner = p;
-        }
-        if (first && ms > 4.0 * best) goto next_mode;
-        first = false;
-      }
-    }
-  next_mode:;
-  }
   // Query ordering pays through the walks' cache locality, which a strided
   // sample does not have. When the whole set is cheap to run -- at most
   // kOrderTuneQueries queries and, going by the sample, at most kMaxPairs
   // results -- the winning plan is timed on the whole set in both orders.
-  // (On the 100k x 100k point query, ordering cost 0.088 ms and saved
-  // 0.022 ms of traversal: 0.164 against 0.100 ms per call.)
-  bool order_tuned = whole, order = winner.sort;
+  const bool sample_is_all = m == n;
   const double est_all = (double)total * (double)n / (double)std::max<uint64_t>(m, 1);
-  if (!whole && n <= kOrderTuneQueries && ix->cfg.coord != RTS_COORD_F64_AS_F32 &&
-      est_all <= (double)kMaxPairs) {
-    void* all_arg = counter;
-    uint64_t cap = 0;
-    if (handler == RTS_HANDLER_COLLECT) {
-      cap = (uint64_t)(est_all * 1.5) + 4096;
-      RTS_HIP(dev_alloc(&tb.all_pairs, cap));
-      rts_dev_queue q{tb.all_pairs, cap, counter};
-      RTS_HIP(hipMemcpyAsync(tb.small + 40, &q, sizeof(q), hipMemcpyHostToDevice, stream));
-      all_arg = tb.small + 40;
-    }
-    double ms_in[2] = {0, 0};
-    bool fits = true;
-    // Both orders get their full repetitions (the early exit compares
-    // against the sample's best time).
-    const double sample_best = best;
-    best = 1e300;
-    for (int o = 0; o < 2 && fits; ++o) {
-      Plan p = winner;
-      p.sort = o == 1;
-      rc = time_on(p, queries, n, all_arg, &ms_in[o]);
-      if (rc) return rc;
-      if (handler == RTS_HANDLER_COLLECT) {
+  const bool whole_set = !sample_is_all && n <= kOrderTuneQueries &&
+                         ix->cfg.coord != RTS_COORD_F64_AS_F32 && est_all <= (double)kMaxPairs;
+  const double mean_results = (double)total / (double)std::max<uint64_t>(m, 1);
+  void* all_arg = counter;
+  uint64_t all_cap = 0;
+  if (whole_set && handler == RTS_HANDLER_COLLECT) {
+    all_cap = (uint64_t)(est_all * 1.5) + 4096;
+    RTS_HIP(dev_alloc(&tb.all_pairs, all_cap));
+    rts_dev_queue q{tb.all_pairs, all_cap, counter};
+    RTS_HIP(hipMemcpyAsync(tb.small + 40, &q, sizeof(q), hipMemcpyHostToDevice, stream));
+    all_arg = tb.small + 40;
+  }
+  // Octets are not timed where they collect more than 256 results a query: 32k
+  // windows of 260 results on 10M boxes take 0.24 ms by octets and 0.19 by
+  // waves, of 1020 0.85 and 0.28, of 4030 3.3 and 0.60 (of 66 0.077 and 0.087).
+  // Counting, octets lead up to some 2500 results and lose little beyond (4030:
+  // 0.18 and 0.16).
+  constexpr double kOctetMaxResults = 256.0;
+  const bool octets = handler == RTS_HANDLER_COUNT || mean_results <= kOctetMaxResults;
+  Tuned own;
+  rc = tune_plans(
+      cfg, 1u, base, base.traversal == RTS_TRAVERSAL_THREAD || octets, sample_is_all, whole_set,
+      tb.ev, stream,
+      [&](const Plan& p, bool all) -> int {
+        RTS_HIP(hipMemsetAsync(counter, 0, sizeof(*counter), stream));
+        return run_plan(ix, p, pred, all ? queries : tb.sample, all ? n : m, pts, f64, handler,
+                        all ? all_arg : arg, stream);
+      },
+      [&](bool* ok) -> int {
+        if (handler != RTS_HANDLER_COLLECT) return RTS_OK;
         unsigned long long got = 0;
         RTS_HIP(hipMemcpyAsync(&got, counter, sizeof(got), hipMemcpyDeviceToHost, stream));
         RTS_HIP(hipStreamSynchronize(stream));
-        fits = got <= cap;
-      }
-    }
-    best = sample_best;
-    if (fits) {
-      order_tuned = true;
-      order = ms_in[1] < ms_in[0];
-      plans += 2;
-    }
+        *ok = got <= all_cap;
+        return RTS_OK;
+      },
+      &own);
+  if (rc) return rc;
+
+  // The same of handlers' calls, which walk the binary tree (over the main
+  // tree's leaves; one made for this goes again). A query per lane is not timed
+  // where queries average more than 256 results: a lane emits one result per
+  // step, while a wavefront scans 512 leaves (on a 10M-box index intersects
+  // queries with ~1e4 results each took 446 ms per lane and 6 per wavefront).
+  constexpr double kLaneMaxResults = 256.0;
+  const Plan handler_base = plan_query(ix, pred, pts, n, true);
+  RTS_HIP(dev_alloc(&tb.sink, whole_set ? n : m));
+  RTS_HIP(launch_fill_u32(tb.sink, 0u, whole_set ? n : m, stream));
+  const bool made = ix->bcap == 0;
+  rc = ensure_binary(ix, stream);
+  Tuned han;
+  if (!rc)
+    rc = tune_plans(
+        cfg, cfg.leaf_sizes & 0x7Eu, handler_base,
+        handler_base.traversal == RTS_TRAVERSAL_THREAD || mean_results <= kLaneMaxResults,
+        sample_is_all, whole_set, tb.ev, stream,
+        [&](const Plan& p, bool all) -> int {
+          return run_handler(ix, p, pred, all ? queries : tb.sample, all ? n : m, pts, f64,
+                             handler == RTS_HANDLER_COLLECT, tb.sink, stream);
+        },
+        [](bool*) -> int { return RTS_OK; }, &han);
+  if (made) {
+    (void)hipStreamSynchronize(stream);
+    free_binary(ix);
   }
+  if (rc) return rc;
   rc = check_device_error(ix);
   if (rc) return rc;
   if (cfg.apply) {
-    rts_index::TunedPlan& t = ix->tuned[pred][pts ? 1 : 0];
-    t.valid = true;
-    t.traversal = (uint32_t)winner.traversal;
-    t.sort = order;
-    t.sort_tuned = order_tuned;
-    // The ordering measured at n queries moves the size rule's threshold:
-    // calls of at least min(n, the rule's size) are ordered when ordering
-    // won, calls of at most max(n, ...) are not when it lost.
-    t.sort_min_n = order ? std::min<uint64_t>(n, kSortMinQueries)
-                         : std::max<uint64_t>(n + 1, kSortMinQueries);
-    t.leaf_size = winner.leaf_size;
+    ix->tuned[pred][pts ? 1 : 0] = stored_plan(own, n, false);
+    ix->handler_tuned[pred][pts ? 1 : 0] = stored_plan(han, n, true);
   }
-  out->leaf_size = winner.leaf_size;
-  out->traversal = (uint32_t)winner.traversal;
-  out->sort_queries = order_tuned ? (order ? 1 : 2) : 0;
-  out->plans = plans;
+  out->leaf_size = han.winner.leaf_size;
+  out->traversal = (uint32_t)own.winner.traversal;
+  out->sort_queries = own.order_tuned ? (own.order ? 1 : 2) : 0;
+  out->plans = han.plans;
   out->sample = m;
   out->sample_results = total;
-  out->best_ms = best;
-  out->default_ms = default_ms;
+  out->best_ms = own.best;
+  out->default_ms = own.default_ms;
   return RTS_OK;
 }
 

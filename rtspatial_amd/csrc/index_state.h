@@ -98,16 +98,17 @@ struct rts_index {
 
   // Plans stored by rts_index_autotune, per [predicate][points]; kept until
   // the next tuning of that kind (Clear keeps them: they describe the
-  // workload, not the stored boxes).
+  // workload, not the stored boxes). Those of the library's own walks and those
+  // of the binary tree's, which handlers run, are timed apart.
   struct TunedPlan {
     bool valid = false;
     uint32_t traversal = 0;
-    bool sort = false;
     bool sort_tuned = false;  // ordering was timed on the whole query set
     uint64_t sort_min_n = 0;  // with sort_tuned: calls of at least this many queries are ordered
-    uint32_t leaf_size = 0;
+    uint32_t leaf_size = 0;   // handlers' plans only
   };
   TunedPlan tuned[3][2];
+  TunedPlan handler_tuned[3][2];
 
   bool f64() const { return cfg.coord != RTS_COORD_F32; }
 };

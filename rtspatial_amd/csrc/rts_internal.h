@@ -195,6 +195,19 @@ enum { kPhaseCount = 0, kPhaseCountSink = 1, kPhaseWrite = 2, kPhaseWriteStaged 
 hipError_t launch_query_wave(const QueryLaunch& q, const WaveArgs& a, int phase,
                              hipStream_t stream);
 
+// handler_tune.hip: a call of the handlers' kernels, for the autotuner.
+struct HandlerCall {
+  TreeView tree;  // with a binary tree
+  int pred;
+  bool points, f64;
+  bool wave, pairs;       // traversal; whether the handler takes pairs
+  const void* queries;
+  uint32_t n;
+  const uint32_t* order;  // optional permutation
+  uint32_t* sink;         // n words
+};
+hipError_t launch_handler_call(const HandlerCall& c, hipStream_t stream);
+
 // scan.hip
 size_t scan_scratch_bytes(uint64_t n);
 // offsets[i] = counts[0] + ... + counts[i-1]; *total = the sum of all counts.

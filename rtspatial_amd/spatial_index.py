@@ -301,9 +301,11 @@ class SpatialIndex:
     def Autotune(self, predicate, queries, collect=True, sample=32768, leaf_sizes=(4, 8, 16, 32),
                  reps=3, apply=True, stream=None):
         """Times the query over a strided sample of `queries` under every
-        plan (leaf size, per-octet or per-wavefront traversal, Morton or input
-        order) and, with `apply`, keeps the fastest for later queries of this
-        predicate and query kind. Returns the choice and the sample timings."""
+        plan (per-octet or per-wavefront traversal, Morton or input order) and,
+        with `apply`, keeps the fastest for later queries of this predicate and
+        query kind; also the plans of calls with caller-compiled handlers
+        (leaf size, traversal, order). Returns the choice and the sample
+        timings."""
         _check_array(queries, None, self.coord_t, "Autotune")
         if queries.dim() != 2 or queries.shape[1] not in (2, 4):
             raise ValueError("Autotune: queries must be [n, 2] points or [n, 4] envelopes")

@@ -519,13 +519,16 @@ hipError_t launch_wave_f(const QueryLaunch& q, const WaveArgs& a, int phase, hip
       return hipErrorInvalidValue;
     }
     default: {
-      if (a.log.entries) {
-        auto* k = &k_window_write<PRED, POINTS, F64>;
-        const uint32_t most = device_cus() * kWindowWaves;
-        uint32_t blocks = q.n < most ? std::min(most, 512 + 4 * q.n) : most;
-        blocks = (blocks + kXcds - 1) / kXcds * kXcds;
-        hipLaunchKernelGGL(k, dim3(blocks), dim3(kWave), 0, stream, q, a);
-        break;
+      // (Segment walks log nothing that is written: they are staged, or walk again.)
+      if constexpr (PRED != kPredLine) {
+        if (a.log.entries) {
+          auto* k = &k_window_write<PRED, POINTS, F64>;
+          const uint32_t most = device_cus() * kWindowWaves;
+          uint32_t blocks = q.n < most ? std::min(most, 512 + 4 * q.n) : most;
+          blocks = (blocks + kXcds - 1) / kXcds * kXcds;
+          hipLaunchKernelGGL(k, dim3(blocks), dim3(kWave), 0, stream, q, a);
+          break;
+        }
       }
       auto* k = &k_wave_write<PRED, POINTS, F64>;
       static const uint32_t resident = resident_waves(k);

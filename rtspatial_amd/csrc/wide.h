@@ -512,9 +512,19 @@ __device__ __forceinline__ void oct_replay(const TreeView& t, const uint2* entri
 
 // Emits the logged results [lo, hi) of one query. Blocks are taken 8 at a time,
 // one per octet: each lane stores the result its mask bit names, and the
-// wave's stores of a round are consecutive pairs. Runs of leaves are copied 64
-// (4 x 64 while they last) at a time. The next 64 entries are in flight while
-// these are emitted.
+// wave's stores of a round are consecutive pairs. Runs of up to 64 leaves (most
+// are nodes of 64) are copied kShortRuns at a time, with as many loads of ids in
+// flight; longer ones 4 x 64 leaves at a time. The next 64 entries are in flight
+// while these are emitted.
+// One run at a time, each waiting for its own load, held large queries' write
+// passes back. Served intersects requests, 9e10 pairs on 10M boxes, one batch in
+// flight: 340-391 ms of write passes by where the arena lies, now 304-310 (the
+// walk that logs replaced took 307); within requests 288-331, now 265-302 (298);
+// four at a time lies halfway. Windows in the walks' Morton order instead of the
+// output's, which fetch a third as much, gain nothing here, and on a million
+// boxes or a clustered set they are 1.1-2.4x slower: neighbouring waves then
+// write far apart.
+constexpr int kShortRuns = 8;
 template <typename Emit>
 __device__ void wide_replay(const TreeView& t, const RangeLog& lg, uint32_t lo, uint32_t hi,
                             const uint32_t qid, const Emit& emit) {
@@ -552,6 +562,26 @@ __device__ void wide_replay(const TreeView& t, const RangeLog& lg, uint32_t lo, 
         if ((hm >> r) & 1u) emit(at[r], gid[r], qid);
     }
     uint64_t rm = ballot(run && off < hi && off + cnt > lo);
+    uint64_t sm = rm & ballot(cnt <= (uint32_t)kWave);
+    rm &= ~sm;
+    while (sm) {
+      uint32_t gid[kShortRuns], at[kShortRuns];
+      uint32_t hm = 0;
+#pragma unroll
+      for (int u = 0; u < kShortRuns; u++) {
+        const int l = sm ? __builtin_ctzll(sm) : 0;
+        const uint32_t f = readlane_u32(en.x, l) & ~kLogRange;
+        const uint32_t c = sm ? readlane_u32(cnt, l) : 0u;
+        sm &= sm - 1;  // (zero stays zero)
+        at[u] = readlane_u32(off, l) + lane;
+        const bool hit = lane < c && at[u] >= lo && at[u] < hi;
+        hm |= (hit ? 1u : 0u) << u;
+        gid[u] = hit ? t.leaf_ids[f + lane] : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < kShortRuns; u++)
+        if ((hm >> u) & 1u) emit(at[u], gid[u], qid);
+    }
     while (rm) {
       const int l = __builtin_ctzll(rm);
       rm &= rm - 1;

@@ -94,12 +94,4 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
   return v;
 }
 
-// Device-scope relaxed atomics for flags that carry their own payload.
-__device__ __forceinline__ uint32_t load_relaxed_agent(const uint32_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void store_relaxed_agent(uint32_t* p, uint32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 }  // namespace rts

@@ -1,8 +1,9 @@
-// Device-side LBVH traversal cores shared by the library's query kernels
-// (one query per lane or per wavefront, per request or in persistent
-// batches) and by kernels a caller compiles around its own result handler
-// (rtspatial/device/query.h). Results leave through an emitter:
-// emit(k, geom_id, query_id) is called for the k-th result of a query.
+// Queries, their exact tests and emitters, shared by the library's kernels and
+// by kernels a caller compiles around its own result handler
+// (rtspatial/device/query.h), and the latter's walks of the binary tree, one
+// query per lane or per wavefront (the library's own walk the packed tree).
+// Results leave through an emitter: emit(k, geom_id, query_id) is called for
+// the k-th result of a query.
 //
 // Node tests are necessary conditions of the leaf predicate on exact FP32
 // bounds, so pruning never drops a true pair; every reported pair passed the
@@ -215,9 +216,9 @@ __device__ __forceinline__ bool leaf_test(const TreeView& t, uint32_t leaf, cons
 
 // A result pair stored with a non-temporal hint: the walk never reads its
 // output back, and streaming it past the caches keeps the leaf ids it reads
-// resident (2e9 pairs of 10M boxes x 200k queries are written in 9.0 ms with
-// ordinary stores 10.1). For stores that a wave makes side by side: parts of a
-// line that come apart go to memory twice.
+// resident (2e9 pairs of 10M boxes x 200k queries are written in 9.0 ms, with
+// ordinary stores in 10.1). It suits stores that a wave makes side by side:
+// where a line's parts are stored apart, the line goes to memory twice.
 static_assert(sizeof(rts_pair) == 8 && offsetof(rts_pair, geom_id) == 0, "pair layout");
 __device__ __forceinline__ void store_pair(rts_pair* p, uint32_t geom_id, uint32_t query_id) {
   const uint64_t bits = ((uint64_t)query_id << 32) | geom_id;  // rts_pair: geom_id first
@@ -308,9 +309,9 @@ __device__ __forceinline__ void load_q(const void* queries, bool, uint32_t i, Qu
 constexpr int kWaveStack = 256;     // LDS stack entries per wave
 constexpr int kWaveRanges = 256;    // leaf ranges per wave before a scan
 // Scan once this many leaves are queued. Deferring the scan past one step's
-// 512 leaves leaves fewer part-filled final steps: on the 10M x 1M
-// intersects join 44.5 -> 42.4 ms per step (512 -> 2048; 4096 and 8192 no
-// better), segment join 12.81 -> 12.63 ms.
+// 512 leaves leaves fewer part-filled final steps: the 10M x 1M intersects
+// join, collected by this walk, 44.5 -> 42.4 ms per step (512 -> 2048; 4096 and
+// 8192 no better), the segment join 12.81 -> 12.63 ms.
 constexpr int kFlushLeaves = 2048;
 constexpr int kPerLane = 8;         // leaves per lane per scan step
 constexpr uint32_t kScanStep = kPerLane * kWave;

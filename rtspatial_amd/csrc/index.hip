@@ -321,9 +321,9 @@ int build_tree(rts_index* ix, hipStream_t stream) {
   return RTS_OK;
 }
 
-// Builds the delta tree over ids [n_main, n) alone: its own scene bounds,
-// Morton sort and hierarchy, in the tails of the shared arrays. The main tree
-// is left as it is (refitted first if a mutation left it pending).
+// Builds the delta tree over ids [n_main, n) alone: its own scene bounds and
+// Hilbert sort, in the tails of the shared arrays, and nodes of its own. The
+// main tree is left as it is (refitted first if a mutation left it pending).
 int build_delta(rts_index* ix, hipStream_t stream) {
   const uint64_t off = ix->n_main;
   const uint32_t nd = (uint32_t)(ix->n - off);
@@ -362,14 +362,16 @@ bool delta_ok(const rts_index* ix) {
          extra * 100 <= ix->n_main * (uint64_t)ix->cfg.insert_delta_pct;
 }
 
-// Under RTS_REBUILD_SAH, updates that give new envelopes to at least 1/200
-// of the tree's boxes since its last build mark it stale: a full build costs
-// ~1.5x a refit here (10M boxes: 2.8 vs 1.7 ms), while a refit over boxes
-// moved beyond their old extents leaves the tree slower to query. On the
-// served stream's 100k-box update batches (1% of 10M boxes, each moved by up
-// to 10x its size) the tree cost grew ~2% per batch and never reached the
-// 1.5x ratio; rebuilding instead raised saturated throughput from 27.8 to
-// 30.1 Mq/s.
+// Under RTS_REBUILD_SAH, updates that give new envelopes to at least 1/200 of
+// the tree's boxes since its last build mark it stale. A build takes 0.68 ms for
+// 10M boxes and bounding the tree again 0.05 (1M: 0.12 and 0.015), but boxes
+// moved by up to 10x their size slow every query until the next build: on 10M
+// skewed boxes with 1% of them moved, 1M points take 0.59 ms instead of 0.41 and
+// a join with 200k queries 1.29 instead of 1.17, with 5% 1.28 and 1.72, with 20%
+// 3.56 and 2.91 (uniform boxes, 1%: 0.30 instead of 0.22, 0.28 instead of 0.24;
+// with 0.4% 0.26 and 0.25). At 1/200 the 0.63 ms are back after some seven calls
+// of 1M points or ten such joins. (The tree cost grows by 5% with 0.4% of the
+// boxes moved, so sah_rebuild_ratio alone would rebuild at some 4%.)
 constexpr uint64_t kRebuildUpdateShare = 200;
 
 // Update and Delete only mark the tree: the refit (or rebuild) runs once, at

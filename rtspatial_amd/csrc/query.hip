@@ -460,16 +460,25 @@ void launch_persistent(K kernel, uint32_t resident, uint32_t group, const QueryL
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWave), 0, stream, q, a, group);
 }
 
-// Calls of at least kOctetTickets queries per wave run the octets first, 8 to a
-// ticket, and 16 once every wave gets one; smaller ones leave each wave up to
-// kFewQueries queries of its own, without tickets. (20k intersects queries of
-// 1000 results: 0.30 ms so, 0.36 with octets; 30k within queries of 20: 0.16
-// without octets, 0.09 with them.)
+// Calls of at least kOctetQueries queries per wave run the octets first, 8 to a
+// ticket, and 16 once every wave gets a ticket; smaller ones leave each wave up
+// to kFewQueries queries of its own, without tickets. How heavy the queries are
+// shows only on the device, so one line stands for all. Whole collecting calls
+// on 10M boxes, us, waves alone / octets first, by results per query:
+//              1        20       60       200       1000
+//     8k    51 / 44   48 / 51  51 / 67   59 / 100   87 / 125
+//    16k    64 / 46   65 / 58  69 / 73   79 / 150  132 / 200
+//    24k    73 / 49   77 / 62  82 / 76   97 / 159  175 / 230
+//    32k    99 / 51  112 / 66 121 / 81  141 / 184  250 / 277
+//    64k   139 / 69  149 / 92 168 / 124 205 / 294  407 / 482
+// (counting calls alike, 10M or 1M boxes). Up to the line light calls lose at
+// most a third by going without; beyond it they lose half, and the trial that
+// heavy ones pay for, some 70 us, becomes a smaller part of them.
 constexpr uint32_t kFewQueries = 4;
-constexpr uint32_t kOctetTickets = 3;
+constexpr uint32_t kOctetQueries = 3;
 uint32_t octet_group(uint32_t n) {
   const uint32_t waves = device_cus() * 32;
-  return n >= kGroup * waves ? kGroup : n >= kOctetTickets * waves ? 8u : 0u;
+  return n >= kGroup * waves ? kGroup : n >= kOctetQueries * waves ? 8u : 0u;
 }
 
 template <int PRED, bool POINTS, bool LOG, bool F64>

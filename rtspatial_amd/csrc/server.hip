@@ -355,10 +355,10 @@ int copy_out(Engine& E, const Chunk& c, const rts_pair* src, uint64_t cnt, hipSt
   return RTS_OK;
 }
 
-// Tile mode of a request: the serve config's traversal
-// if it names one, else the plan stored by rts_index_autotune for this
-// (predicate, query kind), else one query per wavefront for envelope
-// intersects / within and 64 per tile otherwise.
+// Tile mode of a request: the serve config's traversal if it names one, else
+// that of the plan stored by rts_index_autotune for this (predicate, query
+// kind), else one query per wavefront for envelope intersects / within and
+// tiles of 64, one query per octet at a time, otherwise.
 uint32_t tile_flags(const Engine& E, const rts_request& r) {
   if (is_ext(E.ix, r)) return kReqExt;
   const bool pts = r.points == kPoints;
@@ -377,8 +377,8 @@ uint32_t tile_flags(const Engine& E, const rts_request& r) {
 }
 
 // Range-log entries of a slot (8 bytes each): 192 per query of a full batch
-// (envelope queries of the served mix log a few hundred leaf ranges each; a
-// query past its wave's share is walked again), at most 2^30.
+// (envelope queries of the served mix log a few hundred blocks and runs of
+// leaves each; a query past its wave's share is walked again), at most 2^30.
 uint64_t serve_log_entries(uint64_t max_batch_queries) {
   return std::min<uint64_t>(max_batch_queries * 192, 1ull << 30);
 }

@@ -239,6 +239,15 @@ int build_binary(rts_index* ix, hipStream_t stream) {
   return RTS_OK;
 }
 
+// Waits for all work queued on the device, as freeing memory does: legal within
+// a Relaxed scope while a stream is captured, which hipDeviceSynchronize is not.
+// (An event after each build to wait for instead cost every build 5 us.)
+hipError_t wait_for_device() {
+  void* p = nullptr;
+  const hipError_t e = hipMalloc(&p, 256);
+  return e == hipSuccess ? hipFree(p) : e;
+}
+
 // Brings the binary tree over the main tree's leaves up to date for work on
 // `stream`; there is no delta tree (ensure_built with `single`).
 int ensure_binary(rts_index* ix, hipStream_t stream) {
@@ -256,7 +265,7 @@ int ensure_binary(rts_index* ix, hipStream_t stream) {
     if (aside) {
       if (!ix->bin_stream)
         RTS_HIP(hipStreamCreateWithFlags(&ix->bin_stream, hipStreamNonBlocking));
-      RTS_HIP(hipStreamWaitEvent(ix->bin_stream, ix->tree_done, 0));
+      RTS_HIP(wait_for_device());
     }
     const hipStream_t s = aside ? ix->bin_stream : stream;
     const int rc = build_binary(ix, s);
@@ -483,7 +492,6 @@ int ensure_built(rts_index* ix, hipStream_t stream, bool single) {
   }
   if (rc) return rc;
   ix->tree_captured = capturing(stream);
-  if (!ix->tree_captured) RTS_HIP(hipEventRecord(ix->tree_done, stream));
   return RTS_OK;
 }
 
@@ -547,7 +555,6 @@ int rts_index_create(const rts_config* cfg, rts_index** out) {
   RTS_HIP(hipHostMalloc(reinterpret_cast<void**>(&ix->h_cost), 4 * sizeof(double)));
   RTS_HIP(hipEventCreateWithFlags(&ix->ev_cost_build, hipEventDisableTiming));
   RTS_HIP(hipEventCreateWithFlags(&ix->ev_cost_refit, hipEventDisableTiming));
-  RTS_HIP(hipEventCreateWithFlags(&ix->tree_done, hipEventDisableTiming));
   RTS_HIP(hipEventCreateWithFlags(&ix->bin_done, hipEventDisableTiming));
   if (ix->cfg.preallocate && ix->cfg.max_geometries) {
     int rc = ensure_id_capacity(ix, ix->cfg.max_geometries, nullptr);
@@ -585,7 +592,6 @@ int rts_index_destroy(rts_index* ix) {
   if (ix->h_cost) (void)hipHostFree(ix->h_cost);
   if (ix->ev_cost_build) (void)hipEventDestroy(ix->ev_cost_build);
   if (ix->ev_cost_refit) (void)hipEventDestroy(ix->ev_cost_refit);
-  if (ix->tree_done) (void)hipEventDestroy(ix->tree_done);
   if (ix->bin_done) (void)hipEventDestroy(ix->bin_done);
   if (ix->bin_stream) (void)hipStreamDestroy(ix->bin_stream);
   if (ix->counted) workspace_index_end(ix->device);

@@ -52,14 +52,13 @@ struct rts_index {
   // does not queue the trees' builds again, so one taken on another stream than
   // the binary tree was queued on waits for that (bin_done), and one taken
   // while a graph is captured must not leave the tree to the graph's replay: it
-  // is then built at once on bin_stream, after what the trees were last built
-  // or refitted by (tree_done), unless that was captured too.
+  // is then built at once on bin_stream, after all work queued so far, unless
+  // the trees' own last build or refit was captured too.
   uint64_t bcap = 0;
   bool bin_valid = false;         // it has the current leaves' hierarchy
   bool bin_refit_needed = false;  // boxes changed in place since it was fitted
   bool bin_pending = false;       // bin_done may not have passed yet
   bool tree_captured = false;     // the last build or refit was queued under capture
-  hipEvent_t tree_done = nullptr;
   hipEvent_t bin_done = nullptr;
   hipStream_t bin_stream = nullptr;
   rts::NodeRec* nodes = nullptr;

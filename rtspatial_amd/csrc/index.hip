@@ -1069,11 +1069,12 @@ struct Tuned {
 // a call on all queries, whether its results had room. A time is the fastest
 // of `reps` runs, after an untimed one when the traversal mode has not run yet
 // (its kernels then load and warm up); a plan whose first run is already 3x
-// slower than the best so far is not repeated.
+// slower than the best so far is not repeated. On all queries an order has to
+// win by `order_margin`.
 template <typename Run, typename Fits>
 int tune_plans(const rts_tune_config& cfg, uint32_t leaf_sizes, const Plan& base, bool try_other,
-               bool sample_is_all, bool whole_set, hipEvent_t* ev, hipStream_t stream, Run&& run,
-               Fits&& fits, Tuned* out) {
+               bool sample_is_all, bool whole_set, double order_margin, hipEvent_t* ev,
+               hipStream_t stream, Run&& run, Fits&& fits, Tuned* out) {
   Tuned& t = *out;
   bool warm[3] = {false, false, false};
   auto time_on = [&](const Plan& p, bool all, double best, double* ms_out) -> int {
@@ -1157,6 +1158,7 @@ int tune_plans(const rts_tune_config& cfg, uint32_t leaf_sizes, const Plan& base
         rc = time_on(p, true, 1e300, &ms);
         if (!rc) rc = fits(&ok);
         if (rc) return rc;
+        if (o == 1) ms *= order_margin;
         if (ms < best_ms) {
           best_ms = ms;
           best_plan = p;
@@ -1524,8 +1526,9 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
   if (rc) return rc;
 
   // An evenly strided sample, shrunk until its results fit kMaxPairs (512 MiB
-  // of pairs: one timed run then writes at most that much, about 2 ms on the
-  // 10M-box index, which keeps a predicate's tuning under 50 ms). A double index's
+  // of pairs: one timed run then writes at most that much, some 4 ms on the
+  // 10M-box index; a predicate's tuning takes 60 to 110 ms there, a third of it
+  // for the tree that handlers walk). A double index's
   // sample is taken in doubles; one that rounds doubles to floats times the
   // rounded sample.
   const size_t qbytes = query_bytes(pts, ix->f64());
@@ -1597,7 +1600,7 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
   Tuned own;
   rc = tune_plans(
       cfg, 1u, base, base.traversal == RTS_TRAVERSAL_THREAD || octets, sample_is_all, whole_set,
-      tb.ev, stream,
+      1.0, tb.ev, stream,
       [&](const Plan& p, bool all) -> int {
         RTS_HIP(hipMemsetAsync(counter, 0, sizeof(*counter), stream));
         return run_plan(ix, p, pred, all ? queries : tb.sample, all ? n : m, pts, f64, handler,
@@ -1620,6 +1623,10 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
   // step, while a wavefront scans 512 leaves (on a 10M-box index intersects
   // queries with ~1e4 results each took 446 ms per lane and 6 per wavefront).
   constexpr double kLaneMaxResults = 256.0;
+  // An order scatters what a handler keeps by query id: three atomics a pair on
+  // 200k queries of 80 results took 1.18 ms in Morton order and 0.65 in input
+  // order, where the walks alone tie at 0.47.
+  constexpr double kHandlerOrderMargin = 1.1;
   const Plan handler_base = plan_query(ix, pred, pts, n, true);
   RTS_HIP(dev_alloc(&tb.sink, whole_set ? n : m));
   RTS_HIP(launch_fill_u32(tb.sink, 0u, whole_set ? n : m, stream));
@@ -1630,7 +1637,7 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
     rc = tune_plans(
         cfg, cfg.leaf_sizes & 0x7Eu, handler_base,
         handler_base.traversal == RTS_TRAVERSAL_THREAD || mean_results <= kLaneMaxResults,
-        sample_is_all, whole_set, tb.ev, stream,
+        sample_is_all, whole_set, kHandlerOrderMargin, tb.ev, stream,
         [&](const Plan& p, bool all) -> int {
           return run_handler(ix, p, pred, all ? queries : tb.sample, all ? n : m, pts, f64,
                              handler == RTS_HANDLER_COLLECT, tb.sink, stream);

@@ -1627,13 +1627,14 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
   // 200k queries of 80 results took 1.18 ms in Morton order and 0.65 in input
   // order, where the walks alone tie at 0.47.
   constexpr double kHandlerOrderMargin = 1.1;
+  // Where there is no room for that tree handlers' calls keep their plan.
   const Plan handler_base = plan_query(ix, pred, pts, n, true);
-  RTS_HIP(dev_alloc(&tb.sink, whole_set ? n : m));
-  RTS_HIP(launch_fill_u32(tb.sink, 0u, whole_set ? n : m, stream));
-  const bool made = ix->bcap == 0;
-  rc = ensure_binary(ix, stream);
   Tuned han;
-  if (!rc)
+  han.winner = handler_base;
+  const bool made = ix->bcap == 0;
+  const bool room = dev_alloc(&tb.sink, whole_set ? n : m) == hipSuccess &&
+                    ensure_binary(ix, stream) == RTS_OK;
+  if (room)
     rc = tune_plans(
         cfg, cfg.leaf_sizes & 0x7Eu, handler_base,
         handler_base.traversal == RTS_TRAVERSAL_THREAD || mean_results <= kLaneMaxResults,
@@ -1652,7 +1653,7 @@ int rts_index_autotune(rts_index* ix, rts_predicate pred, const void* queries, u
   if (rc) return rc;
   if (cfg.apply) {
     ix->tuned[pred][pts ? 1 : 0] = stored_plan(own, n, false);
-    ix->handler_tuned[pred][pts ? 1 : 0] = stored_plan(han, n, true);
+    if (room) ix->handler_tuned[pred][pts ? 1 : 0] = stored_plan(han, n, true);
   }
   out->leaf_size = han.winner.leaf_size;
   out->traversal = (uint32_t)own.winner.traversal;

@@ -510,24 +510,36 @@ __device__ __forceinline__ void oct_replay(const TreeView& t, const uint2* entri
   }
 }
 
+// Two neighbouring pairs of a query, as store_pair.
+__device__ __forceinline__ void store_two_pairs(rts_pair* p, uint32_t g0, uint32_t g1,
+                                                uint32_t query_id) {
+  typedef uint32_t Words __attribute__((ext_vector_type(4), aligned(4)));
+  const Words w = {g0, query_id, g1, query_id};
+  __builtin_nontemporal_store(w, reinterpret_cast<Words*>(p));
+}
+
 // Emits the logged results [lo, hi) of one query. Blocks are taken 8 at a time,
 // one per octet: each lane stores the result its mask bit names, and the
 // wave's stores of a round are consecutive pairs. Runs of up to 64 leaves (most
 // are nodes of 64) are copied kShortRuns at a time, with as many loads of ids in
-// flight; longer ones 4 x 64 leaves at a time. The next 64 entries are in flight
-// while these are emitted.
+// flight; longer ones kRunStore leaves at a time, from a line of the output on
+// as whole lines, two pairs a lane. The next 64 entries are in flight while
+// these are emitted.
 // One run at a time, each waiting for its own load, held large queries' write
 // passes back. Served intersects requests, 9e10 pairs on 10M boxes, one batch in
-// flight: 340-391 ms of write passes by where the arena lies, now 304-310 (the
-// walk that logs replaced took 307); within requests 288-331, now 265-302 (298);
-// four at a time lies halfway. Windows in the walks' Morton order instead of the
+// flight: 340-391 ms of write passes by where the arena lies, then 304-310 (the
+// walk that logs replaced took 307); within requests 288-331, then 265-302 (298);
+// four at a time lies halfway. Whole lines: the served mix, 5.9e10 pairs, 216-236
+// ms with neither, 195-217 without, now 184-198 (184-201); 10M boxes x 200k
+// queries 10.2-10.4 ms without, now 9.1-9.9 (8.9). Windows in the walks' Morton order instead of the
 // output's, which fetch a third as much, gain nothing here, and on a million
 // boxes or a clustered set they are 1.1-2.4x slower: neighbouring waves then
 // write far apart.
 constexpr int kShortRuns = 8;
-template <typename Emit>
-__device__ void wide_replay(const TreeView& t, const RangeLog& lg, uint32_t lo, uint32_t hi,
-                            const uint32_t qid, const Emit& emit) {
+constexpr uint32_t kRunStore = 4 * kWave;
+__device__ __forceinline__ void wide_replay(const TreeView& t, const RangeLog& lg, uint32_t lo,
+                                            uint32_t hi, const uint32_t qid,
+                                            const QueueEmit& emit) {
   const uint32_t lane = lane_id(), j = lane & 7u, oct = lane >> 3;
   uint32_t first = 0;  // wave-uniform: result of the next entry
   uint2 next = lane < lg.n_in ? log_load(lg.entries + lane) : make_uint2(0u, 0u);
@@ -589,6 +601,22 @@ __device__ void wide_replay(const TreeView& t, const RangeLog& lg, uint32_t lo, 
       const uint32_t c = readlane_u32(cnt, l);
       uint32_t k = lo > at ? lo - at : 0u;
       const uint32_t n = hi - at < c ? hi - at : c;
+      if (k + 2 * kRunStore <= n && emit.base + at + n <= emit.cap) {
+        rts_pair* const first_out = emit.out + emit.base + at;
+        const uint32_t past = (uint32_t)((uintptr_t)(first_out + k) / sizeof(rts_pair)) % 16u;
+        const uint32_t head = (16u - past) % 16u;  // up to a line's start
+        if (lane < head) emit(at + k + lane, t.leaf_ids[f + k + lane], qid);
+        k += head;
+        for (; k + kRunStore <= n; k += kRunStore) {
+          uint2 gid[kRunStore / (2 * kWave)];
+#pragma unroll
+          for (uint32_t u = 0; u < kRunStore / (2 * kWave); u++)
+            __builtin_memcpy(&gid[u], t.leaf_ids + f + k + 2 * (u * kWave + lane), sizeof(uint2));
+#pragma unroll
+          for (uint32_t u = 0; u < kRunStore / (2 * kWave); u++)
+            store_two_pairs(first_out + k + 2 * (u * kWave + lane), gid[u].x, gid[u].y, qid);
+        }
+      }
       for (; k + 4 * kWave <= n; k += 4 * kWave) {
         uint32_t gid[4];
 #pragma unroll
